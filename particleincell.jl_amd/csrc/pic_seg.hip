@@ -200,9 +200,21 @@ inline bool multi_tile_shape(int kernel) {
 // 1e7 particles, 128^2): 166.7 us per pass bounded at eight waves per SIMD,
 // 164.2 at four, 161.2 at four with the early load (at eight with the early
 // load the pass spilled: 165.7).
+//
+// The pass without a deposit (the loop's last, and the adjoint's
+// recomputation) is the same: it comes several steps after the sort, so it
+// needs at least the drift margin of the passes before it.  With the 40 KiB
+// window and 512-thread blocks of the deposit-only pass (M6: a margin of 11
+// cells) a quarter of its waves queued on the deferred list's counter.
+// Measured on MI355X, the last pass of 24 steps (Landau M6, 1e7 particles,
+// 128^2, 11 steps after the sort): 567 us in 40 KiB, 75 in 80 KiB (two
+// blocks per CU, margin 20), 71 in 160 KiB (one block, margin 32, next
+// particle loaded early); 2e8 particles on 512^2, 3 steps after the sort:
+// 13.8, 1.73 and 1.79 ms; CIC, 1e8 on 256^2: 874, 844 and 822 us; the
+// adjoint's recomputation (CIC, 2e6, 128^2): 18.8, 17.7 and 17.0 us.
 template <int K, bool DRIFT, bool DEPOSIT, int ACC>
 constexpr bool seg32_wide() {
-    return multi_tile_shape<K>() && ACC >= 2 && DRIFT && DEPOSIT;
+    return !DEPOSIT || (multi_tile_shape<K>() && ACC >= 2 && DRIFT);
 }
 template <int K, bool DRIFT, bool DEPOSIT, int ACC, bool PERM>
 constexpr int seg32_waves() {
@@ -216,8 +228,10 @@ constexpr int seg32_waves() {
 // such block per CU); the others SEG_T.
 template <int K, bool DRIFT, bool DEPOSIT, int ACC>
 constexpr int seg32_threads() {
-    return multi_tile_shape<K>() && ACC >= 2 && DRIFT && DEPOSIT ? 1024 : SEG_T;
+    return seg32_wide<K, DRIFT, DEPOSIT, ACC>() ? 1024 : SEG_T;
 }
+
+constexpr size_t SEG_KICK_LDS_BYTES = 160 * 1024;  // the pass without a deposit
 
 template <int K, bool GATHER, bool DRIFT, bool DEPOSIT, int BZ, int ACC, bool PERM>
 __global__ __launch_bounds__((seg32_threads<K, DRIFT, DEPOSIT, ACC>()),
@@ -718,7 +732,8 @@ static int seg32_mode(const Ctx *c, const SegF32 &a, int mode, int bz, size_t sm
     switch (mode) {
         case 0: seg32_bz<K, false, true, true, ACC, P>(c, a, PIC_BZ_NONE, sm); break;
         case 1: seg32_bz<K, true, true, true, ACC, P>(c, a, bz, sm); break;
-        case 2: seg32_bz<K, true, true, false, ACC, P>(c, a, bz, sm); break;
+        // no deposit: one kernel whatever the charge accumulation
+        case 2: seg32_bz<K, true, true, false, 2, P>(c, a, bz, sm); break;
         case 3: seg32_bz<K, false, false, true, ACC, P>(c, a, PIC_BZ_NONE, sm); break;
         default: return fail(PIC_ERR_ARG, "pass mode %d", mode);
     }
@@ -798,9 +813,13 @@ int launch_seg32(Ctx *c, int kernel, int mode, double dt, double dtd) {
                             (mode == 2 ? 0 : acc == 2 ? 4 * a.tiles : 8);
     // the drift-and-deposit passes with fixed-point tiles run 1024-thread
     // blocks with the context's window (pic_set_f32_window, 160 KiB by
-    // default: one block per CU); the others 40 KiB
+    // default: one block per CU), the pass without a deposit 1024-thread
+    // blocks with 160 KiB; the deposit-only pass and the other accumulation
+    // modes 40 KiB
     const bool wide = acc == 2 && multi_tile_shape(kernel) && (mode == 0 || mode == 1);
-    const size_t win = wide ? (size_t)c->f32_window_kib * 1024 : SEG_LDS_BYTES;
+    const size_t win = wide        ? (size_t)c->f32_window_kib * 1024
+                       : mode == 2 ? SEG_KICK_LDS_BYTES
+                                   : SEG_LDS_BYTES;
     a.cap = (int)(win / (per_node ? per_node : 8)) & ~15;
     a.slow = c->slow_chunks;
     PIC_TRY(ensure_defer(c));
