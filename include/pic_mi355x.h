@@ -431,14 +431,15 @@ int pic_fdtd_energy(pic_ctx *ctx, double *energy);
  * energy[s] = compute_energy after iteration s+1 (examples/vm2d.jl:55; may
  * be NULL).  One launch per iteration when 8 (nx(ny+1) + (nx+1)ny + 6 nx ny)
  * bytes fit in 150 KiB of LDS (132 KiB at 128 x 16), else two up to 3072
- * cells, else one kernel per reference function.  kernel must be PIC_CIC;
- * FP64 state. */
+ * cells, else three up to 81,920 (the current summed in LDS in up to eight
+ * parts; a second set of particle arrays with more than one), else one
+ * kernel per reference function.  kernel must be PIC_CIC; FP64 state. */
 int pic_run_maxwell(pic_ctx *ctx, int kernel, double dt, int nsteps, double *energy);
 
 /* How pic_run_maxwell launches an iteration: 0 (the default) the most
  * fused form the grid allows in LDS (one launch per iteration up to 2048
- * cells, two up to 3072), 2 at most two launches, 3 one kernel per
- * reference function.  All compute the same arithmetic; for tests and
+ * cells, two up to 3072, three up to 81,920), 2 the same without the
+ * one-launch form, 3 one kernel per reference function.  All compute the same arithmetic; for tests and
  * measurements.  No reference counterpart. */
 int pic_set_maxwell_path(pic_ctx *ctx, int path);
 

@@ -859,8 +859,8 @@ class Simulation:
         return f
 
     def set_maxwell_path(self, path):
-        """0: the most fused launch form the grid allows; 2: at most two
-        launches per iteration; 3: one kernel per reference function
+        """0: the most fused launch form the grid allows; 2: the same without
+        the one-launch form; 3: one kernel per reference function
         (pic_set_maxwell_path)."""
         L.call("pic_set_maxwell_path", self.ctx.h, int(path))
 

@@ -160,6 +160,11 @@ struct Ctx {
     double *fd2_ex = nullptr, *fd2_ey = nullptr, *fd2_bz = nullptr;
     double *jb[4] = {nullptr, nullptr, nullptr, nullptr};  // J1 x, y, J2 x, y
     int vm_path = 0;  // pic_set_maxwell_path
+    // the three-launch iteration of larger grids: (ex, ey, bz, -) per node,
+    // and a copy of (jx, jy) per chunk of particles
+    void *vm_nodes = nullptr;
+    double *vm_copies = nullptr;
+    int64_t vm_copies_cap = 0;
 
     // UA (ua_type.jl): ntau, eps; per particle b, t (Particles.b, .t), the
     // positions at the start of a UA step and, between its prediction and
@@ -224,7 +229,9 @@ int settle_state(Ctx *c);
 int alt_f32(Ctx *c, int32_t **cell, float4 **ov);
 void swap_alt_f32(Ctx *c);
 int alt_f64(Ctx *c, double **x, double **y, double **vx, double **vy, double **w);
-void swap_alt_f64(Ctx *c);
+// Without `weights` the weights stay in the current array (a pass that keeps
+// the particles in their slots).
+void swap_alt_f64(Ctx *c, bool weights = true);
 
 int launch_fill(Ctx *c, double *p, double v, int64_t n);
 

@@ -9,6 +9,8 @@
 //                                             k_vm_pass, one pass per particle
 //   faraday(dt/2), ampere_maxwell!(dt)        k_faraday, k_ampere
 //   compute_energy                            k_fdtd_energy
+// or, the default, in one launch (up to 2048 cells), two (up to 3072) or three
+// (k_vm_pass_part, k_vm_reduce, k_vm_fields_tile; up to 81,920).
 // The field kernels follow the reference's arithmetic term by term, so they
 // agree with it bit for bit; the current is summed with FP64 atomics (in an
 // LDS copy of the whole grid when it fits), which reorders its sums.
@@ -66,18 +68,26 @@ __global__ void k_ampere(int nx, int ny, double dx, double dy, double *__restric
 
 // update_fields!: fdtd.jl:60-77 on the nodes i <= nx, j <= ny (the ghost
 // row and column of the reference are their periodic images).
+// nodes (may be null): the three components of a node side by side as well.
+struct VmNode {
+    double ex, ey, bz, pad;
+};
 __global__ void k_update_fields(int nx, int ny, const double *__restrict__ fex,
                                 const double *__restrict__ fey, const double *__restrict__ fbz,
                                 double *__restrict__ ex, double *__restrict__ ey,
-                                double *__restrict__ bz) {
+                                double *__restrict__ bz, VmNode *__restrict__ nodes) {
     const int t = blockIdx.x * MT + threadIdx.x;
     if (t >= nx * ny) return;
     const int i = t % nx + 1, j = t / nx + 1;
-    ex[t] = 0.5 * (fex[m1z(i - 1, nx) + nx * (j - 1)] + fex[m1z(i, nx) + nx * (j - 1)]);
-    ey[t] = 0.5 * (fey[(i - 1) + (nx + 1) * m1z(j - 1, ny)] + fey[(i - 1) + (nx + 1) * m1z(j, ny)]);
-    bz[t] = 0.25 * (((fbz[m1z(i - 1, nx) + nx * m1z(j - 1, ny)] + fbz[m1z(i, nx) + nx * m1z(j - 1, ny)]) +
-                     fbz[m1z(i - 1, nx) + nx * m1z(j, ny)]) +
-                    fbz[m1z(i, nx) + nx * m1z(j, ny)]);
+    const double e1 = 0.5 * (fex[m1z(i - 1, nx) + nx * (j - 1)] + fex[m1z(i, nx) + nx * (j - 1)]);
+    const double e2 = 0.5 * (fey[(i - 1) + (nx + 1) * m1z(j - 1, ny)] + fey[(i - 1) + (nx + 1) * m1z(j, ny)]);
+    const double b3 = 0.25 * (((fbz[m1z(i - 1, nx) + nx * m1z(j - 1, ny)] + fbz[m1z(i, nx) + nx * m1z(j - 1, ny)]) +
+                               fbz[m1z(i - 1, nx) + nx * m1z(j, ny)]) +
+                              fbz[m1z(i, nx) + nx * m1z(j, ny)]);
+    ex[t] = e1;
+    ey[t] = e2;
+    bz[t] = b3;
+    if (nodes) nodes[t] = {e1, e2, b3, 0.0};
 }
 
 // The reference's CIC cell (floor) and offset of a coordinate
@@ -593,6 +603,315 @@ __global__ __launch_bounds__(VT) void k_vm_step(VmArgs a, VmStepIo io) {
     flush_current<VT>(m, sjx, sjy, io.jacc_x, io.jacc_y);
 }
 
+// ------------------------------------------- three launches per iteration
+//
+// Grids whose node fields no longer fit one workgroup's LDS: the current does,
+// whole or in parts.  Per iteration:
+//   k_vm_pass_part    the particle half.  Block (chunk, r) runs chunk's
+//                     particles and sums part r of the 2 nx ny values of
+//                     (jx, jy) in LDS, then stores it, without atomics, as
+//                     the chunk's copy of that part;
+//   k_vm_reduce       jx, jy: the chunks' copies summed in chunk order, and
+//                     faraday!(dt/2);
+//   k_vm_fields_tile  ampere_maxwell!(dt), the energy, and the next iteration's
+//                     faraday!(dt/2) and update_fields!, tile by tile.
+// The arithmetic is that of the kernels above, term by term.
+//
+// One FP64 global atomic per node and component costs more than everything
+// else here: measured on MI355X, scattered ones retire at 24e9/s and runs of
+// consecutive ones at 180e9/s, so the eight of each particle took 356 us per
+// iteration at 128 x 64 cells and 1,024,000 particles (64 MB of state: 13 us
+// at the copy rate).  256 blocks adding whole LDS copies of that grid would
+// take 23 us, storing them 7 and summing them 4.
+//
+// With R = 1 part a block updates its particles in place.  With more the R
+// blocks of a chunk all push its particles, block r = 0 alone stores them, into
+// the alternate arrays, since the others may still be reading; R parts cost
+// R times the push, so past VM_PARTS_MAX the loop falls back to atomics.
+constexpr size_t VM_PART_LDS = 160 * 1024;
+constexpr int VM_PARTS_MAX = 8;
+constexpr int VM_TX = 32, VM_TY = 8;  // tile of k_vm_fields_tile, one node per thread
+
+struct VmPart {
+    const VmNode *nodes;
+    double *copies;               // chunk c's 2 nx ny values at c * 2 nx ny
+    double *xo, *yo, *vxo, *vyo;  // the state after the pass
+    int chunks, parts, len;       // len values per part
+};
+
+template <bool SPLIT>
+__global__ __launch_bounds__(VT) void k_vm_pass_part(VmArgs a, VmPart q) {
+    extern __shared__ double lds[];
+    constexpr int P = 2;  // particles per thread and round, their loads issued together
+    const int nx = a.nx, ny = a.ny, m = nx * ny, tid = threadIdx.x;
+    const int chunk = SPLIT ? blockIdx.x / q.parts : blockIdx.x;
+    const int r0 = SPLIT ? blockIdx.x - chunk * q.parts : 0;
+    const int lo = r0 * q.len, len = min(q.len, 2 * m - lo);
+    const bool store = !SPLIT || r0 == 0;
+    const int64_t p0 = a.n * chunk / q.chunks, p1 = a.n * (chunk + 1) / q.chunks;
+    const double dt = a.dt, h = 0.5 * dt;
+    double px[P], py[P], v1[P], v2[P], wg[P];
+    auto load = [&](int64_t base) {
+#pragma unroll
+        for (int r = 0; r < P; ++r) {
+            const int64_t k = min(base + r * VT + tid, p1 - 1);
+            px[r] = a.x[k];
+            py[r] = a.y[k];
+            v1[r] = a.vx[k];
+            v2[r] = a.vy[k];
+            wg[r] = a.w ? a.w[k] : a.w0;
+        }
+    };
+    if (p0 < p1) load(p0);
+    for (int t = tid; t < len; t += VT) lds[t] = 0.0;
+    __syncthreads();
+    auto add = [&](int t, double v) {
+        if (SPLIT) {
+            t -= lo;
+            if ((unsigned)t >= (unsigned)len) return;
+        }
+        __hip_atomic_fetch_add(&lds[t], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    for (int64_t base = p0; base < p1; base += VT * P) {
+        VmNode c[P][4];
+        double fx[P], fy[P];
+#pragma unroll
+        for (int r = 0; r < P; ++r) {
+            const int i = cic_cell(px[r], a.dx, nx, fx[r]), j = cic_cell(py[r], a.dy, ny, fy[r]);
+            const int ip = i + 1 == nx ? 0 : i + 1, jp = j + 1 == ny ? 0 : j + 1;
+            c[r][0] = q.nodes[i + nx * j];
+            c[r][1] = q.nodes[ip + nx * j];
+            c[r][2] = q.nodes[ip + nx * jp];
+            c[r][3] = q.nodes[i + nx * jp];
+        }
+        double x[P], y[P], u1[P], u2[P], w[P];
+#pragma unroll
+        for (int r = 0; r < P; ++r) {
+            x[r] = px[r];
+            y[r] = py[r];
+            u1[r] = v1[r];
+            u2[r] = v2[r];
+            w[r] = wg[r];
+        }
+        if (base + VT * P < p1) load(base + VT * P);
+#pragma unroll
+        for (int r = 0; r < P; ++r) {
+            const int64_t k = base + r * VT + tid;
+            if (k >= p1) continue;
+            {  // push_v!: pushers_cic.jl:13-51
+                const double dxp = fx[r], dyp = fy[r];
+                const double a1 = (1 - dxp) * (1 - dyp), a2 = dxp * (1 - dyp), a3 = dxp * dyp,
+                             a4 = (1 - dxp) * dyp;
+                const double e1 = a1 * c[r][0].ex + a2 * c[r][1].ex + a3 * c[r][2].ex + a4 * c[r][3].ex;
+                const double e2 = a1 * c[r][0].ey + a2 * c[r][1].ey + a3 * c[r][2].ey + a4 * c[r][3].ey;
+                const double b3 = a1 * c[r][0].bz + a2 * c[r][1].bz + a3 * c[r][2].bz + a4 * c[r][3].bz;
+                u1[r] += 0.5 * dt * e1;
+                u2[r] += 0.5 * dt * e2;
+                const double tantheta = 0.5 * dt * b3;
+                const double sintheta = 2 * tantheta / (1 + tantheta * tantheta);
+                u1[r] += u2[r] * tantheta;
+                u2[r] += -u1[r] * sintheta;
+                u1[r] += u2[r] * tantheta;
+                u1[r] = u1[r] + 0.5 * dt * e1;
+                u2[r] = u2[r] + 0.5 * dt * e2;
+            }
+            auto drift = [&]() {  // push_x!(dt/2): pushers_cic.jl:55-72
+                double q1 = x[r] + h * u1[r], q2 = y[r] + h * u2[r];
+                if (q1 > a.dimx) q1 -= a.dimx;
+                if (q2 > a.dimy) q2 -= a.dimy;
+                if (q1 < 0.0) q1 += a.dimx;
+                if (q2 < 0.0) q2 += a.dimy;
+                x[r] = q1;
+                y[r] = q2;
+            };
+            drift();
+            {  // compute_current!: cloud_in_cell.jl:31-60
+                double dxp, dyp;
+                const int i = cic_cell(x[r], a.dx, nx, dxp), j = cic_cell(y[r], a.dy, ny, dyp);
+                const int ip = i + 1 == nx ? 0 : i + 1, jp = j + 1 == ny ? 0 : j + 1;
+                const double a1 = (1 - dxp) * (1 - dyp), a2 = dxp * (1 - dyp), a3 = dxp * dyp,
+                             a4 = (1 - dxp) * dyp;
+                const double w1 = u1[r] * a.scaling * w[r], w2 = u2[r] * a.scaling * w[r];
+                const int n4[4] = {i + nx * j, ip + nx * j, ip + nx * jp, i + nx * jp};
+                const double q4[4] = {a1, a2, a3, a4};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    add(n4[e], q4[e] * w1);
+                    add(m + n4[e], q4[e] * w2);
+                }
+            }
+            drift();
+            if (store) {
+                q.xo[k] = x[r];
+                q.yo[k] = y[r];
+                q.vxo[k] = u1[r];
+                q.vyo[k] = u2[r];
+            }
+        }
+    }
+    __syncthreads();
+    double *out = q.copies + (size_t)chunk * 2 * m + lo;
+    for (int t = tid; t < len; t += VT) out[t] = lds[t];
+}
+
+// (jx, jy)[t] = the sum of the chunks' copies, 64 values per block, W waves
+// each taking every W-th chunk, the waves' sums added in order; and
+// bz1 = bz + faraday!(dt/2) with the fields of the iteration's start.
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_vm_reduce(int nx, int ny, double dx, double dy,
+                                                      double dt, const double *__restrict__ copies,
+                                                      int chunks, double *__restrict__ jx,
+                                                      double *__restrict__ jy,
+                                                      const double *__restrict__ ex,
+                                                      const double *__restrict__ ey,
+                                                      const double *__restrict__ bz,
+                                                      double *__restrict__ bz1) {
+    __shared__ double sh[64 * W];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, m = nx * ny;
+    const int t = blockIdx.x * 64 + lane;
+    double s = 0.0;
+    if (t < 2 * m) {
+#pragma unroll 8
+        for (int b = wv; b < chunks; b += W) s += copies[(size_t)b * 2 * m + t];
+    }
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    if (wv != 0 || t >= 2 * m) return;
+    for (int k = 1; k < W; ++k) s += sh[64 * k + lane];
+    if (t >= m) {
+        jy[t - m] = s;
+        return;
+    }
+    jx[t] = s;
+    const int j = t / nx, i = t - j * nx;  // faraday!: fdtd.jl:24-36
+    const int ip = i + 1 == nx ? 0 : i + 1, jp = j + 1 == ny ? 0 : j + 1;
+    const double dex_dy = (ex[i + nx * jp] - ex[i + nx * j]) / dy;
+    const double dey_dx = (ey[ip + (nx + 1) * j] - ey[i + (nx + 1) * j]) / dx;
+    bz1[t] = bz[t] + dt * (dex_dy - dey_dx);
+}
+
+struct VmTile {
+    int nx, ny;
+    double dx, dy, dt;
+    const double *ex, *ey, *bz1, *jx, *jy;  // before ampere_maxwell!
+    double *exo, *eyo, *bzo;                // after the field work
+    double *nex, *ney, *nbz;                // node fields of the next iteration
+    VmNode *nodes;
+    double *part;                           // energy: a partial sum per block
+    unsigned *count;
+    double *energy;
+    int next;                               // another iteration follows
+};
+
+// One tile of VM_TX x VM_TY nodes per block: ampere_maxwell!(dt) on the tile
+// and the neighbours its later stages read (recomputed, the same operations
+// on the same inputs as in their own tile), the energy, then faraday!(dt/2)
+// and update_fields! of the next iteration.  The ghost row of fdtd.ex and
+// column of fdtd.ey are updated from their own values, as the reference's.
+__global__ __launch_bounds__(VM_TX *VM_TY) void k_vm_fields_tile(VmTile a) {
+    constexpr int T = VM_TX * VM_TY, XW = VM_TX + 1, YW = VM_TX + 2;
+    __shared__ double sx[XW * (VM_TY + 2)];  // ex at i0 - 1 .., j0 - 1 .. j0 + VM_TY
+    __shared__ double sy[YW * (VM_TY + 1)];  // ey at i0 - 1 .. i0 + VM_TX, j0 - 1 ..
+    __shared__ double sb[XW * (VM_TY + 1)];  // bz at i0 - 1 .., j0 - 1 ..
+    __shared__ double red[T / 64];
+    __shared__ bool last;
+    const int nx = a.nx, ny = a.ny, tid = threadIdx.x;
+    const int i0 = blockIdx.x * VM_TX, j0 = blockIdx.y * VM_TY;
+    const double dt = a.dt;
+    auto wrap = [](int k, int n) { return k < 0 ? k + n : (k >= n ? k - n : k); };
+    // the clamp keeps the tile's unused columns past the mesh in range
+    auto col = [&](int u) { return wrap(min(i0 + u, nx), nx); };
+    auto row = [&](int v) { return wrap(min(j0 + v, ny), ny); };
+    // ampere_maxwell!: fdtd.jl:40-54
+    auto ampx = [&](double e, int i, int jc) {
+        const int jm = jc == 0 ? ny - 1 : jc - 1, ip = i + 1 == nx ? 0 : i + 1;
+        const double dbz_dy = (a.bz1[i + nx * jc] - a.bz1[i + nx * jm]) / a.dy;
+        return e + (dt * dbz_dy - dt * 0.5 * (a.jx[i + nx * jc] + a.jx[ip + nx * jc]));
+    };
+    auto ampy = [&](double e, int ic, int j) {
+        const int im = ic == 0 ? nx - 1 : ic - 1, jp = j + 1 == ny ? 0 : j + 1;
+        const double dbz_dx = (a.bz1[ic + nx * j] - a.bz1[im + nx * j]) / a.dx;
+        return e - (dt * dbz_dx - dt * 0.5 * (a.jy[ic + nx * j] + a.jy[ic + nx * jp]));
+    };
+    for (int t = tid; t < XW * (VM_TY + 2); t += T) {
+        const int v = t / XW, u = t - v * XW, i = col(u - 1), j = row(v - 1);
+        sx[t] = ampx(a.ex[i + nx * j], i, j);
+    }
+    for (int t = tid; t < YW * (VM_TY + 1); t += T) {
+        const int v = t / YW, u = t - v * YW, i = col(u - 1), j = row(v - 1);
+        sy[t] = ampy(a.ey[i + (nx + 1) * j], i, j);
+    }
+    __syncthreads();
+    const int v = tid / VM_TX, u = tid - v * VM_TX, i = i0 + u, j = j0 + v;
+    const bool in = i < nx && j < ny;
+    double e2 = 0.0;
+    if (in) {
+        const double x = sx[(u + 1) + XW * (v + 1)];
+        a.exo[i + nx * j] = x;
+        a.eyo[i + (nx + 1) * j] = sy[(u + 1) + YW * (v + 1)];
+        e2 = x * x;
+        if (j == ny - 1) {
+            const double g = ampx(a.ex[i + nx * ny], i, 0);
+            a.exo[i + nx * ny] = g;
+            e2 += g * g;
+        }
+        if (i == nx - 1) a.eyo[nx + (nx + 1) * j] = ampy(a.ey[nx + (nx + 1) * j], 0, j);
+    }
+    // compute_energy (fdtd.jl:79-80) in a fixed order: a wave butterfly, the
+    // waves, the blocks
+    for (int o = 32; o > 0; o >>= 1) e2 += __shfl_xor(e2, o);
+    if ((tid & 63) == 0) red[tid >> 6] = e2;
+    if (a.next) {
+        for (int t = tid; t < XW * (VM_TY + 1); t += T) {  // faraday!: fdtd.jl:24-36
+            const int w = t / XW, q = t - w * XW, ii = col(q - 1), jj = row(w - 1);
+            const double dex_dy = (sx[q + XW * (w + 1)] - sx[q + XW * w]) / a.dy;
+            const double dey_dx = (sy[(q + 1) + YW * w] - sy[q + YW * w]) / a.dx;
+            sb[t] = a.bz1[ii + nx * jj] + 0.5 * dt * (dex_dy - dey_dx);
+        }
+    }
+    __syncthreads();
+    if (in) {
+        const int g = i + nx * j;
+        if (a.next) {  // update_fields!: fdtd.jl:60-77
+            const double b00 = sb[u + XW * v], b10 = sb[(u + 1) + XW * v],
+                         b01 = sb[u + XW * (v + 1)], b11 = sb[(u + 1) + XW * (v + 1)];
+            a.bzo[g] = b11;
+            const double n1 = 0.5 * (sx[u + XW * (v + 1)] + sx[(u + 1) + XW * (v + 1)]);
+            const double n2 = 0.5 * (sy[(u + 1) + YW * v] + sy[(u + 1) + YW * (v + 1)]);
+            const double n3 = 0.25 * (((b00 + b10) + b01) + b11);
+            a.nex[g] = n1;
+            a.ney[g] = n2;
+            a.nbz[g] = n3;
+            a.nodes[g] = {n1, n2, n3, 0.0};
+        } else {
+            a.bzo[g] = a.bz1[g];
+        }
+    }
+    const int nblk = gridDim.x * gridDim.y, blk = blockIdx.x + gridDim.x * blockIdx.y;
+    if (tid == 0) {
+        double s = 0.0;
+        for (int k = 0; k < T / 64; ++k) s += red[k];
+        a.part[blk] = s;
+        __threadfence();
+        last = atomicAdd(a.count, 1u) == (unsigned)(nblk - 1);
+    }
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    double s = 0.0;
+    for (int k = tid; k < nblk; k += T)
+        s += __hip_atomic_load(&a.part[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if ((tid & 63) == 0) red[tid >> 6] = s;
+    __syncthreads();
+    if (tid == 0) {
+        s = 0.0;
+        for (int k = 0; k < T / 64; ++k) s += red[k];
+        *a.energy = 0.5 * log(s * a.dx * a.dy);
+        *a.count = 0u;
+    }
+}
+
 inline size_t vm_field_lds(const Ctx *c) {
     const size_t nx = c->nx, ny = c->ny;
     return (nx * (ny + 1) + (nx + 1) * ny + 3 * nx * ny) * 8;
@@ -652,10 +971,11 @@ int ampere(Ctx *c, double dt) {
     return PIC_OK;
 }
 
-int update_fields(Ctx *c) {
+int update_fields(Ctx *c, VmNode *nodes = nullptr) {
     hipLaunchKernelGGL(k_update_fields, blocks_for((int64_t)c->nx * c->ny), dim3(MT), 0,
                        c->stream, c->nx, c->ny, (const double *)c->fd_ex,
-                       (const double *)c->fd_ey, (const double *)c->fd_bz, c->ex, c->ey, c->bz);
+                       (const double *)c->fd_ey, (const double *)c->fd_bz, c->ex, c->ey, c->bz,
+                       nodes);
     PIC_HIP(hipGetLastError());
     c->bz_mode = PIC_BZ_GRID;
     return PIC_OK;
@@ -768,6 +1088,70 @@ int vm_pass_lds_launch(Ctx *c, double dt) {
         hipLaunchKernelGGL((k_vm_pass_lds<VT, 4>), dim3((unsigned)nb), dim3(VT), lds, c->stream, a,
                            fx, fy, fb, c->ex, c->ey, c->bz);
     PIC_HIP(hipGetLastError());
+    return PIC_OK;
+}
+
+// Parts of the current (VM_PART_LDS each) and chunks of particles of
+// k_vm_pass_part; parts > VM_PARTS_MAX or tiles past the partial sums'
+// room: the grid is too large for it.
+struct VmPartPlan {
+    int parts, chunks, len, tiles;
+    bool ok;
+};
+
+VmPartPlan vm_part_plan(const Ctx *c) {
+    VmPartPlan p;
+    const int64_t m2 = (int64_t)2 * c->nx * c->ny;
+    const int64_t room = (int64_t)(VM_PART_LDS / 8);
+    p.parts = (int)std::min<int64_t>((m2 + room - 1) / room, VM_PARTS_MAX + 1);
+    p.len = (int)((m2 + p.parts - 1) / p.parts);
+    // one block per compute unit, at least a particle per thread
+    const int64_t want = (c->n + VT - 1) / VT;
+    p.chunks = (int)std::max<int64_t>(1, std::min<int64_t>(want, c->ncu / p.parts));
+    p.tiles = ((c->nx + VM_TX - 1) / VM_TX) * ((c->ny + VM_TY - 1) / VM_TY);
+    p.ok = p.parts <= VM_PARTS_MAX && p.tiles <= 4 * RED_BLOCKS;
+    return p;
+}
+
+int ensure_part_buffers(Ctx *c, const VmPartPlan &p) {
+    const size_t m = (size_t)c->nx * c->ny;
+    if (!c->vm_nodes) PIC_HIP(hipMalloc(&c->vm_nodes, m * sizeof(VmNode)));
+    const int64_t need = (int64_t)p.chunks * 2 * (int64_t)m;
+    if (need > c->vm_copies_cap) {
+        if (c->vm_copies) (void)hipFree(c->vm_copies);
+        c->vm_copies = nullptr;
+        c->vm_copies_cap = 0;
+        PIC_HIP(hipMalloc(&c->vm_copies, (size_t)need * 8));
+        c->vm_copies_cap = need;
+    }
+    return PIC_OK;
+}
+
+int vm_pass_part(Ctx *c, double dt, const VmPartPlan &p) {
+    VmArgs a = vm_args(c, dt);
+    VmPart q;
+    q.nodes = static_cast<const VmNode *>(c->vm_nodes);
+    q.copies = c->vm_copies;
+    q.chunks = p.chunks;
+    q.parts = p.parts;
+    q.len = p.len;
+    const size_t lds = (size_t)p.len * 8;
+    if (p.parts == 1) {
+        q.xo = c->x; q.yo = c->y; q.vxo = c->vx; q.vyo = c->vy;
+        PIC_HIP(hipFuncSetAttribute((const void *)k_vm_pass_part<false>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(k_vm_pass_part<false>, dim3((unsigned)p.chunks), dim3(VT), lds,
+                           c->stream, a, q);
+        PIC_HIP(hipGetLastError());
+        return PIC_OK;
+    }
+    PIC_TRY(alt_f64(c, &q.xo, &q.yo, &q.vxo, &q.vyo, nullptr));
+    PIC_HIP(hipFuncSetAttribute((const void *)k_vm_pass_part<true>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_vm_pass_part<true>, dim3((unsigned)(p.chunks * p.parts)), dim3(VT), lds,
+                       c->stream, a, q);
+    PIC_HIP(hipGetLastError());
+    swap_alt_f64(c, false);
     return PIC_OK;
 }
 
@@ -939,6 +1323,8 @@ int pic_run_maxwell(pic_ctx *ctx, int kernel, double dt, int nsteps, double *ene
     const bool one = slds <= VM_STEP_LDS_MAX && flds <= VM_STEP_LDS_MAX && c->vm_path != 2;
     const bool fused = !one && flds <= VM_LDS_BYTES_MAX && plds <= VM_LDS_BYTES_MAX &&
                        c->vm_path != 3;
+    const VmPartPlan pp = vm_part_plan(c);
+    const bool parted = !one && !fused && c->vm_path != 3 && pp.ok && c->n > 0;
     auto timed_pass = [&](bool lds) {
         int r = c->timing ? mark() : PIC_OK;
         if (r == PIC_OK) r = lds ? vm_pass_lds_launch(c, dt) : vm_pass(c, dt);
@@ -1012,7 +1398,53 @@ int pic_run_maxwell(pic_ctx *ctx, int kernel, double dt, int nsteps, double *ene
             }
         }
     }
-    for (int s = 1; s <= nsteps && rc == PIC_OK && !fused && !one; ++s) {
+    if (parted) {
+        // fdtd.ex, fdtd.ey alternate between the context's arrays and the
+        // second set; bz goes through the second set within an iteration
+        rc = ensure_step_buffers(c);
+        if (rc == PIC_OK) rc = ensure_part_buffers(c, pp);
+        double *ex[2] = {c->fd_ex, c->fd2_ex}, *ey[2] = {c->fd_ey, c->fd2_ey};
+        VmNode *nodes = static_cast<VmNode *>(c->vm_nodes);
+        if (rc == PIC_OK) rc = update_fields(c, nodes);
+        for (int s = 1; s <= nsteps && rc == PIC_OK; ++s) {
+            if (c->timing) rc = mark();
+            if (rc == PIC_OK) rc = vm_pass_part(c, dt, pp);
+            if (rc == PIC_OK && c->timing) rc = mark();
+            if (rc != PIC_OK) break;
+            const int in = (s - 1) & 1, out = s & 1;
+            auto reduce = [&](auto kern, int w) {
+                hipLaunchKernelGGL(kern, dim3((unsigned)((2 * m + 63) / 64)), dim3(64 * w), 0,
+                                   c->stream, c->nx, c->ny, c->dx, c->dy, 0.5 * dt,
+                                   (const double *)c->vm_copies, pp.chunks, c->jx, c->jy,
+                                   (const double *)ex[in], (const double *)ey[in],
+                                   (const double *)c->fd_bz, c->fd2_bz);
+            };
+            if (pp.chunks > 32) reduce(k_vm_reduce<8>, 8);
+            else reduce(k_vm_reduce<1>, 1);
+            VmTile t;
+            t.nx = c->nx; t.ny = c->ny; t.dx = c->dx; t.dy = c->dy; t.dt = dt;
+            t.ex = ex[in]; t.ey = ey[in]; t.bz1 = c->fd2_bz; t.jx = c->jx; t.jy = c->jy;
+            t.exo = ex[out]; t.eyo = ey[out]; t.bzo = c->fd_bz;
+            t.nex = c->ex; t.ney = c->ey; t.nbz = c->bz; t.nodes = nodes;
+            t.part = c->red_part; t.count = c->red_count;
+            t.energy = c->energy_hist + (s - 1);
+            t.next = s < nsteps;
+            hipLaunchKernelGGL(k_vm_fields_tile,
+                               dim3((unsigned)((c->nx + VM_TX - 1) / VM_TX),
+                                    (unsigned)((c->ny + VM_TY - 1) / VM_TY)),
+                               dim3(VM_TX * VM_TY), 0, c->stream, t);
+            if (hipGetLastError() != hipSuccess) rc = fail(PIC_ERR_HIP, "field kernel launch");
+        }
+        if (rc == PIC_OK && nsteps % 2 != 0) {  // the fields back into the context's arrays
+            const size_t bx = (size_t)c->nx * (c->ny + 1) * 8, by = (size_t)(c->nx + 1) * c->ny * 8;
+            if (hipMemcpyAsync(c->fd_ex, c->fd2_ex, bx, hipMemcpyDeviceToDevice, c->stream) !=
+                    hipSuccess ||
+                hipMemcpyAsync(c->fd_ey, c->fd2_ey, by, hipMemcpyDeviceToDevice, c->stream) !=
+                    hipSuccess)
+                rc = fail(PIC_ERR_HIP, "field copy");
+        }
+    }
+    for (int s = 1; s <= nsteps && rc == PIC_OK && !fused && !one && !parted; ++s) {
         if (s > 1) rc = faraday(c, 0.5 * dt);
         if (rc == PIC_OK) rc = update_fields(c);
         if (rc == PIC_OK) rc = launch_fill(c, c->jx, 0.0, m);

@@ -556,7 +556,7 @@ int alt_f64(Ctx *c, double **x, double **y, double **vx, double **vy, double **w
     return PIC_OK;
 }
 
-void swap_alt_f64(Ctx *c) {
+void swap_alt_f64(Ctx *c, bool weights) {
     int s[5] = {0, 0, 0, 0, 0};
     (void)alt_slot(c, c->x, &s[0]);
     (void)alt_slot(c, c->y, &s[1]);
@@ -566,7 +566,7 @@ void swap_alt_f64(Ctx *c) {
     alt_swap(c, c->y, s[1]);
     alt_swap(c, c->vx, s[2]);
     alt_swap(c, c->vy, s[3]);
-    if (!c->uniform_w) {
+    if (weights && !c->uniform_w) {
         (void)alt_slot(c, c->w, &s[4]);
         alt_swap(c, c->w, s[4]);
     }

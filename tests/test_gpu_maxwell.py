@@ -297,3 +297,43 @@ def test_run_maxwell_continues(gpu, O):
     assert np.max(np.abs(e - eo)) < 1e-10 * np.max(np.abs(eo))
     for a, b in ((g.ex, o.ex), (g.ey, o.ey), (g.bz, o.bz)):
         assert np.max(np.abs(a - b)) <= 1e-10 * np.max(np.abs(b))
+
+
+@pytest.mark.parametrize("nx,ny,n,steps,weighted", [
+    (96, 40, 1, 3, False),           # one particle, one chunk
+    (97, 33, 1023, 4, True),         # one part of the current, ragged tiles
+    (128, 80, 262_144 + 5, 5, False),  # the largest grid of one part
+    (129, 80, 30_001, 4, True),      # two parts
+    (33, 700, 5_000, 3, False),      # three, narrow tiles
+    (288, 284, 40_003, 2, False)])   # eight, the most
+def test_three_launch_iteration_matches_one_kernel_per_function(gpu, nx, ny, n, steps, weighted):
+    """The three-launch iteration (the current in LDS, whole or in parts)
+    against one kernel per reference function on random fields whose ghost row
+    and column are not periodic images: particles, FDTD fields, current,
+    node fields and energies.  Only the order of the current's sums differs,
+    at most a few thousand terms a node: 1e-12 of the largest value."""
+    pic = gpu
+    L = pic._lib
+    rng = np.random.default_rng(nx * ny + n)
+    mesh = pic.TwoDGrid(0.0, 3.0, nx, 0.0, 2.0, ny)
+    w = mesh.dimx * mesh.dimy / n
+    p = random_particles(rng, n, mesh.dimx, mesh.dimy,
+                         w=w * rng.uniform(0.5, 1.5, n) if weighted else None)
+    f = pic.FDTD(mesh)
+    for a in (f.ex, f.ey, f.bz):
+        a[...] = 0.1 * rng.normal(size=a.shape)
+    got = []
+    for path in (0, 3):
+        sim = pic.Simulation(mesh, p, pic.CloudInCell())
+        sim.set_maxwell_path(path)
+        sim.set_fdtd(f)
+        e = [sim.run_maxwell(0.01, steps), sim.run_maxwell(0.01, 1)]
+        g = sim.fdtd()
+        nodes = [sim.grid(k) for k in (L.PIC_GRID_EX, L.PIC_GRID_EY, L.PIC_GRID_BZ)]
+        # one ampere_maxwell! more: the current the run left
+        L.call("pic_ampere_maxwell", sim.ctx.h, 0.01)
+        g2 = sim.fdtd()
+        got.append([np.concatenate(e), sim.particles(), g.ex, g.ey, g.bz, g2.ex, g2.ey] + nodes)
+        sim.close()
+    for a, b in zip(*got):
+        assert np.max(np.abs(a - b)) <= 1e-12 * max(1.0, np.max(np.abs(b)))
