@@ -256,6 +256,7 @@ static int set_particles_impl(Ctx *c, const double *d_p, int64_t n) {
     c->n = n;
     c->state = PIC_STATE_F64;
     c->seg_valid = false;
+    c->near_order = false;
     c->sort_fresh = false;
     if (n == 0) {
         c->uniform_w = true;
@@ -413,8 +414,10 @@ int pic_ctx_destroy(pic_ctx *ctx) {
     dfree(c->fd2_ex); dfree(c->fd2_ey); dfree(c->fd2_bz);
     for (double *&p : c->jb) dfree(p);
     if (c->vm_nodes) (void)hipFree(c->vm_nodes);
-    dfree(c->vm_copies);
+    dfree(c->copies);
     dfree(c->ua_b); dfree(c->ua_t); dfree(c->ua_x0); dfree(c->ua_y0); dfree(c->ua_fhat);
+    dfree(c->ua_e);
+    if (c->ua_tab) (void)hipFree(c->ua_tab);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return PIC_OK;
@@ -619,6 +622,7 @@ int pic_set_state_f32(pic_ctx *ctx, const int32_t *cell, const float *ox, const 
     PIC_HIP(hipStreamSynchronize(c->stream));
     c->state = PIC_STATE_F32;
     c->seg_valid = false;
+    c->near_order = false;
     c->sort_fresh = false;
     return PIC_OK;
 }

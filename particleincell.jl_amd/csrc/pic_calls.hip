@@ -63,7 +63,18 @@ __global__ void k_interpolate_cic(int64_t n, const double *x, const double *y, i
 
 using picd::jl_fmod;
 
-// compute_rho_m6!(fields, particles): compute_rho_m6.jl:181-316, raw
+// compute_rho_m6!(fields, particles)'s positions into [x0, x0 + dimx), [y0,
+// y0 + dimy) (compute_rho_m6.jl:201-207), for the deposit of pic_deposit.hip.
+__global__ void k_mf_wrap(int64_t n, double *x, double *y, double x0, double y0, double dimx,
+                          double dimy) {
+    int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    x[k] = jl_fmod(x[k] - x0, dimx) + x0;
+    y[k] = jl_fmod(y[k] - y0, dimy) + y0;
+}
+
+// compute_rho_m6!(fields, particles) on grids past that deposit's reach:
+// compute_rho_m6.jl:181-316, raw
 // accumulation into acc (nx*ny, the ghost copies are implied).  compat
 // selects the reference's swapped bounds and mod1 neighbours (see the C ABI
 // header).  Weights are the M6 pieces in FP64.
@@ -180,6 +191,11 @@ int pic_compute_rho(pic_ctx *ctx, int kernel) {
     PIC_CHECK(valid_shape(kernel), PIC_ERR_ARG, "kernel %d", kernel);
     Ctx *c = ctx_of(ctx);
     PIC_HIP(hipSetDevice(c->device));
+    if (c->state == PIC_STATE_F64 && !c->near_order && deposit_lds_ok(c)) {
+        PIC_TRY(deposit_rho(c, kernel));
+        PIC_HIP(hipStreamSynchronize(c->stream));
+        return PIC_OK;
+    }
     PIC_TRY(launch_fill(c, c->rho_acc, 0.0, (int64_t)c->nx * c->ny));
     if (c->state == PIC_STATE_F64)
         PIC_TRY(launch_step64(c, kernel, 3, 0.0, 0.0));
@@ -258,9 +274,17 @@ int pic_compute_rho_m6_fields(pic_ctx *ctx, int compat) {
     Ctx *c = ctx_of(ctx);
     PIC_HIP(hipSetDevice(c->device));
     PIC_TRY(need_f64(c));
+    const double x0 = compat ? c->xmax : c->xmin, y0 = compat ? c->ymax : c->ymin;
+    if (deposit_lds_ok(c)) {
+        hipLaunchKernelGGL(k_mf_wrap, grid1(c->n), dim3(256), 0, c->stream, c->n, c->x, c->y, x0,
+                           y0, c->dimx, c->dimy);
+        PIC_HIP(hipGetLastError());
+        PIC_TRY(deposit_rho_mf(c, x0, y0, compat != 0));
+        PIC_HIP(hipStreamSynchronize(c->stream));
+        return PIC_OK;
+    }
     PIC_TRY(launch_fill(c, c->rho_acc, 0.0, (int64_t)c->nx * c->ny));
     if (c->n) {
-        double x0 = compat ? c->xmax : c->xmin, y0 = compat ? c->ymax : c->ymin;
         hipLaunchKernelGGL(k_mf_rho_m6, grid1(c->n), dim3(256), 0, c->stream, c->n, c->x, c->y,
                            c->w0, c->nx, c->ny, x0, y0, c->dimx, c->dimy, c->dx, c->dy,
                            compat ? 1 : 0, c->rho_acc);

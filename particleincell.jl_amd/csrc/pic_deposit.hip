@@ -1,0 +1,239 @@
+// pic_deposit.hip -- the charge deposit of particles in any order, with the
+// whole grid's charge in LDS.
+//
+// Particles that are not sorted by cell put their charge anywhere, and one
+// FP64 global atomic per stencil node is what that costs.  Measured on MI355X,
+// scattered FP64 global atomics retire at 24e9/s while their targets span
+// 128 KiB, and at 1.3e9/s and 0.3e9/s over 320 KiB and 1 MiB; 204,800 M6
+// particles on 128 x 64 cells took 324 us.  Here block (chunk, r) takes a chunk
+// of the particles and sums the nodes of part r of the grid in LDS (one part
+// up to 20,480 nodes, at most DEP_PARTS_MAX), then stores its copy of that
+// part without atomics; k_deposit_reduce adds the copies in chunk order, and
+// sums the grid for the neutralising shift on the way.  Measured: those 204,800 particles 13
+// us, and 9 for the reduction; 10,000,000 unsorted M6 particles on 128 x 128
+// cells 0.29 ms for the whole call, on 256 x 256 (four parts) 0.71 ms.
+//
+// With R parts every chunk is read and its weights formed R times, so past
+// DEP_PARTS_MAX parts the chunk kernels of pic_step.hip serve; and for particles
+// that a sort put near their cells' order (Ctx::near_order), whose chunks cover
+// small boxes: measured on lane-sorted M6 particles they take as long as one
+// part does (10,000,000 on 128 x 128: 195 against 174 us; 300,000 CIC on 100 x
+// 100: 28 against 36) and less than several (2,000,000 on 400 x 400: 71 us
+// against 363).
+#include <algorithm>
+
+#include "pic_internal.h"
+#include "pic_push64.h"
+
+namespace pic {
+
+namespace {
+
+constexpr int DT = 1024;
+constexpr size_t DEP_LDS = 160 * 1024;
+
+// How a position gives a cell and an in-cell offset, and where the weights go.
+//   DEP_REF     compute_rho(p, kernel, mesh): pushers_cic.jl:84-105 (trunc for
+//               CIC), pushers_m6.jl:246-338 (floor)
+//   DEP_MF      the MeshFields M6 deposit at x - x0, in [0, dimx]
+//               (compute_rho_m6.jl:70-81)
+//   DEP_COMPAT  the same with the reference's neighbour indices of
+//               compute_rho_m6!(fields, particles) (:216-227), every
+//               off-centre weight one node low
+enum { DEP_REF, DEP_MF, DEP_COMPAT };
+
+struct DepArgs {
+    int64_t n;
+    const double *x, *y, *w;  // w null: w0
+    double w0, x0, y0, dx, dy;
+    int nx, ny;
+    double *copies;           // chunk c's grid at c * nx * ny
+    int chunks, parts, len;   // len nodes per part
+};
+
+template <int K, int HOW, bool SPLIT>
+__global__ __launch_bounds__(DT) void k_deposit_lds(DepArgs a) {
+    extern __shared__ double lds[];
+    constexpr int S = Shape<K>::S, HL = Shape<K>::HL;
+    const int nx = a.nx, ny = a.ny, tid = threadIdx.x;
+    const int chunk = SPLIT ? blockIdx.x / a.parts : blockIdx.x;
+    const int r0 = SPLIT ? blockIdx.x - chunk * a.parts : 0;
+    const int lo = r0 * a.len, len = min(a.len, nx * ny - lo);
+    const int64_t p0 = a.n * chunk / a.chunks, p1 = a.n * (chunk + 1) / a.chunks;
+    double x = 0.0, y = 0.0, w = 0.0;
+    auto load = [&](int64_t k) {
+        x = a.x[k];
+        y = a.y[k];
+        w = a.w ? a.w[k] : a.w0;
+    };
+    if (p0 + tid < p1) load(p0 + tid);
+    for (int t = tid; t < len; t += DT) lds[t] = 0.0;
+    __syncthreads();
+    for (int64_t k = p0 + tid; k < p1; k += DT) {
+        double fx, fy;
+        int ci, cj;
+        if (HOW == DEP_REF) {
+            ci = ref_cell_s(x, a.dx, nx, K == PIC_CIC, fx);
+            cj = ref_cell_s(y, a.dy, ny, K == PIC_CIC, fy);
+        } else {
+            const double px = (x - a.x0) / a.dx, py = (y - a.y0) / a.dy;
+            ci = (int)px;
+            cj = (int)py;
+            fx = px - (double)ci;
+            fy = py - (double)cj;
+        }
+        const double wk = w;
+        if (k + DT < p1) load(k + DT);
+        int col[S], row[S];
+#pragma unroll
+        for (int u = 0; u < S; ++u) {
+            const int o = u - HL - (HOW == DEP_COMPAT && u != HL ? 1 : 0);
+            col[u] = picd::wrap2(ci + o, nx);
+            row[u] = picd::wrap2(cj + o, ny);
+            // a position outside the domain (NaN, or one no call wrapped)
+            // must not leave the grid
+            if (HOW != DEP_REF) {
+                col[u] = min(max(col[u], 0), nx - 1);
+                row[u] = min(max(row[u], 0), ny - 1);
+            }
+            row[u] = row[u] * nx - lo;
+        }
+        charge64<K>(fx, fy, ci, cj, wk, [&](int u, int v, double q) {
+            const int t = row[v] + col[u];
+            if (SPLIT && (unsigned)t >= (unsigned)len) return;
+            __hip_atomic_fetch_add(&lds[t], q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        });
+    }
+    __syncthreads();
+    double *out = a.copies + (size_t)chunk * nx * ny + lo;
+    for (int t = tid; t < len; t += DT) out[t] = lds[t];
+}
+
+// acc[t] = the copies' sum, 64 nodes per block, W waves each taking every W-th
+// chunk, the waves' sums added in order; *total = the sum of acc (a wave
+// butterfly, then the blocks in a fixed order by the last one to arrive).
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_deposit_reduce(const double *__restrict__ copies,
+                                                           int chunks, int m,
+                                                           double *__restrict__ acc, double *part,
+                                                           unsigned *count, double *total) {
+    __shared__ double sh[64 * W];
+    __shared__ bool last;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int t = blockIdx.x * 64 + lane;
+    double s = 0.0;
+    if (t < m) {
+#pragma unroll 8
+        for (int b = wv; b < chunks; b += W) s += copies[(size_t)b * m + t];
+    }
+    sh[tid] = s;
+    __syncthreads();
+    if (wv == 0) {
+        for (int k = 1; k < W; ++k) s += sh[64 * k + lane];
+        if (t < m) acc[t] = s;
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        if (lane == 0) {
+            part[blockIdx.x] = s;
+            __threadfence();
+            last = atomicAdd(count, 1u) == gridDim.x - 1;
+        }
+    }
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    s = 0.0;
+    for (int k = tid; k < (int)gridDim.x; k += 64 * W)
+        s += __hip_atomic_load(&part[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (lane == 0) sh[wv] = s;
+    __syncthreads();
+    if (tid == 0) {
+        for (int k = 1; k < W; ++k) s += sh[k];
+        *total = s;
+        *count = 0u;
+    }
+}
+
+constexpr int DEP_PARTS_MAX = 8;
+
+template <int K, int HOW>
+int launch(Ctx *c, const DepArgs &a) {
+    const size_t lds = (size_t)a.len * 8;
+    auto go = [&](auto kern) -> int {
+        PIC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kern, dim3((unsigned)(a.chunks * a.parts)), dim3(DT), lds, c->stream, a);
+        PIC_HIP(hipGetLastError());
+        return PIC_OK;
+    };
+    return a.parts == 1 ? go(k_deposit_lds<K, HOW, false>) : go(k_deposit_lds<K, HOW, true>);
+}
+
+int parts_of(const Ctx *c) {
+    const int64_t m = (int64_t)c->nx * c->ny, room = (int64_t)(DEP_LDS / 8);
+    return (int)std::min<int64_t>((m + room - 1) / room, DEP_PARTS_MAX + 1);
+}
+
+int deposit(Ctx *c, int kernel, int how, double x0, double y0) {
+    const int64_t m = (int64_t)c->nx * c->ny;
+    DepArgs a;
+    a.n = c->n;
+    a.x = c->x;
+    a.y = c->y;
+    a.w = c->uniform_w ? nullptr : c->w;
+    a.w0 = c->w0;
+    a.x0 = x0;
+    a.y0 = y0;
+    a.dx = c->dx;
+    a.dy = c->dy;
+    a.nx = c->nx;
+    a.ny = c->ny;
+    a.parts = parts_of(c);
+    a.len = (int)((m + a.parts - 1) / a.parts);
+    // one block per compute unit, at least a particle per thread
+    a.chunks = (int)std::max<int64_t>(1, std::min<int64_t>((c->n + DT - 1) / DT, c->ncu / a.parts));
+    const int nblk = (int)((m + 63) / 64);
+    PIC_TRY(ensure_copies(c, (int64_t)a.chunks * m + nblk));
+    a.copies = c->copies;
+    int rc = PIC_OK;
+    if (how == DEP_REF) {
+        PIC_SHAPE_SWITCH(kernel, rc = (launch<KK, DEP_REF>(c, a)));
+    } else if (how == DEP_MF) {
+        rc = launch<PIC_M6, DEP_MF>(c, a);
+    } else {
+        rc = launch<PIC_M6, DEP_COMPAT>(c, a);
+    }
+    PIC_TRY(rc);
+    double *part = c->copies + (size_t)a.chunks * m, *total = c->red_part + 2 * RED_BLOCKS;
+    auto reduce = [&](auto kern, int w) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(64 * w), 0, c->stream,
+                           (const double *)c->copies, a.chunks, (int)m, c->rho_acc, part,
+                           c->red_count, total);
+    };
+    if (a.chunks > 32) reduce(k_deposit_reduce<8>, 8);
+    else reduce(k_deposit_reduce<1>, 1);
+    PIC_HIP(hipGetLastError());
+    return shift_rho(c, kernel);
+}
+
+}  // namespace
+
+int ensure_copies(Ctx *c, int64_t count) {
+    if (count <= c->copies_cap) return PIC_OK;
+    if (c->copies) (void)hipFree(c->copies);
+    c->copies = nullptr;
+    c->copies_cap = 0;
+    PIC_HIP(hipMalloc(&c->copies, (size_t)count * 8));
+    c->copies_cap = count;
+    return PIC_OK;
+}
+
+bool deposit_lds_ok(const Ctx *c) { return c->n > 0 && parts_of(c) <= DEP_PARTS_MAX; }
+
+int deposit_rho(Ctx *c, int kernel) { return deposit(c, kernel, DEP_REF, 0.0, 0.0); }
+
+int deposit_rho_mf(Ctx *c, double x0, double y0, bool compat) {
+    return deposit(c, PIC_M6, compat ? DEP_COMPAT : DEP_MF, x0, y0);
+}
+
+}  // namespace pic

@@ -114,6 +114,8 @@ struct Ctx {
     // after a lane sort, segment s occupies slots [cell_off[64 s],
     // cell_off[min(64 s + 64, ncells)]) until the next sort
     bool seg_valid = false;             // cell_off describes the current slots
+    // a sort of either kind put the current particles near their cells' order
+    bool near_order = false;
     // the particles sit in the order the last lane sort left (or its pending
     // permutation gives) and have not moved since: pic_run can skip its own
     // first sort
@@ -160,11 +162,12 @@ struct Ctx {
     double *fd2_ex = nullptr, *fd2_ey = nullptr, *fd2_bz = nullptr;
     double *jb[4] = {nullptr, nullptr, nullptr, nullptr};  // J1 x, y, J2 x, y
     int vm_path = 0;  // pic_set_maxwell_path
-    // the three-launch iteration of larger grids: (ex, ey, bz, -) per node,
-    // and a copy of (jx, jy) per chunk of particles
+    // the three-launch iteration of larger grids: (ex, ey, bz, -) per node
     void *vm_nodes = nullptr;
-    double *vm_copies = nullptr;
-    int64_t vm_copies_cap = 0;
+    // a copy of the grid's charge, or of its current, per chunk of particles
+    // (ensure_copies)
+    double *copies = nullptr;
+    int64_t copies_cap = 0;
 
     // UA (ua_type.jl): ntau, eps; per particle b, t (Particles.b, .t), the
     // positions at the start of a UA step and, between its prediction and
@@ -174,6 +177,8 @@ struct Ctx {
     int64_t ua_cap = 0;
     double *ua_b = nullptr, *ua_t = nullptr, *ua_x0 = nullptr, *ua_y0 = nullptr;
     double *ua_fhat = nullptr;
+    void *ua_tab = nullptr;             // tables of ua_ntau entries
+    double *ua_e = nullptr;             // (ex, ey) interleaved FP64 per node
 
     // adjoint reverse sweep: steps whose positions are kept at once (0 =
     // the most the free device memory allows), and the last sweep's plan
@@ -210,15 +215,30 @@ int ensure_defer(Ctx *c);
 // ------------------------------------------------------ module entry points
 int poisson_init(Ctx *c);
 void poisson_free(Ctx *c);
-int poisson_solve_e(Ctx *c, const double *rho_in, double scale, int make_e32, int energy_slot);
+int poisson_solve_e(Ctx *c, const double *rho_in, double scale, int make_e32, int energy_slot,
+                    double2 *e2 = nullptr);
 int poisson_solve_phi(Ctx *c);
 int poisson_adjoint(Ctx *c, const double *lex, const double *ley, double *lrho, double scale);
 int finalize_rho(Ctx *c, int kernel);
+// finalize_rho's second half: rho from rho_acc and its sum, which the caller
+// left in red_part[2 RED_BLOCKS].
+int shift_rho(Ctx *c, int kernel);
+// compute_rho of the FP64 state's particles, in any order, on grids whose
+// charge fits LDS in a few parts (deposit_lds_ok): rho_acc and rho.
+// deposit_rho_mf: the MeshFields M6 deposit at x - x0, y - y0.
+bool deposit_lds_ok(const Ctx *c);
+int deposit_rho(Ctx *c, int kernel);
+int deposit_rho_mf(Ctx *c, double x0, double y0, bool compat);
+int ensure_copies(Ctx *c, int64_t count);
 int field_energy(Ctx *c, double *out2);
-// Queues meshfields.jl:105-106's energy sums of the current ex, ey: the
-// interior sums times dx dy into energy_hist[2 slot], [2 slot + 1] and the
-// ghost-node terms (without dx dy) into the device double *ghost.  No wait.
-int field_energy_async(Ctx *c, int slot, double *ghost);
+// Queues solve!(fields, poisson): E from rho, and with slot >= 0
+// meshfields.jl:105-106's energy sums: the interior sums times dx dy into
+// energy_hist[2 slot], [2 slot + 1] and the ghost-node terms (without dx dy)
+// into the device double *ghost.  No wait.
+// e2 (may be null) also receives (ex, ey) side by side per node.
+int solve_fields_async(Ctx *c, int slot, double *ghost, double2 *e2 = nullptr);
+// (ex, ey) side by side per node, from the context's fields.
+int interleave_fields(Ctx *c, double2 *e2);
 
 // Stable sort by cell (lanes: then the lane-spread order of the segment
 // passes).  apply = false with lanes leaves the permutation pending in

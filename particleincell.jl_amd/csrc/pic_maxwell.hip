@@ -1116,22 +1116,14 @@ VmPartPlan vm_part_plan(const Ctx *c) {
 int ensure_part_buffers(Ctx *c, const VmPartPlan &p) {
     const size_t m = (size_t)c->nx * c->ny;
     if (!c->vm_nodes) PIC_HIP(hipMalloc(&c->vm_nodes, m * sizeof(VmNode)));
-    const int64_t need = (int64_t)p.chunks * 2 * (int64_t)m;
-    if (need > c->vm_copies_cap) {
-        if (c->vm_copies) (void)hipFree(c->vm_copies);
-        c->vm_copies = nullptr;
-        c->vm_copies_cap = 0;
-        PIC_HIP(hipMalloc(&c->vm_copies, (size_t)need * 8));
-        c->vm_copies_cap = need;
-    }
-    return PIC_OK;
+    return ensure_copies(c, (int64_t)p.chunks * 2 * (int64_t)m);
 }
 
 int vm_pass_part(Ctx *c, double dt, const VmPartPlan &p) {
     VmArgs a = vm_args(c, dt);
     VmPart q;
     q.nodes = static_cast<const VmNode *>(c->vm_nodes);
-    q.copies = c->vm_copies;
+    q.copies = c->copies;
     q.chunks = p.chunks;
     q.parts = p.parts;
     q.len = p.len;
@@ -1415,7 +1407,7 @@ int pic_run_maxwell(pic_ctx *ctx, int kernel, double dt, int nsteps, double *ene
             auto reduce = [&](auto kern, int w) {
                 hipLaunchKernelGGL(kern, dim3((unsigned)((2 * m + 63) / 64)), dim3(64 * w), 0,
                                    c->stream, c->nx, c->ny, c->dx, c->dy, 0.5 * dt,
-                                   (const double *)c->vm_copies, pp.chunks, c->jx, c->jy,
+                                   (const double *)c->copies, pp.chunks, c->jx, c->jy,
                                    (const double *)ex[in], (const double *)ey[in],
                                    (const double *)c->fd_bz, c->fd2_bz);
             };
@@ -1476,6 +1468,7 @@ int pic_run_maxwell(pic_ctx *ctx, int kernel, double dt, int nsteps, double *ene
     }
     for (hipEvent_t e : ev) (void)hipEventDestroy(e);
     c->seg_valid = false;
+    c->near_order = false;
     c->sort_fresh = false;
     return rc;
 }

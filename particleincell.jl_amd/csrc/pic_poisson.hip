@@ -226,8 +226,8 @@ __device__ __forceinline__ void block_sum2(double &a, double &b, double *sh) {
 }
 
 // After the inverse transform: (ex, ey) from z (real, imaginary parts) when z
-// is given, else read from ex, ey; optional FP32 interleaved copy, optional
-// zeroing of the raw deposit accumulator for the next step, and the energy
+// is given, else read from ex, ey; optional FP32 and FP64 (e2) interleaved
+// copies, optional zeroing of the raw deposit accumulator for the next step, and the energy
 // sums sum(ex^2)*dxdy, sum(ey^2)*dxdy written by the last block to arrive
 // into hist[2*slot] (slot >= 0), hist[2*(*counter)] with *counter
 // incremented (slot == -2) or nowhere (slot == -1).  Partial sums are per
@@ -239,7 +239,8 @@ __global__ __launch_bounds__(RED_THREADS) void k_post(const double2 *__restrict_
                                                       float2 *__restrict__ e32,
                                                       double *__restrict__ zero_acc,
                                                       double *part, unsigned *count, double *hist,
-                                                      int slot, int *counter, double dxdy) {
+                                                      int slot, int *counter, double dxdy,
+                                                      double2 *__restrict__ e2) {
     __shared__ double sh[2 * RED_THREADS];
     __shared__ bool last;
     double sx = 0.0, sy = 0.0;
@@ -259,6 +260,7 @@ __global__ __launch_bounds__(RED_THREADS) void k_post(const double2 *__restrict_
         sx += a * a;
         sy += b * b;
         if (e32) e32[k] = make_float2((float)a, (float)b);
+        if (e2) e2[k] = make_double2(a, b);
         if (zero_acc) zero_acc[k] = 0.0;
     }
     block_sum2<RED_THREADS>(sx, sy, sh);
@@ -472,7 +474,8 @@ __global__ __launch_bounds__(FFT_T) void k_fft_rows_inv(
     const double2 *__restrict__ B, int nx, int ny, int lognx, const double2 *__restrict__ tw,
     double *__restrict__ ex,
     double *__restrict__ ey, float2 *__restrict__ e32, double *__restrict__ zero_acc,
-    double *part, unsigned *count, double *hist, int slot, int *counter, double dxdy) {
+    double *part, unsigned *count, double *hist, int slot, int *counter, double dxdy,
+    double2 *__restrict__ e2) {
     extern __shared__ double2 fsm[];
     __shared__ double sh[2 * FFT_T];
     __shared__ bool last;
@@ -492,6 +495,7 @@ __global__ __launch_bounds__(FFT_T) void k_fft_rows_inv(
             sx += a * a;
             sy += b * b;
             if (e32) e32[k] = make_float2((float)a, (float)b);
+            if (e2) e2[k] = make_double2(a, b);
             if (zero_acc) zero_acc[k] = 0.0;
         }
     }
@@ -585,7 +589,7 @@ __global__ __launch_bounds__(64) void k_wrows_inv(
     const double2 *__restrict__ B, int nx, int ny, int lognx, const double2 *__restrict__ tw,
     double *__restrict__ ex, double *__restrict__ ey, float2 *__restrict__ e32,
     double *__restrict__ zero_acc, double *part, unsigned *count, double *hist, int slot,
-    int *counter, double dxdy) {
+    int *counter, double dxdy, double2 *__restrict__ e2) {
     __shared__ double2 w[256];
     __shared__ double sh[2 * FFT_T];
     __shared__ bool last;
@@ -607,6 +611,7 @@ __global__ __launch_bounds__(64) void k_wrows_inv(
             sx += a * a;
             sy += b * b;
             if (e32) e32[k] = make_float2((float)a, (float)b);
+            if (e2) e2[k] = make_double2(a, b);
             if (zero_acc) zero_acc[k] = 0.0;
         }
     }
@@ -637,7 +642,8 @@ static void with_points(int n, F &&f) {
     }
 }
 
-static int solve_e_wave(Ctx *c, const double *rho_in, double scale, int post, int energy_slot) {
+static int solve_e_wave(Ctx *c, const double *rho_in, double scale, int post, int energy_slot,
+                        double2 *e2) {
     const int nx = c->nx, ny = c->ny, lx = log2_exact(nx), ly = log2_exact(ny);
     double2 *At = c->zf, *B = c->zg;  // (nx/2+1) x ny column-major; nx x ny
     const double2 *twx = (const double2 *)c->fft_tw, *twy = twx + nx;
@@ -656,7 +662,7 @@ static int solve_e_wave(Ctx *c, const double *rho_in, double scale, int post, in
                            c->stream, (const double2 *)B, nx, ny, lx, twx, c->ex, c->ey,
                            (post & 1) ? (float2 *)c->e32 : nullptr,
                            (post & 2) ? c->rho_acc : nullptr, c->red_part, c->red_count,
-                           c->energy_hist, energy_slot, c->step_counter, c->dx * c->dy);
+                           c->energy_hist, energy_slot, c->step_counter, c->dx * c->dy, e2);
     });
     PIC_HIP(hipGetLastError());
     return PIC_OK;
@@ -672,10 +678,11 @@ static int fft_tw_init(Ctx *c) {
     return PIC_OK;
 }
 
-static int solve_e_fused(Ctx *c, const double *rho_in, double scale, int post, int energy_slot) {
+static int solve_e_fused(Ctx *c, const double *rho_in, double scale, int post, int energy_slot,
+                         double2 *e2) {
     const int nx = c->nx, ny = c->ny, lx = log2_exact(nx), ly = log2_exact(ny);
     double2 *At = c->zf, *B = c->zg;  // (nx/2+1) x ny column-major; nx x ny
-    if (lx >= 6 && ly >= 6) return solve_e_wave(c, rho_in, scale, post, energy_slot);
+    if (lx >= 6 && ly >= 6) return solve_e_wave(c, rho_in, scale, post, energy_slot, e2);
     hipLaunchKernelGGL(k_fft_rows_fwd, dim3((unsigned)ny), dim3(FFT_T),
                        (size_t)(nx + nx / 2) * sizeof(double2), c->stream, rho_in, nx, ny, lx,
                        (const double2 *)c->fft_tw, At);
@@ -689,7 +696,7 @@ static int solve_e_fused(Ctx *c, const double *rho_in, double scale, int post, i
                        nx, ny, lx, (const double2 *)c->fft_tw, c->ex, c->ey,
                        (post & 1) ? (float2 *)c->e32 : nullptr,
                        (post & 2) ? c->rho_acc : nullptr, c->red_part, c->red_count,
-                       c->energy_hist, energy_slot, c->step_counter, c->dx * c->dy);
+                       c->energy_hist, energy_slot, c->step_counter, c->dx * c->dy, e2);
     PIC_HIP(hipGetLastError());
     return PIC_OK;
 }
@@ -706,9 +713,10 @@ static int spectral(Ctx *c, double scale) {
 // rho_in (nx*ny real) -> ex, ey.  post: bit 0 writes the FP32 interleaved
 // field copy, bit 1 clears the raw deposit accumulator (after the forward
 // transform has read it).  energy_slot as in k_post.
-int poisson_solve_e(Ctx *c, const double *rho_in, double scale, int post, int energy_slot) {
+int poisson_solve_e(Ctx *c, const double *rho_in, double scale, int post, int energy_slot,
+                    double2 *e2) {
     if (c->fused_solve && fused_solve_ok(c))
-        return solve_e_fused(c, rho_in, scale, post, energy_slot);
+        return solve_e_fused(c, rho_in, scale, post, energy_slot, e2);
     const int64_t mm = (int64_t)c->nx * c->ny;
     hipLaunchKernelGGL(k_pack, grid_of(mm), dim3(256), 0, c->stream, rho_in, (const double *)nullptr,
                        mm, c->zf);
@@ -721,7 +729,7 @@ int poisson_solve_e(Ctx *c, const double *rho_in, double scale, int post, int en
     hipLaunchKernelGGL(k_post, dim3(blocks), dim3(RED_THREADS), 0, c->stream, c->zg, c->ex, c->ey,
                        mm, (post & 1) ? (float2 *)c->e32 : nullptr,
                        (post & 2) ? c->rho_acc : nullptr, c->red_part, c->red_count,
-                       c->energy_hist, energy_slot, c->step_counter, c->dx * c->dy);
+                       c->energy_hist, energy_slot, c->step_counter, c->dx * c->dy, e2);
     PIC_HIP(hipGetLastError());
     return PIC_OK;
 }
@@ -807,6 +815,13 @@ int finalize_rho(Ctx *c, int kernel) {
     double *tot = c->red_part + 2 * RED_BLOCKS;  // spare slot after the partials
     hipLaunchKernelGGL(k_sum, dim3(blocks), dim3(RED_THREADS), 0, c->stream, c->rho_acc, m,
                        c->red_part, c->red_count, tot);
+    PIC_HIP(hipGetLastError());
+    return shift_rho(c, kernel);
+}
+
+int shift_rho(Ctx *c, int kernel) {
+    const int64_t m = (int64_t)c->nx * c->ny;
+    const double *tot = c->red_part + 2 * RED_BLOCKS;
     hipLaunchKernelGGL(k_finalize_rho, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, c->stream,
                        c->rho_acc, c->rho, m, c->dx * c->dy, tot, kernel, c->dx, c->dy, c->dimx,
                        c->dimy);
@@ -815,29 +830,34 @@ int finalize_rho(Ctx *c, int kernel) {
 }
 
 // The ghost-node terms of meshfields.jl:105-106's energy sum: column i = 0,
-// row j = 0, then node (0,0) once more, added in that order by one thread
-// (the order of a sequential loop over the nodes, so the sum does not depend
-// on the launch).
-__global__ void k_ghost_energy(const double *__restrict__ ex, const double *__restrict__ ey,
-                               int nx, int ny, double *out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// row j = 0, then node (0,0) once more.  One wave, each lane every 64th node,
+// the lanes added by a butterfly: the same order on every run.  (One thread
+// adding the nodes in turn took 20.7 us at 128 x 64, each a global load after
+// the last.)
+__global__ __launch_bounds__(64) void k_ghost_energy(const double *__restrict__ ex,
+                                                     const double *__restrict__ ey, int nx, int ny,
+                                                     double *out) {
     double g = 0.0;
-    for (int j = 0; j < ny; ++j) {
+    for (int j = threadIdx.x; j < ny; j += 64) {
         const int64_t k = (int64_t)nx * j;
         g += ex[k] * ex[k] + ey[k] * ey[k];
     }
-    for (int i = 0; i < nx; ++i) g += ex[i] * ex[i] + ey[i] * ey[i];
-    g += ex[0] * ex[0] + ey[0] * ey[0];
-    *out = g;
+    for (int i = threadIdx.x; i < nx; i += 64) g += ex[i] * ex[i] + ey[i] * ey[i];
+    for (int o = 32; o > 0; o >>= 1) g += __shfl_xor(g, o);
+    if (threadIdx.x == 0) *out = g + (ex[0] * ex[0] + ey[0] * ey[0]);
 }
 
-int field_energy_async(Ctx *c, int slot, double *ghost) {
+int interleave_fields(Ctx *c, double2 *e2) {
     const int64_t mm = (int64_t)c->nx * c->ny;
-    int blocks = (int)((mm + RED_THREADS - 1) / RED_THREADS);
-    if (blocks > RED_BLOCKS) blocks = RED_BLOCKS;
-    hipLaunchKernelGGL(k_post, dim3(blocks), dim3(RED_THREADS), 0, c->stream,
-                       (const double2 *)nullptr, c->ex, c->ey, mm, nullptr, nullptr, c->red_part,
-                       c->red_count, c->energy_hist, slot, c->step_counter, c->dx * c->dy);
+    hipLaunchKernelGGL(k_pack, grid_of(mm), dim3(256), 0, c->stream, (const double *)c->ex,
+                       (const double *)c->ey, mm, e2);
+    PIC_HIP(hipGetLastError());
+    return PIC_OK;
+}
+
+int solve_fields_async(Ctx *c, int slot, double *ghost, double2 *e2) {
+    PIC_TRY(poisson_solve_e(c, c->rho, 1.0 / ((double)c->nx * (double)c->ny), 1, slot, e2));
+    if (slot < 0) return PIC_OK;
     hipLaunchKernelGGL(k_ghost_energy, dim3(1), dim3(64), 0, c->stream, c->ex, c->ey, c->nx,
                        c->ny, ghost);
     PIC_HIP(hipGetLastError());
@@ -851,7 +871,8 @@ int field_energy(Ctx *c, double *out2) {
     if (blocks > RED_BLOCKS) blocks = RED_BLOCKS;
     hipLaunchKernelGGL(k_post, dim3(blocks), dim3(RED_THREADS), 0, c->stream,
                        (const double2 *)nullptr, c->ex, c->ey, mm, nullptr, nullptr, c->red_part,
-                       c->red_count, c->energy_hist, 0, c->step_counter, c->dx * c->dy);
+                       c->red_count, c->energy_hist, 0, c->step_counter, c->dx * c->dy,
+                       (double2 *)nullptr);
     PIC_HIP(hipGetLastError());
     PIC_HIP(hipMemcpyAsync(out2, c->energy_hist, 2 * sizeof(double), hipMemcpyDeviceToHost,
                            c->stream));
@@ -894,14 +915,14 @@ int pic_solve_fields(pic_ctx *ctx, double *energy) {
     PIC_CHECK(ctx, PIC_ERR_ARG, "null context");
     Ctx *c = ctx_of(ctx);
     PIC_HIP(hipSetDevice(c->device));
-    PIC_TRY(poisson_solve_e(c, c->rho, 1.0 / ((double)c->nx * (double)c->ny), 1, -1));
+    if (!energy) PIC_TRY(solve_fields_async(c, -1, nullptr));
     if (energy) {
         // meshfields.jl:105-106 sums over the (nx+1)(ny+1) ghosted nodes: the
         // interior, plus column i = 0 and row j = 0 again, plus node (0,0) a
-        // third time (the ghost corner).  Interior sums (k_post) and ghost
+        // third time (the ghost corner).  Interior sums (the solve's) and ghost
         // terms (k_ghost_energy) on the device, one copy of three values.
         PIC_TRY(ensure_energy(c, 2));
-        PIC_TRY(field_energy_async(c, 0, c->energy_hist + 2));
+        PIC_TRY(solve_fields_async(c, 0, c->energy_hist + 2));
         double s[3];
         PIC_HIP(hipMemcpyAsync(s, c->energy_hist, 3 * sizeof(double), hipMemcpyDeviceToHost,
                                c->stream));

@@ -706,6 +706,7 @@ int sort_by_cell(Ctx *c, int32_t *perm_host, bool lanes, bool apply) {
         PIC_HIP(hipStreamSynchronize(c->stream));
     }
     c->sort_fresh = lanes;
+    c->near_order = true;
     return PIC_OK;
 }
 

@@ -7,15 +7,31 @@
 // A particle is worked by ntau consecutive lanes of one wave, lane m holding
 // the tau-sample m of its (ntau, 2) arrays; the reference's (ntau, 2, n)
 // layout is then read and written coalesced.  The tau-FFTs are radix-2
-// transforms across those lanes with wave shuffles (FFTW's signs; the inverse
-// scales by 1/ntau as Julia's ifft does).  The fused loop keeps between the
-// prediction and the correction only the positions at the step's start and
-// the tau-spectra of fx, fy; everything else is recomputed from them with the
-// same operations, so it is bit-identical to what the reference holds.
+// transforms across those lanes (FFTW's signs; the inverse scales by 1/ntau
+// as Julia's ifft does): decimation in frequency forward, in time backward, so
+// that a spectrum stays in the bit-reversed order it comes out in, lane m
+// holding the frequency of bitrev(m), and no permutation is needed between the
+// two.  What a transform would only undo or what is known in closed form is
+// not transformed (see ua_prep and k_ua_predict).
+//
+// The kernels are bound by FP64 VALU issue: 16 samples of a particle at ntau
+// 16 are 16 lanes, so every instruction counts per sample.  Transforms with
+// general lane shuffles, selects and a bit-reversal each, 18 of them in the
+// prediction and 20 in the correction, and twiddles, cosines and FP64
+// divisions formed anew for every particle took 304 and 458 us (204,800
+// particles, 128 x 64 cells, ntau 16, deposit not counted) against 190 and 215
+// now: 1,209 and 1,701 VALU instructions per wave, 57 % and 72 % of the issue
+// rate, the rest waiting for the gather's nodes.  Three waves per SIMD: at
+// four the correction spills (269 us).
+//
+// The fused loop keeps between the prediction and the correction only the
+// positions at the step's start and the tau-spectra of fx, fy; everything else
+// is recomputed from them.
 #include <algorithm>
 #include <cmath>
 #include <vector>
 
+#include "pic_fftlanes.h"
 #include "pic_internal.h"
 
 namespace pic {
@@ -23,6 +39,7 @@ namespace pic {
 namespace {
 
 constexpr int UB = 256;  // threads per block
+constexpr int UA_WAVES = 3;
 
 struct cd {
     double re, im;
@@ -37,9 +54,8 @@ __device__ __forceinline__ cd operator*(double s, cd a) { return {s * a.re, s * 
 __device__ __forceinline__ cd operator/(cd a, double s) { return {a.re / s, a.im / s}; }
 __device__ __forceinline__ cd operator+(double s, cd a) { return {s + a.re, a.im}; }
 
-__device__ __forceinline__ cd shfl_xor(cd z, int mask) {
-    return {__shfl_xor(z.re, mask), __shfl_xor(z.im, mask)};
-}
+// Keeps the computation of x where it is written.
+__device__ __forceinline__ void pin(double &x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ cd shfl(cd z, int src) { return {__shfl(z.re, src), __shfl(z.im, src)}; }
 
 template <int NT>
@@ -52,69 +68,144 @@ __device__ __forceinline__ int bitrev(int m) {
 
 constexpr int ilog2(int n) { return n <= 1 ? 0 : 1 + ilog2(n / 2); }
 
-// This lane's twiddle of every FFT stage: stage h = NT/2, NT/4, ..., 1 uses
-// cos(pi j / h) and sin(pi j / h), j = m mod h (computed once per kernel).
+// a / b for a divisor used several times: with r = 1/b rounded, q = a r and
+// one correction by the exact remainder a - q b give the rounded quotient
+// (Markstein), 3 operations against about 14 of a division.
+struct Div {
+    double b, r;
+    __host__ __device__ Div() {}
+    __host__ __device__ explicit Div(double b_) : b(b_), r(1.0 / b_) {}
+    __device__ Div(double b_, double r_) : b(b_), r(r_) {}
+    __device__ __forceinline__ double of(double a) const {
+        const double q = a * r;
+        return __builtin_fma(__builtin_fma(-q, b, a), r, q);
+    }
+    __device__ __forceinline__ cd of(cd a) const { return {of(a.re), of(a.im)}; }
+};
+
+// Tables of ntau entries, made once for an ntau (k_ua_tables): cos and sin of
+// tau[k] = k dtau and 1/ltau[k], 1/ltau[k]^2 (ua_type.jl:18-24; 1 at k = 0),
+// cos and sin of 2 pi k / ntau.
+struct UaTable {
+    double c, s, rl, rl2, wc, ws;
+};
+__global__ void k_ua_tables(int nt, UaTable *t) {
+    const int k = threadIdx.x;
+    if (k >= nt) return;
+    const double l = k == 0 ? 1.0 : k < nt / 2 ? (double)k : (double)(k - nt);
+    sincos((double)k * (2 * M_PI / nt), &t[k].s, &t[k].c);
+    sincospi((double)(2 * k) / nt, &t[k].ws, &t[k].wc);
+    t[k].rl = 1.0 / l;
+    t[k].rl2 = 1.0 / (l * l);
+}
+
+// This lane's constants of UA(ntau, eps): cos(tau[m]), sin(tau[m]); ltau of
+// the frequency bitrev(m) it holds of a spectrum, and its square, as divisors
+// (1 at frequency 0); the lane that holds the opposite frequency; and of every
+// transform stage h the sign of its own value, -1 in the upper half of a pair,
+// and its twiddle exp(-pi i (m mod h) / h) there (1 in the lower half).
 template <int NT>
-struct Twiddles {
-    double c[ilog2(NT)], s[ilog2(NT)];
-    __device__ explicit Twiddles(int m) {
-        int q = 0;
+struct UaLane {
+    static constexpr int LOG = ilog2(NT);
+    int m, base, mirror;
+    double l, c, s;
+    Div dl, dl2;
+    double sg[LOG], wr[LOG], wi[LOG];
+    __device__ UaLane(const UaTable *__restrict__ t, int m_, int base_) : m(m_), base(base_) {
+        const int k = bitrev<NT>(m);
+        l = k < NT / 2 ? (double)k : (double)(k - NT);
+        mirror = base + bitrev<NT>((NT - k) & (NT - 1));
+        c = t[m].c;
+        s = t[m].s;
+        dl = Div(k == 0 ? 1.0 : l, t[k].rl);
+        dl2 = Div(k == 0 ? 1.0 : l * l, t[k].rl2);
 #pragma unroll
-        for (int h = NT / 2; h >= 1; h >>= 1, ++q)
-            sincospi((double)(m & (h - 1)) / (double)h, &s[q], &c[q]);
+        for (int q = 0; q < LOG; ++q) {
+            const int h = 1 << q;
+            const bool up = (m & h) != 0;
+            const int j = up ? (m & (h - 1)) * (NT / (2 * h)) : 0;
+            sg[q] = up ? -1.0 : 1.0;
+            wr[q] = t[j].wc;
+            wi[q] = -t[j].ws;
+        }
     }
 };
 
-// Radix-2 decimation-in-frequency FFT over the NT lanes of a group (lane m
-// holds element m in and out): forward exp(-2 pi i jk / NT), or the inverse
-// with exp(+...) scaled by 1/NT.
-template <int NT, bool INV>
-__device__ __forceinline__ cd fft_lanes(cd z, int m, int base, const Twiddles<NT> &w) {
-    int q = 0;
-#pragma unroll
-    for (int h = NT / 2; h >= 1; h >>= 1, ++q) {
-        // lower lane: z + p; upper lane: (p - z) w, without a branch
-        const cd p = shfl_xor(z, h);
-        const bool up = (m & h) != 0;
-        const cd d = up ? p - z : z + p;
-        z = up ? d * mk(w.c[q], INV ? w.s[q] : -w.s[q]) : d;
-    }
-    z = shfl(z, base + bitrev<NT>(m));
-    if (INV) z = mk(z.re * (1.0 / NT), z.im * (1.0 / NT));
+template <int H>
+__device__ __forceinline__ cd xor_cd(cd z) {
+    return {xor_lane<H>(z.re), xor_lane<H>(z.im)};
+}
+
+// One stage of distance H = 2^Q: the lower lane of a pair takes a + b, the
+// upper (a - b) w forward, a + b w backward (conj w).
+template <int NT, int Q, bool INV>
+__device__ __forceinline__ cd fft_pair(cd z, const UaLane<NT> &L) {
+    const double wi = INV ? -L.wi[Q] : L.wi[Q];
+    if (INV && Q > 0)
+        z = {__builtin_fma(z.re, L.wr[Q], -(z.im * wi)), __builtin_fma(z.re, wi, z.im * L.wr[Q])};
+    const cd p = xor_cd<(1 << Q)>(z);
+    z = {__builtin_fma(L.sg[Q], z.re, p.re), __builtin_fma(L.sg[Q], z.im, p.im)};
+    if (!INV && Q > 0)
+        z = {__builtin_fma(z.re, L.wr[Q], -(z.im * wi)), __builtin_fma(z.re, wi, z.im * L.wr[Q])};
     return z;
+}
+
+// Forward: lane m's sample in, frequency bitrev(m) out.
+template <int NT>
+__device__ __forceinline__ cd fft_fwd(cd z, const UaLane<NT> &L) {
+    if constexpr (NT >= 64) z = fft_pair<NT, 5, false>(z, L);
+    if constexpr (NT >= 32) z = fft_pair<NT, 4, false>(z, L);
+    if constexpr (NT >= 16) z = fft_pair<NT, 3, false>(z, L);
+    if constexpr (NT >= 8) z = fft_pair<NT, 2, false>(z, L);
+    if constexpr (NT >= 4) z = fft_pair<NT, 1, false>(z, L);
+    return fft_pair<NT, 0, false>(z, L);
+}
+
+// Backward, scaled by 1/NT: frequency bitrev(m) in, sample m out.
+template <int NT>
+__device__ __forceinline__ cd fft_inv(cd z, const UaLane<NT> &L) {
+    z = fft_pair<NT, 0, true>(z, L);
+    if constexpr (NT >= 4) z = fft_pair<NT, 1, true>(z, L);
+    if constexpr (NT >= 8) z = fft_pair<NT, 2, true>(z, L);
+    if constexpr (NT >= 16) z = fft_pair<NT, 3, true>(z, L);
+    if constexpr (NT >= 32) z = fft_pair<NT, 4, true>(z, L);
+    if constexpr (NT >= 64) z = fft_pair<NT, 5, true>(z, L);
+    return mk(z.re * (1.0 / NT), z.im * (1.0 / NT));
+}
+
+// The value lane bitrev(m) of the group holds: a spectrum between its
+// bit-reversed and the reference's order (either way).
+template <int NT>
+__device__ __forceinline__ cd reorder(cd z, const UaLane<NT> &L) {
+    return shfl(z, L.base + bitrev<NT>(L.m));
 }
 
 // Sum over the NT lanes of a group (every lane receives it).
 template <int NT>
-__device__ __forceinline__ cd lane_sum(cd z) {
-#pragma unroll
-    for (int h = 1; h < NT; h <<= 1) z = z + shfl_xor(z, h);
+__device__ __forceinline__ double lane_sum(double z) {
+    z += xor_lane<1>(z);
+    if constexpr (NT >= 4) z += xor_lane<2>(z);
+    if constexpr (NT >= 8) z += xor_lane<4>(z);
+    if constexpr (NT >= 16) z += xor_lane<8>(z);
+    if constexpr (NT >= 32) z += xor_lane<16>(z);
+    if constexpr (NT >= 64) z += xor_lane<32>(z);
     return z;
 }
-
-// Per-lane constants of UA(ntau, eps): tau = m dtau, ltau (ua_type.jl:18-24),
-// and the lane's FFT twiddles.
 template <int NT>
-struct UaLane {
-    int m;
-    double l, c, s;  // ltau[m], cos(tau[m]), sin(tau[m])
-    Twiddles<NT> w;
-    __device__ explicit UaLane(int m_) : m(m_), w(m_) {
-        l = m < NT / 2 ? (double)m : (double)(m - NT);
-        const double tau = (double)m * (2 * M_PI / NT);
-        sincos(tau, &s, &c);
-    }
-};
+__device__ __forceinline__ cd lane_sum(cd z) {
+    return {lane_sum<NT>(z.re), lane_sum<NT>(z.im)};
+}
 
-// exp(sg 1im l t / eps) as Julia evaluates it: cis(((sg l) t) / eps).
-__device__ __forceinline__ cd ua_cis(int sg, double l, double t, double eps) {
-    const double th = (((double)sg * l) * t) / eps;
+// exp(-1im l t / eps) as Julia evaluates it: cis(((-l) t) / eps).
+__device__ __forceinline__ cd ua_cis(double l, double t, Div eps) {
+    const double th = eps.of(-l * t);
     double s, c;
     sincos(th, &s, &c);
     return mk(c, s);
 }
 
-// pl[m], ql[m] of preparation! (ua_steps.jl:26-33); elt = exp(-1im l t / eps).
+// pl, ql of preparation! (ua_steps.jl:26-33) at this lane's frequency; elt =
+// exp(-1im l t / eps).
 template <int NT>
 __device__ __forceinline__ void ua_plql(const UaLane<NT> &L, double t, double eps, cd elt, cd &pl,
                                         cd &ql) {
@@ -123,94 +214,183 @@ __device__ __forceinline__ void ua_plql(const UaLane<NT> &L, double t, double ep
         ql = mk(t * t / 2);
         return;
     }
-    pl = (mk(0.0, eps) * (elt - mk(1.0))) / L.l;                         // eps*1im*(elt-1)/l
-    ql = (eps * (eps * (mk(1.0) - elt) - mk(0.0 * t, L.l * t))) / (L.l * L.l);  // eps*(eps*(1-elt)-1im*l*t)/l^2
+    pl = L.dl.of(mk(0.0, eps) * (elt - mk(1.0)));                          // eps*1im*(elt-1)/l
+    ql = L.dl2.of(eps * (eps * (mk(1.0) - elt) - mk(0.0 * t, L.l * t)));  // eps*(eps*(1-elt)-1im*l*t)/l^2
 }
 
-// preparation! for one particle (ua_steps.jl:3-83): b, t, xt (real) and yt
-// at this lane's tau.
+// preparation! for one particle (ua_steps.jl:3-83): b, t, xt (real) at this
+// lane's tau, and the spectrum Z of r~ = r[0] + 1im r[1] (both real).
+struct UaPrep {
+    double b, t, interv, vxb, vyb, xt[2];
+    Div db;
+    cd Z;
+};
 template <int NT>
-__device__ __forceinline__ void ua_prep(const UaLane<NT> &L, int base, double x1, double x2,
-                                        double vx, double vy, double ex, double ey, double dt,
-                                        double eps, double &b, double &t, double xt[2], cd yt[2],
-                                        double &interv_out) {
-    b = 1 + 0.5 * sin(x1) * sin(x2);
-    t = dt * b;
-    const double vxb = vx / b, vyb = vy / b;
+__device__ __forceinline__ void ua_prep(const UaLane<NT> &L, double x1, double x2, double vx,
+                                        double vy, double ex, double ey, double dt, double eps,
+                                        Div deps, UaPrep &p) {
+    // sin(x1) on the even lanes, sin(x2) on the odd ones, exchanged
+    const double sq = sin((L.m & 1) ? x2 : x1), so = xor_lane<1>(sq);
+    p.b = 1 + 0.5 * ((L.m & 1) ? so : sq) * ((L.m & 1) ? sq : so);
+    p.t = dt * p.b;
+    p.db = Div(p.b);
+    p.vxb = p.db.of(vx);
+    p.vyb = p.db.of(vy);
     const double c = L.c, s = L.s;
-    const double h1 = eps * (s * vxb - c * vyb);
-    const double h2 = eps * (s * vyb + c * vxb);
-    xt[0] = x1 + h1 + eps * vyb;
-    xt[1] = x2 + h2 - eps * vxb;
-    const double interv = (1 + 0.5 * sin(xt[0]) * sin(xt[1]) - b) / eps;
-    interv_out = interv;
-    const double exb = ((c * vy - s * vx) * interv + ex) / b;
-    const double eyb = ((-c * vx - s * vy) * interv + ey) / b;
-    cd r[2] = {mk(c * exb - s * eyb), mk(s * exb + c * eyb)};
+    const double h1 = eps * (s * p.vxb - c * p.vyb);
+    const double h2 = eps * (s * p.vyb + c * p.vxb);
+    p.xt[0] = x1 + h1 + eps * p.vyb;
+    p.xt[1] = x2 + h2 - eps * p.vxb;
+    p.interv = deps.of(1 + 0.5 * sin(p.xt[0]) * sin(p.xt[1]) - p.b);
+    const double exb = p.db.of((c * vy - s * vx) * p.interv + ex);
+    const double eyb = p.db.of((-c * vx - s * vy) * p.interv + ey);
+    p.Z = fft_fwd<NT>(mk(c * exb - s * eyb, s * exb + c * eyb), L);
+}
+
+// -1im R / l, the spectrum of the tau-antiderivative of preparation!
+// (ua_steps.jl:60-74); frequency 0 stays.
+template <int NT>
+__device__ __forceinline__ cd ua_integrate(const UaLane<NT> &L, cd R) {
+    if (L.m == 0) return R;
+    return L.dl.of(mk(R.im, -R.re));
+}
+
+// yt of preparation! (ua_steps.jl:76-82) at this lane's tau.  The integral is
+// linear, so both components go through one inverse transform as the real and
+// imaginary part of r~'s; but for the middle frequency -NT/2, whose -1im/l
+// makes the term of a real sequence imaginary: it is left out there and added
+// to each component by itself.
+template <int NT>
+__device__ __forceinline__ void ua_yt(const UaLane<NT> &L, const UaPrep &p, double vx, double vy,
+                                      double eps, cd yt[2]) {
+    // lane 1 holds frequency -NT/2: Z there is R0 + 1im R1, both real
+    const cd mid = shfl(p.Z, L.base + 1);
+    const cd w = fft_inv<NT>(L.m == 1 ? mk(0.0) : ua_integrate<NT>(L, p.Z), L);
+    const cd w0 = shfl(w, L.base);
+    // -1im R / (-NT/2) (-1)^m / NT, less its value at m = 0
+    const double n = (L.m & 1) ? -4.0 / ((double)NT * NT) : 0.0;
+    yt[0] = mk(vx + eps * (w.re - w0.re), eps * (n * mid.re));
+    yt[1] = mk(vy + eps * (w.im - w0.im), eps * (n * mid.im));
+}
+
+// The spectra of xt and yt at this lane's frequency, without transforms: xt is
+// a constant and the first harmonic, and fft(r) is the spectrum r came from.
+template <int NT>
+__device__ __forceinline__ void ua_xs(const UaLane<NT> &L, const UaPrep &p, double x1, double x2,
+                                      double eps, cd xs[2]) {
+    xs[0] = xs[1] = mk(0.0);
+    if (L.m == 0) {
+        xs[0] = mk(NT * (x1 + eps * p.vyb));
+        xs[1] = mk(NT * (x2 - eps * p.vxb));
+    } else if (NT == 2) {  // tau = 0, pi: cos = 1, -1, sin = 0
+        xs[0] = mk(-2.0 * (eps * p.vyb));
+        xs[1] = mk(2.0 * (eps * p.vxb));
+    } else if (L.l == 1.0 || L.l == -1.0) {
+        const double q = -0.5 * NT * L.l;  // sin: -1im NT/2 at l = 1
+        xs[0] = mk(-0.5 * NT * (eps * p.vyb), q * (eps * p.vxb));
+        xs[1] = mk(0.5 * NT * (eps * p.vxb), q * (eps * p.vyb));
+    }
+}
+template <int NT>
+__device__ __forceinline__ void ua_ys(const UaLane<NT> &L, const UaPrep &p, double vx, double vy,
+                                      double eps, cd ys[2]) {
+    const cd zm = shfl(p.Z, L.mirror);
+    const cd r[2] = {ua_integrate<NT>(L, mk(0.5 * (p.Z.re + zm.re), 0.5 * (p.Z.im - zm.im))),
+                     ua_integrate<NT>(L, mk(0.5 * (p.Z.im + zm.im), -0.5 * (p.Z.re - zm.re)))};
+    const double v[2] = {vx, vy};
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-        cd R = fft_lanes<NT, false>(r[q], L.m, base, L.w);
-        if (L.m != 0) R = mk(R.im / L.l, -R.re / L.l);  // -1im * R / l
-        r[q] = fft_lanes<NT, true>(R, L.m, base, L.w);
+        const cd r0 = lane_sum<NT>(r[q]);  // NT r at tau = 0
+        ys[q] = eps * r[q];
+        if (L.m == 0) ys[q] = ys[q] + mk(NT * v[q]) - eps * r0;
     }
-    const cd r10 = shfl(r[0], base), r20 = shfl(r[1], base);
-    yt[0] = vx + eps * (r[0] - r10);
-    yt[1] = vy + eps * (r[1] - r20);
 }
 
 // (1 + sin(x1) sin(x2)/2 - b)/eps at the lane's position (ua_steps.jl:55, :130).
-__device__ __forceinline__ double ua_interv(const double xt[2], double b, double eps) {
-    return (1 + 0.5 * sin(xt[0]) * sin(xt[1]) - b) / eps;
+__device__ __forceinline__ double ua_interv(const double xt[2], double b, Div deps) {
+    return deps.of(1 + 0.5 * sin(xt[0]) * sin(xt[1]) - b);
 }
 
 // compute_f! at this lane's tau (ua_steps.jl:117-145), before its FFTs;
 // interv from ua_interv at xt.
 template <int NT>
-__device__ __forceinline__ void ua_f(const UaLane<NT> &L, double b, double interv,
-                                     const cd yt[2], const double et[2], cd fx[2], cd fy[2]) {
+__device__ __forceinline__ void ua_f(const UaLane<NT> &L, Div db, double interv, const cd yt[2],
+                                     const double et[2], cd fx[2], cd fy[2]) {
     const double c = L.c, s = L.s;
-    fx[0] = (c * yt[0] + s * yt[1]) / b;
-    fx[1] = (-s * yt[0] + c * yt[1]) / b;
+    fx[0] = db.of(c * yt[0] + s * yt[1]);
+    fx[1] = db.of(-s * yt[0] + c * yt[1]);
     const cd tmp1 = et[0] + interv * (c * yt[1] - s * yt[0]);
     const cd tmp2 = et[1] + interv * (-c * yt[0] - s * yt[1]);
-    fy[0] = (c * tmp1 - s * tmp2) / b;
-    fy[1] = (s * tmp1 + c * tmp2) / b;
-}
-
-// The gather of update_particles_e! at real(xt) (interpolation_m6.jl:22-120).
-__device__ __forceinline__ void ua_gather(const double xt[2], int nx, int ny, double xmin,
-                                          double ymin, double dimx, double dimy, double dx,
-                                          double dy, const double *ex, const double *ey,
-                                          double et[2]) {
-    const double xn = picd::jl_mod_pos(xt[0] - xmin, dimx);
-    const double yn = picd::jl_mod_pos(xt[1] - ymin, dimy);
-    const double px = xn / dx, py = yn / dy;
-    const int i = (int)px, j = (int)py;
-    picd::mf_gather_m6(i, j, px - (double)i, py - (double)j, nx, ny, ex, ey, et[0], et[1]);
+    fy[0] = db.of(c * tmp1 - s * tmp2);
+    fy[1] = db.of(s * tmp1 + c * tmp2);
 }
 
 struct UaGrid {
     int nx, ny;
     double xmin, ymin, dimx, dimy, dx, dy;
-    const double *ex, *ey;  // node fields, nx x ny
-    double *rho_acc;        // raw charge, nx x ny
+    Div ddx, ddy;
+    const double2 *e;       // node fields (ex, ey), nx x ny
+    double *rho_acc;        // raw charge, nx x ny, or null: no deposit here
     double w;               // particle weight
 };
 
+// The gather of update_particles_e! at real(xt) (interpolation_m6.jl:22-120):
+// nodes i-2..i+3 and j-2..j+3, wrapped, (ex, ey) of a node in one 16-byte load
+// at a 32-bit offset.  Sums with FMAs, y inner.
+__device__ __forceinline__ void ua_gather(const double xt[2], const UaGrid &g, double et[2]) {
+    const double px = g.ddx.of(picd::jl_mod_pos(xt[0] - g.xmin, g.dimx));
+    const double py = g.ddy.of(picd::jl_mod_pos(xt[1] - g.ymin, g.dimy));
+    // (clamped: NaN and what rounding leaves on the far edge stay in the mesh)
+    const int i = min(max((int)px, 0), g.nx), j = min(max((int)py, 0), g.ny);
+    double wx[6], wy[6];
+    picd::m6_weights_d(px - (double)i, wx);
+    picd::m6_weights_d(py - (double)j, wy);
+    unsigned row[6];
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+        int q = j - 2 + b;
+        q = q < 0 ? q + g.ny : q;
+        q = q >= g.ny ? q - g.ny : q;
+        row[b] = (unsigned)(q * g.nx);
+    }
+    et[0] = 0.0;
+    et[1] = 0.0;
+#pragma unroll
+    for (int a = 0; a < 6; ++a) {
+        int q = i - 2 + a;
+        q = q < 0 ? q + g.nx : q;
+        q = q >= g.nx ? q - g.nx : q;
+        double t1 = 0.0, t2 = 0.0;
+#pragma unroll
+        for (int b = 0; b < 6; ++b) {
+            const double2 e = g.e[row[b] + (unsigned)q];
+            t1 = __builtin_fma(wy[b], e.x, t1);
+            t2 = __builtin_fma(wy[b], e.y, t2);
+        }
+        et[0] = __builtin_fma(wx[a], t1, et[0]);
+        et[1] = __builtin_fma(wx[a], t2, et[1]);
+    }
+    // the sums are taken here: left to itself the compiler moves them past the
+    // branches of the cosines that follow and spills the 36 loaded nodes
+    pin(et[0]);
+    pin(et[1]);
+}
+
 // update_particles_x! for one particle (compute_rho_m6.jl:37-164): x(t) from
-// its tau-samples, into the domain, stored; the M6 deposit (nodes i-2..i+3,
-// wrapped, as in :70-81) spread over the group's lanes.
-// eplus = exp(+1im l t / eps), the conjugate of elt (cos is even and sin odd
-// in the device library, and the two angles differ only in sign).
+// the spectrum of its tau-samples, into the domain, stored; the M6 deposit
+// (nodes i-2..i+3, wrapped, as in :70-81) spread over the group's lanes where
+// the grid is too large for pic_deposit.hip's.  eplus = exp(+1im l t / eps), the
+// conjugate of elt (cos is even and sin odd in the device library, and the two
+// angles differ only in sign).
 template <int NT>
-__device__ __forceinline__ void ua_reconstruct_deposit(const UaLane<NT> &L, int base, cd eplus,
-                                                       const cd xt[2], const UaGrid &g, bool live,
+__device__ __forceinline__ void ua_reconstruct_deposit(const UaLane<NT> &L, cd eplus,
+                                                       const cd xs[2], const UaGrid &g, bool live,
                                                        double *xo, double *yo) {
     double pos[2];
-    const cd e = eplus / (double)NT;
 #pragma unroll
     for (int q = 0; q < 2; ++q)
-        pos[q] = lane_sum<NT>(fft_lanes<NT, false>(xt[q], L.m, base, L.w) * e).re;
+        pos[q] = lane_sum<NT>(__builtin_fma(xs[q].re, eplus.re, -(xs[q].im * eplus.im))) *
+                 (1.0 / NT);
     const double xt1 = picd::jl_mod_pos(pos[0] - g.xmin, g.dimx);
     const double xt2 = picd::jl_mod_pos(pos[1] - g.ymin, g.dimy);
     if (!live) return;
@@ -218,8 +398,9 @@ __device__ __forceinline__ void ua_reconstruct_deposit(const UaLane<NT> &L, int 
         *xo = xt1 + g.xmin;
         *yo = xt2 + g.ymin;
     }
+    if (!g.rho_acc) return;  // the deposit follows in launches of its own
     const double px = xt1 / g.dx, py = xt2 / g.dy;
-    const int i = (int)px, j = (int)py;
+    const int i = min(max((int)px, 0), g.nx), j = min(max((int)py, 0), g.ny);
     double wx[6], wy[6];
     picd::m6_weights_d(px - (double)i, wx);
     picd::m6_weights_d(py - (double)j, wy);
@@ -230,16 +411,24 @@ __device__ __forceinline__ void ua_reconstruct_deposit(const UaLane<NT> &L, int 
     }
 }
 
-// compute_v! for one particle (ua_steps.jl:206-224) from the tau-spectrum yt.
+// compute_v! for one particle (ua_steps.jl:206-224) from the tau-spectrum yt;
+// cos and sin of t/eps are elt's at l = 1.
 template <int NT>
-__device__ __forceinline__ void ua_v(const UaLane<NT> &L, double t, double eps, cd eplus,
+__device__ __forceinline__ void ua_v(const UaLane<NT> &L, double t, Div deps, cd eplus,
                                      const cd yt[2], double &v1, double &v2) {
-    const cd e = eplus;
-    const cd px = lane_sum<NT>((yt[0] / (double)NT) * e);
-    const cd py = lane_sum<NT>((yt[1] / (double)NT) * e);
-    const double ct = cos(t / eps), st = sin(t / eps);
-    v1 = ct * px.re + st * py.re;
-    v2 = ct * py.re - st * px.re;
+    double p[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        p[q] = lane_sum<NT>(__builtin_fma(yt[q].re, eplus.re, -(yt[q].im * eplus.im))) * (1.0 / NT);
+    cd e1;
+    if (NT == 2) {  // frequencies 0 and -1 only
+        const double th = deps.of(t);
+        sincos(th, &e1.im, &e1.re);
+    } else {
+        e1 = shfl(eplus, L.base + NT / 2);
+    }
+    v1 = e1.re * p[0] + e1.im * p[1];
+    v2 = e1.re * p[1] - e1.im * p[0];
 }
 
 // Lane, group and particle of this thread.
@@ -263,7 +452,8 @@ __device__ __forceinline__ size_t ux(int m, int c, int64_t k, int nt) {
     return (size_t)m + (size_t)nt * ((size_t)c + 2 * (size_t)k);
 }
 
-// (m, q, k) of the (ntau, 4, n) spectra of fx (q = 0, 1) and fy (q = 2, 3).
+// (m, q, k) of the (ntau, 4, n) spectra of fx (q = 0, 1) and fy (q = 2, 3), in
+// the lanes' bit-reversed order.
 __device__ __forceinline__ size_t uf(int m, int q, int64_t k, int nt) {
     return (size_t)m + (size_t)nt * ((size_t)q + 4 * (size_t)k);
 }
@@ -271,6 +461,8 @@ __device__ __forceinline__ size_t uf(int m, int q, int64_t k, int nt) {
 struct UaArgs {
     int64_t n;
     double eps, dt;
+    Div deps;
+    const UaTable *tab;
     double *x, *y, *vx, *vy;  // Particles.x, .v (SoA)
     const double *epx, *epy;  // Particles.e
     double *b, *t;            // Particles.b, .t
@@ -282,40 +474,40 @@ struct UaArgs {
 // ---------------------------------------------------------------- the loop
 
 // Prediction of test/bupdate.jl:64-84: preparation!, update_particles_e!,
-// compute_f!, x~t = fft(xt), ua_step!, the same for yt, ifft!, then
-// update_particles_x!.  Keeps x at the step's start and the spectra of fx, fy.
+// compute_f!, x~t = fft(xt), ua_step!, then update_particles_x!, which takes the
+// spectrum that the reference's ifft! and fft! would give back.  (The
+// predicted yt is formed by the correction.)  Keeps x at the step's start and
+// the spectra of fx, fy.
 template <int NT>
-__global__ __launch_bounds__(UB) void k_ua_predict(UaArgs a) {
+__global__ __launch_bounds__(UB, UA_WAVES) void k_ua_predict(UaArgs a) {
     const Slot<NT> S(a.n);
-    const UaLane<NT> L(S.m);
+    const UaLane<NT> L(a.tab, S.m, S.base);
+    const bool live = S.live;
     const int64_t k = S.k;
-    const double x1 = a.x[k], x2 = a.y[k];
-    double b, t, xt[2], et[2], interv;
-    cd yt[2], fx[2], fy[2];
-    ua_prep<NT>(L, S.base, x1, x2, a.vx[k], a.vy[k], a.epx[k], a.epy[k], a.dt, a.eps, b, t, xt,
-                yt, interv);
-    ua_gather(xt, a.g.nx, a.g.ny, a.g.xmin, a.g.ymin, a.g.dimx, a.g.dimy, a.g.dx, a.g.dy, a.g.ex,
-              a.g.ey, et);
-    ua_f<NT>(L, b, interv, yt, et, fx, fy);
-    const cd elt = ua_cis(-1, L.l, t, a.eps);
+    const double x1 = a.x[k], x2 = a.y[k], vx = a.vx[k], vy = a.vy[k];
+    UaPrep p;
+    ua_prep<NT>(L, x1, x2, vx, vy, a.epx[k], a.epy[k], a.dt, a.eps, a.deps, p);
+    cd yt[2], fx[2], fy[2], xs[2];
+    ua_yt<NT>(L, p, vx, vy, a.eps, yt);
+    double et[2];
+    ua_gather(p.xt, a.g, et);
+    ua_f<NT>(L, p.db, p.interv, yt, et, fx, fy);
+    const cd elt = ua_cis(L.l, p.t, a.deps);
     cd pl, ql;
-    ua_plql<NT>(L, t, a.eps, elt, pl, ql);
-    cd xn[2], yn[2];
+    ua_plql<NT>(L, p.t, a.eps, elt, pl, ql);
+    ua_xs<NT>(L, p, x1, x2, a.eps, xs);
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-        fx[q] = fft_lanes<NT, false>(fx[q], L.m, S.base, L.w);
-        fy[q] = fft_lanes<NT, false>(fy[q], L.m, S.base, L.w);
-        const cd xs = fft_lanes<NT, false>(mk(xt[q]), L.m, S.base, L.w);
-        const cd ys = fft_lanes<NT, false>(yt[q], L.m, S.base, L.w);
-        xn[q] = fft_lanes<NT, true>(elt * xs + pl * fx[q], L.m, S.base, L.w);
-        yn[q] = fft_lanes<NT, true>(elt * ys + pl * fy[q], L.m, S.base, L.w);
+        fx[q] = fft_fwd<NT>(fx[q], L);
+        fy[q] = fft_fwd<NT>(fy[q], L);
+        xs[q] = elt * xs[q] + pl * fx[q];
     }
-    if (S.live) {
+    if (live) {
         if (S.m == 0) {
             a.x0[k] = x1;
             a.y0[k] = x2;
-            a.b[k] = b;
-            a.t[k] = t;
+            a.b[k] = p.b;
+            a.t[k] = p.t;
         }
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
@@ -323,84 +515,92 @@ __global__ __launch_bounds__(UB) void k_ua_predict(UaArgs a) {
             a.fhat[uf(S.m, 2 + q, k, NT)] = fy[q];
         }
     }
-    ua_reconstruct_deposit<NT>(L, S.base, mk(elt.re, -elt.im), xn, a.g, S.live, &a.x[k],
-                               &a.y[k]);
+    ua_reconstruct_deposit<NT>(L, mk(elt.re, -elt.im), xs, a.g, live, &a.x[k], &a.y[k]);
 }
 
 // Correction of test/bupdate.jl:90-114: the predicted xt, yt rebuilt from the
 // step's start, update_particles_e! on the new field, compute_f!, the
-// corrected ua_step!s, ifft!(xt), update_particles_x! and compute_v!.
+// corrected ua_step!s, update_particles_x! and compute_v!.
 template <int NT>
-__global__ __launch_bounds__(UB) void k_ua_correct(UaArgs a) {
+__global__ __launch_bounds__(UB, UA_WAVES) void k_ua_correct(UaArgs a) {
     const Slot<NT> S(a.n);
-    const UaLane<NT> L(S.m);
+    const UaLane<NT> L(a.tab, S.m, S.base);
+    const bool live = S.live;
     const int64_t k = S.k;
-    double b, t, xt[2], et[2], interv;
-    cd yt[2];
-    ua_prep<NT>(L, S.base, a.x0[k], a.y0[k], a.vx[k], a.vy[k], a.epx[k], a.epy[k], a.dt, a.eps,
-                b, t, xt, yt, interv);
-    const cd elt = ua_cis(-1, L.l, t, a.eps);
-    cd pl, ql;
-    ua_plql<NT>(L, t, a.eps, elt, pl, ql);
-    cd fx[2], fy[2], xs[2], ys[2], xp[2], yp[2];
+    const double x1 = a.x0[k], x2 = a.y0[k], vx = a.vx[k], vy = a.vy[k];
+    cd fx[2], fy[2];
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
         fx[q] = a.fhat[uf(S.m, q, k, NT)];
         fy[q] = a.fhat[uf(S.m, 2 + q, k, NT)];
-        xs[q] = fft_lanes<NT, false>(mk(xt[q]), L.m, S.base, L.w);
-        ys[q] = fft_lanes<NT, false>(yt[q], L.m, S.base, L.w);
-        xp[q] = fft_lanes<NT, true>(elt * xs[q] + pl * fx[q], L.m, S.base, L.w);
-        yp[q] = fft_lanes<NT, true>(elt * ys[q] + pl * fy[q], L.m, S.base, L.w);
     }
-    const double xr[2] = {xp[0].re, xp[1].re};
-    ua_gather(xr, a.g.nx, a.g.ny, a.g.xmin, a.g.ymin, a.g.dimx, a.g.dimy, a.g.dx, a.g.dy, a.g.ex,
-              a.g.ey, et);
-    cd gx[2], gy[2];
-    ua_f<NT>(L, b, ua_interv(xr, b, a.eps), yp, et, gx, gy);
-    cd xn[2], yn[2];
+    UaPrep p;
+    ua_prep<NT>(L, x1, x2, vx, vy, a.epx[k], a.epy[k], a.dt, a.eps, a.deps, p);
+    const cd elt = ua_cis(L.l, p.t, a.deps);
+    cd pl, ql;
+    ua_plql<NT>(L, p.t, a.eps, elt, pl, ql);
+    cd xs[2], ys[2], yp[2];
+    ua_xs<NT>(L, p, x1, x2, a.eps, xs);
+    ua_ys<NT>(L, p, vx, vy, a.eps, ys);
+    double xr[2];
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-        gx[q] = fft_lanes<NT, false>(gx[q], L.m, S.base, L.w);
-        gy[q] = fft_lanes<NT, false>(gy[q], L.m, S.base, L.w);
-        xn[q] = elt * xs[q] + pl * fx[q];
-        xn[q] = xn[q] + (ql * (gx[q] - fx[q])) / t;
-        xn[q] = fft_lanes<NT, true>(xn[q], L.m, S.base, L.w);
-        yn[q] = elt * ys[q] + pl * fy[q];
-        yn[q] = yn[q] + (ql * (gy[q] - fy[q])) / t;
+        xs[q] = elt * xs[q] + pl * fx[q];
+        ys[q] = elt * ys[q] + pl * fy[q];
+        xr[q] = fft_inv<NT>(xs[q], L).re;
+        yp[q] = fft_inv<NT>(ys[q], L);
+    }
+    double et[2];
+    ua_gather(xr, a.g, et);
+    cd gx[2], gy[2];
+    ua_f<NT>(L, p.db, ua_interv(xr, p.b, a.deps), yp, et, gx, gy);
+    const Div dt(p.t);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        xs[q] = xs[q] + dt.of(ql * (fft_fwd<NT>(gx[q], L) - fx[q]));
+        ys[q] = ys[q] + dt.of(ql * (fft_fwd<NT>(gy[q], L) - fy[q]));
     }
     const cd eplus = mk(elt.re, -elt.im);
-    ua_reconstruct_deposit<NT>(L, S.base, eplus, xn, a.g, S.live, &a.x[k], &a.y[k]);
+    ua_reconstruct_deposit<NT>(L, eplus, xs, a.g, live, &a.x[k], &a.y[k]);
     double v1, v2;
-    ua_v<NT>(L, t, a.eps, eplus, yn, v1, v2);
-    if (S.live && S.m == 0) {
+    ua_v<NT>(L, p.t, a.deps, eplus, ys, v1, v2);
+    if (live && S.m == 0) {
         a.vx[k] = v1;
         a.vy[k] = v2;
     }
 }
 
 // ------------------------------------------------------- per-call pieces
+//
+// Spectra enter and leave in the reference's order: lane m's element is that of
+// frequency mr.
+#define UA_CALL_PROLOGUE                  \
+    const Slot<NT> S(a.n);                \
+    const UaLane<NT> L(a.tab, S.m, S.base); \
+    const bool live = S.live;             \
+    const int64_t k = S.k;                \
+    const int mr = bitrev<NT>(S.m);       \
+    (void)mr
 
 // preparation!: b, t, pl, ql, xt, yt (any output may be null).
 template <int NT>
 __global__ __launch_bounds__(UB) void k_ua_prep_call(UaArgs a, cd *pl, cd *ql, cd *xt, cd *yt) {
-    const Slot<NT> S(a.n);
-    const UaLane<NT> L(S.m);
-    const int64_t k = S.k;
-    double b, t, x[2], interv;
-    cd y[2];
-    ua_prep<NT>(L, S.base, a.x[k], a.y[k], a.vx[k], a.vy[k], a.epx[k], a.epy[k], a.dt, a.eps, b,
-                t, x, y, interv);
-    cd p, q;
-    ua_plql<NT>(L, t, a.eps, ua_cis(-1, L.l, t, a.eps), p, q);
-    if (!S.live) return;
+    UA_CALL_PROLOGUE;
+    const double vx = a.vx[k], vy = a.vy[k];
+    UaPrep pr;
+    ua_prep<NT>(L, a.x[k], a.y[k], vx, vy, a.epx[k], a.epy[k], a.dt, a.eps, a.deps, pr);
+    cd y[2], p, q;
+    ua_yt<NT>(L, pr, vx, vy, a.eps, y);
+    ua_plql<NT>(L, pr.t, a.eps, ua_cis(L.l, pr.t, a.deps), p, q);
+    if (!live) return;
     if (S.m == 0) {
-        a.b[k] = b;
-        a.t[k] = t;
+        a.b[k] = pr.b;
+        a.t[k] = pr.t;
     }
-    if (pl) pl[S.m + (size_t)NT * k] = p;
-    if (ql) ql[S.m + (size_t)NT * k] = q;
+    if (pl) pl[mr + (size_t)NT * k] = p;
+    if (ql) ql[mr + (size_t)NT * k] = q;
     for (int c = 0; c < 2; ++c) {
-        if (xt) xt[ux(S.m, c, k, NT)] = mk(x[c]);
+        if (xt) xt[ux(S.m, c, k, NT)] = mk(pr.xt[c]);
         if (yt) yt[ux(S.m, c, k, NT)] = y[c];
     }
 }
@@ -409,12 +609,12 @@ __global__ __launch_bounds__(UB) void k_ua_prep_call(UaArgs a, cd *pl, cd *ql, c
 template <int NT>
 __global__ __launch_bounds__(UB) void k_ua_gather_call(UaArgs a, const cd *xt, double *et) {
     const Slot<NT> S(a.n);
+    const bool live = S.live;
     const int64_t k = S.k;
     const double x[2] = {xt[ux(S.m, 0, k, NT)].re, xt[ux(S.m, 1, k, NT)].re};
     double e[2];
-    ua_gather(x, a.g.nx, a.g.ny, a.g.xmin, a.g.ymin, a.g.dimx, a.g.dimy, a.g.dx, a.g.dy, a.g.ex,
-              a.g.ey, e);
-    if (!S.live) return;
+    ua_gather(x, a.g, e);
+    if (!live) return;
     et[ux(S.m, 0, k, NT)] = e[0];
     et[ux(S.m, 1, k, NT)] = e[1];
 }
@@ -423,23 +623,21 @@ __global__ __launch_bounds__(UB) void k_ua_gather_call(UaArgs a, const cd *xt, d
 template <int NT>
 __global__ __launch_bounds__(UB) void k_ua_f_call(UaArgs a, const cd *xt, const cd *yt,
                                                   const double *et, cd *fx, cd *fy) {
-    const Slot<NT> S(a.n);
-    const UaLane<NT> L(S.m);
-    const int64_t k = S.k;
+    UA_CALL_PROLOGUE;
     const double x[2] = {xt[ux(S.m, 0, k, NT)].re, xt[ux(S.m, 1, k, NT)].re};
     const cd y[2] = {yt[ux(S.m, 0, k, NT)], yt[ux(S.m, 1, k, NT)]};
     const double e[2] = {et[ux(S.m, 0, k, NT)], et[ux(S.m, 1, k, NT)]};
     const double b = a.b[k];
     cd f[2], h[2];
-    ua_f<NT>(L, b, ua_interv(x, b, a.eps), y, e, f, h);
+    ua_f<NT>(L, Div(b), ua_interv(x, b, a.deps), y, e, f, h);
     for (int c = 0; c < 2; ++c) {
-        f[c] = fft_lanes<NT, false>(f[c], L.m, S.base, L.w);
-        h[c] = fft_lanes<NT, false>(h[c], L.m, S.base, L.w);
+        f[c] = fft_fwd<NT>(f[c], L);
+        h[c] = fft_fwd<NT>(h[c], L);
     }
-    if (!S.live) return;
+    if (!live) return;
     for (int c = 0; c < 2; ++c) {
-        fx[ux(S.m, c, k, NT)] = f[c];
-        fy[ux(S.m, c, k, NT)] = h[c];
+        fx[ux(mr, c, k, NT)] = f[c];
+        fy[ux(mr, c, k, NT)] = h[c];
     }
 }
 
@@ -447,16 +645,14 @@ __global__ __launch_bounds__(UB) void k_ua_f_call(UaArgs a, const cd *xt, const 
 template <int NT>
 __global__ __launch_bounds__(UB) void k_ua_step_call(UaArgs a, const cd *xtil, const cd *fx,
                                                      const cd *gx, cd *xt) {
-    const Slot<NT> S(a.n);
-    const UaLane<NT> L(S.m);
-    const int64_t k = S.k;
+    UA_CALL_PROLOGUE;
     const double t = a.t[k];
-    const cd elt = ua_cis(-1, L.l, t, a.eps);
+    const cd elt = ua_cis(L.l, t, a.deps);
     cd pl, ql;
     ua_plql<NT>(L, t, a.eps, elt, pl, ql);
-    if (!S.live) return;
+    if (!live) return;
     for (int c = 0; c < 2; ++c) {
-        const size_t u = ux(S.m, c, k, NT);
+        const size_t u = ux(mr, c, k, NT);
         const cd f = fx[u];
         cd z = elt * xtil[u] + pl * f;
         if (gx) z = z + (ql * (gx[u] - f)) / t;
@@ -467,25 +663,23 @@ __global__ __launch_bounds__(UB) void k_ua_step_call(UaArgs a, const cd *xtil, c
 // update_particles_x!: reconstruction into Particles.x and the deposit.
 template <int NT>
 __global__ __launch_bounds__(UB) void k_ua_rho_call(UaArgs a, const cd *xt) {
-    const Slot<NT> S(a.n);
-    const UaLane<NT> L(S.m);
-    const int64_t k = S.k;
-    const cd x[2] = {xt[ux(S.m, 0, k, NT)], xt[ux(S.m, 1, k, NT)]};
-    ua_reconstruct_deposit<NT>(L, S.base, ua_cis(+1, L.l, a.t[k], a.eps), x, a.g, S.live,
-                               &a.x[k], &a.y[k]);
+    UA_CALL_PROLOGUE;
+    cd x[2] = {xt[ux(S.m, 0, k, NT)], xt[ux(S.m, 1, k, NT)]};
+    for (int c = 0; c < 2; ++c) x[c] = fft_fwd<NT>(x[c], L);
+    const cd elt = ua_cis(L.l, a.t[k], a.deps);
+    ua_reconstruct_deposit<NT>(L, mk(elt.re, -elt.im), x, a.g, live, &a.x[k], &a.y[k]);
 }
 
 // compute_v!.
 template <int NT>
 __global__ __launch_bounds__(UB) void k_ua_v_call(UaArgs a, const cd *yt) {
-    const Slot<NT> S(a.n);
-    const UaLane<NT> L(S.m);
-    const int64_t k = S.k;
-    const cd y[2] = {yt[ux(S.m, 0, k, NT)], yt[ux(S.m, 1, k, NT)]};
+    UA_CALL_PROLOGUE;
+    const cd y[2] = {yt[ux(mr, 0, k, NT)], yt[ux(mr, 1, k, NT)]};
     const double t = a.t[k];
+    const cd elt = ua_cis(L.l, t, a.deps);
     double v1, v2;
-    ua_v<NT>(L, t, a.eps, ua_cis(+1, L.l, t, a.eps), y, v1, v2);
-    if (S.live && S.m == 0) {
+    ua_v<NT>(L, t, a.deps, mk(elt.re, -elt.im), y, v1, v2);
+    if (live && S.m == 0) {
         a.vx[k] = v1;
         a.vy[k] = v2;
     }
@@ -535,6 +729,13 @@ int ua_ensure(Ctx *c) {
         c->ua_cap = (int64_t)n;
     }
     PIC_TRY(ensure_pfields(c));
+    PIC_TRY(ua_alloc(&c->ua_e, (size_t)2 * c->nx * c->ny));
+    if (!c->ua_tab) {  // made for the ntau of pic_ua_init, which drops an older one
+        PIC_HIP(hipMalloc(&c->ua_tab, (size_t)c->ua_ntau * sizeof(UaTable)));
+        hipLaunchKernelGGL(k_ua_tables, dim3(1), dim3(64), 0, c->stream, c->ua_ntau,
+                           static_cast<UaTable *>(c->ua_tab));
+        PIC_HIP(hipGetLastError());
+    }
     return PIC_OK;
 }
 
@@ -542,6 +743,8 @@ UaArgs ua_args(Ctx *c, double dt) {
     UaArgs a;
     a.n = c->n;
     a.eps = c->ua_eps;
+    a.deps = Div(c->ua_eps);
+    a.tab = static_cast<const UaTable *>(c->ua_tab);
     a.dt = dt;
     a.x = c->x; a.y = c->y; a.vx = c->vx; a.vy = c->vy;
     a.epx = c->epx; a.epy = c->epy;
@@ -552,7 +755,8 @@ UaArgs ua_args(Ctx *c, double dt) {
     a.g.xmin = c->xmin; a.g.ymin = c->ymin;
     a.g.dimx = c->dimx; a.g.dimy = c->dimy;
     a.g.dx = c->dx; a.g.dy = c->dy;
-    a.g.ex = c->ex; a.g.ey = c->ey;
+    a.g.ddx = Div(c->dx); a.g.ddy = Div(c->dy);
+    a.g.e = reinterpret_cast<const double2 *>(c->ua_e);
     a.g.rho_acc = c->rho_acc;
     a.g.w = c->w0;
     return a;
@@ -618,7 +822,11 @@ int pic_ua_init(pic_ctx *ctx, int ntau, double eps) {
     PIC_CHECK(eps > 0.0, PIC_ERR_ARG, "eps must be positive");
     Ctx *c = ctx_of(ctx);
     PIC_HIP(hipSetDevice(c->device));
-    if (c->ua_ntau != ntau) ua_free(c);
+    if (c->ua_ntau != ntau) {
+        ua_free(c);
+        if (c->ua_tab) (void)hipFree(c->ua_tab);
+        c->ua_tab = nullptr;
+    }
     c->ua_ntau = ntau;
     c->ua_eps = eps;
     return PIC_OK;
@@ -661,6 +869,7 @@ int pic_ua_interpol(pic_ctx *ctx, const double *xt, double *et) {
     PIC_TRY(to_dev(c, dxt, xt, nc));
     PIC_TRY(alloc_dev(det, (nc + 1) / 2));
     if (n) {
+        PIC_TRY(interleave_fields(c, reinterpret_cast<double2 *>(c->ua_e)));
         const UaArgs a = ua_args(c, 0.0);
         UA_NT_SWITCH(nt, hipLaunchKernelGGL(k_ua_gather_call<NT>, ua_grid(c->n, NT), dim3(UB), 0,
                                             c->stream, a, dxt.p, (double *)det.p));
@@ -732,16 +941,20 @@ int pic_ua_compute_rho(pic_ctx *ctx, const double *t, const double *xt) {
     const size_t n = (size_t)c->n, nc = (size_t)nt * 2 * n;
     DevC dxt;
     PIC_TRY(to_dev(c, dxt, xt, nc));
-    PIC_TRY(launch_fill(c, c->rho_acc, 0.0, (int64_t)c->nx * c->ny));
+    const bool lds = deposit_lds_ok(c);
+    if (!lds) PIC_TRY(launch_fill(c, c->rho_acc, 0.0, (int64_t)c->nx * c->ny));
     if (n) {
-        const UaArgs a = ua_args(c, 0.0);
+        UaArgs a = ua_args(c, 0.0);
+        if (lds) a.g.rho_acc = nullptr;
         UA_NT_SWITCH(nt, hipLaunchKernelGGL(k_ua_rho_call<NT>, ua_grid(c->n, NT), dim3(UB), 0,
                                             c->stream, a, dxt.p));
         PIC_HIP(hipGetLastError());
     }
-    PIC_TRY(finalize_rho(c, PIC_M6));
+    if (lds) PIC_TRY(deposit_rho_mf(c, c->xmin, c->ymin, false));
+    else PIC_TRY(finalize_rho(c, PIC_M6));
     PIC_HIP(hipStreamSynchronize(c->stream));
     c->seg_valid = false;
+    c->near_order = false;
     c->sort_fresh = false;
     return PIC_OK;
 }
@@ -788,17 +1001,24 @@ int pic_ua_run(pic_ctx *ctx, double dt, int nsteps, double *energy) {
     const int64_t nh = 2 * (int64_t)nsteps;
     if (energy) PIC_TRY(ensure_energy(c, nh + (nh + 1) / 2));
     double *ghost = c->energy_hist + 2 * nh;
+    const bool lds = deposit_lds_ok(c);
+    // the gather reads (ex, ey) side by side: the loop's solves write them so
+    double2 *const e2 = reinterpret_cast<double2 *>(c->ua_e);
+    if (c->n && nsteps) PIC_TRY(interleave_fields(c, e2));
     for (int s = 0; s < nsteps; ++s) {
         for (int half = 0; half < 2; ++half) {
-            PIC_TRY(launch_fill(c, c->rho_acc, 0.0, m));
+            if (!lds) PIC_TRY(launch_fill(c, c->rho_acc, 0.0, m));
             if (c->n) {
-                const UaArgs a = ua_args(c, dt);
+                UaArgs a = ua_args(c, dt);
+                if (lds) a.g.rho_acc = nullptr;
                 if (c->timing) PIC_HIP(hipEventRecord(ev[0], c->stream));
                 if (half == 0) {
-                    UA_NT_SWITCH(nt, hipLaunchKernelGGL(k_ua_predict<NT>, ua_grid(c->n, NT),
+                    UA_NT_SWITCH(nt, hipLaunchKernelGGL(k_ua_predict<NT>,
+                                                        ua_grid(c->n, NT),
                                                         dim3(UB), 0, c->stream, a));
                 } else {
-                    UA_NT_SWITCH(nt, hipLaunchKernelGGL(k_ua_correct<NT>, ua_grid(c->n, NT),
+                    UA_NT_SWITCH(nt, hipLaunchKernelGGL(k_ua_correct<NT>,
+                                                        ua_grid(c->n, NT),
                                                         dim3(UB), 0, c->stream, a));
                 }
                 PIC_HIP(hipGetLastError());
@@ -812,10 +1032,11 @@ int pic_ua_run(pic_ctx *ctx, double dt, int nsteps, double *energy) {
                     c->t_ua_n[half] += 1;
                 }
             }
-            PIC_TRY(finalize_rho(c, PIC_M6));
-            // pic_solve_fields without its wait: E, then the energy sums
-            PIC_TRY(poisson_solve_e(c, c->rho, 1.0 / ((double)c->nx * (double)c->ny), 1, -1));
-            if (energy) PIC_TRY(field_energy_async(c, 2 * s + half, ghost + 2 * s + half));
+            if (lds) PIC_TRY(deposit_rho_mf(c, c->xmin, c->ymin, false));
+            else PIC_TRY(finalize_rho(c, PIC_M6));
+            // pic_solve_fields without its wait: E and the energy sums
+            PIC_TRY(solve_fields_async(c, energy ? 2 * s + half : -1,
+                                       energy ? ghost + 2 * s + half : nullptr, e2));
         }
     }
     if (energy && nh > 0) {
@@ -828,6 +1049,7 @@ int pic_ua_run(pic_ctx *ctx, double dt, int nsteps, double *energy) {
     }
     PIC_HIP(hipStreamSynchronize(c->stream));
     c->seg_valid = false;
+    c->near_order = false;
     c->sort_fresh = false;
     return PIC_OK;
 }

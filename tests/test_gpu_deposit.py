@@ -1,0 +1,96 @@
+"""The charge deposit of particles in any order (the whole grid's charge in LDS,
+in one part or several) against the oracle, at the sizes where its parts and
+chunks change, and the UA loop built on it for every ntau."""
+import math
+
+import numpy as np
+import pytest
+
+from conftest import random_particles
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {"cic": "CloudInCell", "m6": "M6", "ngp": "NearestGridPoint",
+          "tsc": "TriangularShapeCloud", "m4": "M4"}
+DIMX, DIMY = 4 * math.pi, 2 * math.pi
+
+
+def _rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("nx,ny,n,weighted", [
+    (4, 4, 1, False),            # one particle, every stencil wraps
+    (160, 128, 1_023, True),     # the largest grid of one part
+    (144, 144, 1_025, False),    # two parts, two chunks
+    (400, 400, 70_001, True),    # eight parts, the most
+    (512, 512, 30_000, False)])  # more: the chunk kernels
+def test_compute_rho_of_unsorted_particles(gpu, O, shape, nx, ny, n, weighted):
+    """compute_rho on particles in random order, some on the domain's far
+    edge: 1e-12 of the oracle normwise, the bar of the FP64 charge sums
+    (atomics and chunks take the same terms in another order)."""
+    pic = gpu
+    rng = np.random.default_rng(nx + n)
+    mesh = pic.TwoDGrid(DIMX, nx, DIMY, ny)
+    p = random_particles(rng, n, mesh.dimx, mesh.dimy)
+    p[0, ::7] = 0.0
+    p[1, 3::11] = np.nextafter(mesh.dimy, 0.0)
+    if weighted:
+        p[4] *= rng.uniform(0.5, 1.5, n)
+    g = pic.ParticleGroup(n)
+    g.array[...] = p
+    got = pic.compute_rho(g, getattr(pic, SHAPES[shape])(), mesh)
+    want = O.compute_rho(p, shape, nx, ny, mesh.dx, mesh.dy, mesh.dimx, mesh.dimy)
+    assert _rel(got, want) < 1e-12
+    assert np.array_equal(g.array, p)
+
+
+@pytest.mark.parametrize("nx,ny,n", [(128, 64, 5_001), (144, 144, 2_000), (512, 512, 3_000)])
+@pytest.mark.parametrize("compat", [True, False])
+def test_meshfields_deposit_parts(gpu, O, compat, nx, ny, n):
+    """compute_rho_m6!(fields, particles) on grids of one part, two, and past
+    the last: charge within 1e-12 normwise, positions as the oracle rewrites
+    them."""
+    pic = gpu
+    rng = np.random.default_rng(n)
+    mesh = pic.TwoDGrid(0.0, DIMX, nx, 0.0, DIMY, ny)
+    p = pic.Particles(n, DIMX * DIMY / n)
+    p.x[0], p.x[1] = rng.uniform(-DIMX, 2 * DIMX, n), rng.uniform(-DIMY, 2 * DIMY, n)
+    f = pic.MeshFields2D(mesh)
+    x = np.asfortranarray(p.x.copy())
+    want = O.compute_rho_m6_fields(x, p.w, nx, ny, 0.0, DIMX, 0.0, DIMY, compat=compat)
+    pic.compute_rho_m6_(f, p, compat=compat)
+    assert np.array_equal(p.x, x)
+    assert _rel(f.rho, want) < 1e-12
+
+
+@pytest.mark.parametrize("ntau,nx,ny,n", [(2, 32, 16, 300), (4, 64, 16, 301), (16, 256, 128, 517),
+                                          (32, 64, 32, 130), (64, 128, 64, 67),
+                                          (8, 512, 512, 200)])
+def test_ua_loop_every_ntau(gpu, O, ntau, nx, ny, n):
+    """Three steps of the UA loop against the oracle's, for every ntau (each
+    its own transform), with the deposit in one part and several and past
+    them: 1e-9, the bar of the loop's other test (the tau-transforms,
+    sines and sums round differently)."""
+    pic = gpu
+    rng = np.random.default_rng(ntau)
+    eps, dt, steps = 0.1, math.pi / 16, 3
+    mesh = pic.TwoDGrid(0.0, DIMX, nx, 0.0, DIMY, ny)
+    p = pic.Particles(n, DIMX * DIMY / n)
+    p.x[0], p.x[1] = rng.uniform(0, DIMX, n), rng.uniform(0, DIMY, n)
+    p.v[...] = rng.normal(size=(2, n))
+    xo = np.asfortranarray(p.x.copy())
+    rho = O.compute_rho_m6_fields(xo, p.w, nx, ny, 0.0, DIMX, 0.0, DIMY, compat=True)
+    e_f, _ = O.solve_fields(rho, 0.0, DIMX, 0.0, DIMY)
+    eo = O.interpol_eb_m6(xo, e_f, nx, ny, 0.0, DIMX, 0.0, DIMY)
+    sim = pic.UASimulation(mesh, p, ntau, eps)
+    en = sim.run(dt, steps)
+    x, v = sim.particles()
+    ef = sim.fields_e()
+    sim.close()
+    vo = np.asfortranarray(p.v.copy())
+    oen = O.ua_run(ntau, eps, dt, steps, xo, vo, eo, p.w, e_f, 0.0, DIMX, 0.0, DIMY)
+    assert _rel(en, oen) < 1e-9
+    assert _rel(x, xo) < 1e-9 and _rel(v, vo) < 1e-9
+    assert _rel(ef, e_f) < 1e-9
