@@ -1,7 +1,7 @@
 // pic_fftlanes.h -- radix-2 transforms across the lanes of a wave: partners
 // exchanged by DPP moves, swizzles and lane permutes instead of LDS round
-// trips.  Used by the one-launch small-grid step (pic_small.hip) and by the
-// three-kernel E solve of pic_poisson.hip for 64 <= nx, ny <= 512.
+// trips.  Used by the three-kernel E solve of pic_poisson.hip for 64 <= nx, ny
+// <= 512; the exchanges also by the UA kernels (pic_ua.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>

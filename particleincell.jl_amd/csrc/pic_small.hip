@@ -19,13 +19,24 @@
 // into, the one cleared for the next launch), so no launch writes what
 // another block of the same launch reads.
 //
-// Transforms: a 1-D transform of length N <= 64 runs in N lanes of one wave
-// (radix-2 decimation in frequency, partners exchanged between lanes by DPP
-// moves and swizzles), each lane working on up to four rows or columns at
-// once; no block-wide barrier between the stages, four between the passes
-// over rows and columns.  Same transforms (unnormalised, exp(-+2 pi i jk/N))
-// and the same spectral arithmetic as the three-kernel solve of
-// pic_poisson.hip; results agree to rounding.
+// Transforms (es_line): N/8 lanes of one wave hold a line's N <= 64 points,
+// eight each (N = 4: one lane, four).  Two steps, N = 8 B: eight-point
+// transforms over the points B apart, twiddles, the lanes' exchange through
+// their line in LDS (no block barrier: a line's lanes are in one wave), then
+// B-point transforms.  Four passes: along x of two real rows packed as one
+// complex line, along y of the half spectrum's columns, back along y, back
+// along x, with three block barriers between them and one within the third.
+// Same transforms (unnormalised, exp(-+2 pi i jk/N)) and the spectral
+// values as the three-kernel solve of pic_poisson.hip; results agree to rounding.
+// Measured on MI355X, Landau CIC 64 x 64 with 204,800 particles, FP32 state, 100
+// steps: 18.6 us per step of wall time against 23.1 (FP64 state 20.2 against
+// 25.9) with a point per lane and
+// radix-2 stages exchanged between lanes (and the self-conjugate columns'
+// projection formed from both halves).  In a block's timestamps: loads 3.4 us,
+// the passes 1.6, 2.0, 2.2 (0.8 of it the spectral values), 2.0 and barriers
+// 1.6, particles 1.3, flush 1.9; the loads and the flush are latency of memory
+// past the L2, the passes that of LDS and of dependent FP64 operations at two
+// waves per SIMD.
 //
 // Charge: FP32 state: int32 fixed-point LDS grid (charge32_fixed) with one
 // quantum for every block, flushed as int64 sums, so the raw charge is exact
@@ -38,7 +49,6 @@
 #include <cmath>
 #include <vector>
 
-#include "pic_fftlanes.h"
 #include "pic_internal.h"
 #include "pic_push32.h"
 #include "pic_push64.h"
@@ -47,15 +57,13 @@ namespace pic {
 
 constexpr int ES_T = 1024;                 // threads per block
 constexpr int ES_WAVES = ES_T / 64;
-constexpr int ES_MAX_SIDE = 64;            // nx, ny <= 64: one transform per wave
-// rows (or columns) per wave and pass: nx ny / (64 ES_WAVES) <= 4
-constexpr int ES_MAX_ROUNDS = ES_MAX_SIDE * ES_MAX_SIDE / (64 * ES_WAVES);
-// Particles per block.  Every block adds its whole charge grid to the global
-// one, so fewer, fuller blocks flush fewer atomics (each node receives one
-// per block); measured on MI355X, Landau CIC 64 x 64 with 204,800 particles:
-// 128 blocks (1.6 particles per thread) 25.5 us per launch in the FP32
-// state and 27.9 in the FP64 state, 200 blocks 27.5 and 29.5, 100 blocks
-// 25.4 and 28.5.
+constexpr int ES_MAX_SIDE = 64;
+constexpr int ES_EPAD = 8;
+// Particles per block.  Every block loads the whole charge and adds its own
+// charge grid to the global one, so fewer, fuller blocks do less of both;
+// measured on MI355X, Landau CIC 64 x 64 with 204,800 particles in the FP32
+// state: 128 blocks (1.6 particles per thread) 18.4 us per step, 200 blocks
+// 20.2, 86 blocks 18.5, 50 blocks 18.5.
 constexpr int64_t ES_BLOCK_PARTICLES = 1600;
 
 struct EsStep {
@@ -80,79 +88,139 @@ struct EsStep {
     double *ex, *ey;
     float2 *e32;
     double *hist;
-    const double2 *tw;  // twiddles: nx/2 along x, then ny/2 along y
+    const double2 *tw;  // twiddles: nx along x, then ny along y
     int nbp;            // particle blocks; block nbp (if launched) the field block
 };
 
-// -i m v scale for complex v.
-__device__ __forceinline__ double2 es_mul_mi(double m, double2 v, double scale) {
-    return make_double2(m * v.y * scale, -(m * v.x) * scale);
+__device__ __forceinline__ double2 operator+(double2 a, double2 b) {
+    return make_double2(a.x + b.x, a.y + b.y);
+}
+__device__ __forceinline__ double2 operator-(double2 a, double2 b) {
+    return make_double2(a.x - b.x, a.y - b.y);
+}
+// a - 1i sg d and a + 1i sg d (sg = 1 forward, -1 backward)
+__device__ __forceinline__ double2 es_sub_i(double2 a, double2 d, double sg) {
+    return make_double2(__builtin_fma(sg, d.y, a.x), __builtin_fma(-sg, d.x, a.y));
+}
+__device__ __forceinline__ double2 es_add_i(double2 a, double2 d, double sg) {
+    return make_double2(__builtin_fma(-sg, d.y, a.x), __builtin_fma(sg, d.x, a.y));
 }
 
-// (Fx, Fy) = -i (kx, ky)/k2 R at half-spectrum index (ih, jh), R[0,0] -> 0.
-__device__ __forceinline__ void es_half(const double2 *S, int PX, int nx, int ih, int jh,
-                                        const double *__restrict__ kxk2,
-                                        const double *__restrict__ kyk2, double scale,
-                                        double2 &f, double2 &g) {
-    const int q = ih + (nx / 2 + 1) * jh;
-    if (q == 0) {
-        f = g = make_double2(0.0, 0.0);
-        return;
+// In-register transforms X[k] = sum_j z[j] exp(-2 pi i sg jk / N), natural
+// order in and out, of the points z[o], z[o + S], ..
+template <int N, int S>
+__device__ __forceinline__ void es_dft(double2 *z, double sg) {
+    if constexpr (N == 2) {
+        const double2 a = z[0], b = z[S];
+        z[0] = a + b;
+        z[S] = a - b;
+    } else if constexpr (N == 4) {
+        const double2 t0 = z[0] + z[2 * S], t1 = z[0] - z[2 * S], t2 = z[S] + z[3 * S],
+                      t3 = z[S] - z[3 * S];
+        z[0] = t0 + t2;
+        z[S] = es_sub_i(t1, t3, sg);
+        z[2 * S] = t0 - t2;
+        z[3 * S] = es_add_i(t1, t3, sg);
+    } else {
+        static_assert(N == 8 && S == 1, "eight points side by side");
+        constexpr double h = 0.70710678118654752440;
+        double2 b[4], c[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            b[k] = z[k] + z[k + 4];
+            c[k] = z[k] - z[k + 4];
+        }
+        // c[k] exp(-2 pi i sg k / 8)
+        const double2 c1 = make_double2(h * __builtin_fma(sg, c[1].y, c[1].x),
+                                        h * __builtin_fma(-sg, c[1].x, c[1].y));
+        const double2 c2 = make_double2(sg * c[2].y, -sg * c[2].x);
+        const double2 c3 = make_double2(h * __builtin_fma(sg, c[3].y, -c[3].x),
+                                        -h * __builtin_fma(sg, c[3].x, c[3].y));
+        c[1] = c1;
+        c[2] = c2;
+        c[3] = c3;
+        es_dft<4, 1>(b, sg);
+        es_dft<4, 1>(c, sg);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            z[2 * k] = b[k];
+            z[2 * k + 1] = c[k];
+        }
     }
-    const double2 R = S[jh * PX + ih];
-    f = es_mul_mi(kxk2[q], R, scale);
-    g = es_mul_mi(kyk2[q], R, scale);
 }
 
-// Full-grid value (ik, jk) of the spectrum whose inverse transform is
-// ex + i ey, from the forward transform S of the charge: the half-spectrum
-// values, the self-conjugate columns (ih = 0, nx/2) projected, columns past
-// nx/2 the conjugates of their mirrors.
-__device__ __forceinline__ double2 es_spectral(const double2 *S, int PX, int nx, int ny, int ik,
-                                               int jk, const double *kxk2, const double *kyk2,
-                                               double scale) {
-    const bool mirror = ik > nx / 2;
-    const int ih = mirror ? nx - ik : ik;
-    const int jh = mirror ? (ny - jk) & (ny - 1) : jk;
-    double2 f, g;
-    es_half(S, PX, nx, ih, jh, kxk2, kyk2, scale, f, g);
-    if (ih == 0 || 2 * ih == nx) {
-        double2 fm, gm;
-        es_half(S, PX, nx, ih, (ny - jh) & (ny - 1), kxk2, kyk2, scale, fm, gm);
-        f = make_double2(0.5 * (f.x + fm.x), 0.5 * (f.y - fm.y));
-        g = make_double2(0.5 * (g.x + gm.x), 0.5 * (g.y - gm.y));
+// One line of N = 2^LOG points: this lane, t of the line's N/8, holds the
+// points t + B n (n < 8) in z[n].  swap(t, c) is the LDS word of element t + c of
+// the line, out(t, c, v) takes element t + c of the result (c, without bits in
+// common with t, is a constant once the loops are unrolled, so that the words
+// share their address arithmetic); tw[k] = exp(-2 pi i k / N).
+template <int LOG, class Swap, class Out>
+__device__ __forceinline__ void es_line(double2 (&z)[8], int t, const double2 *tw, double sg,
+                                        Swap &&swap, Out &&out) {
+    constexpr int N = 1 << LOG, A = N >= 8 ? 8 : 4, B = N / A;
+    es_dft<A, 1>(z, sg);
+    if constexpr (B == 1) {
+#pragma unroll
+        for (int k = 0; k < A; ++k) out(0, k, z[k]);
+    } else {
+        *swap(t, 0) = z[0];
+#pragma unroll
+        for (int k = 1; k < A; ++k) {
+            const double2 w = tw[t * k];
+            const double wy = sg * w.y;
+            *swap(t, B * k) = make_double2(__builtin_fma(z[k].x, w.x, -(z[k].y * wy)),
+                                           __builtin_fma(z[k].x, wy, z[k].y * w.x));
+        }
+        // a wave's LDS operations are done in order: its reads see its writes
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        // 8/B transforms of B points: k = t, t + B, ..; point n of the r-th in
+        // z[r + (8/B) n]
+        constexpr int R = A / B;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int n = 0; n < B; ++n) z[r + R * n] = *swap(B * t, n + B * B * r);
+#pragma unroll
+        for (int r = 0; r < R; ++r) es_dft<B, R>(z + r, sg);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int n = 0; n < B; ++n) out(t, B * r + A * n, z[r + R * n]);
     }
-    if (mirror) {
-        f.y = -f.y;
-        g.y = -g.y;
-    }
-    return make_double2(f.x - g.y, f.y + g.x);
 }
 
 template <int K, bool F32, int BZ>
 __global__ __launch_bounds__(ES_T) void k_es_step(EsStep a) {
     constexpr int HL = Shape<K>::HL;
-    constexpr int NR = ES_MAX_ROUNDS;
     extern __shared__ __align__(16) char es_smem[];
     __shared__ double red[2 * ES_WAVES];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nx = a.nx, ny = a.ny, mx = nx - 1, my = ny - 1, m = nx * ny;
-    const int PX = nx + 1;  // odd row pitch: a column's lanes spread over the banks
-    const int nq = (nx / 2 + 1) * ny;
-    // LDS: the grid (complex), twiddles (nx/2 along x, then ny/2 along y),
-    // the spectral tables, the charge grid
+    // LDS: the grid (complex), the twiddles (nx along x, then ny along y), the
+    // spectral tables, the FP32 state's field, the charge grid
     double2 *X = reinterpret_cast<double2 *>(es_smem);
-    double2 *tw = X + ny * PX;
-    double *tkx = reinterpret_cast<double *>(tw + (nx / 2 + ny / 2)), *tky = tkx + nq;
-    char *tiles = reinterpret_cast<char *>(tky + nq);
+    double2 *tw = X + m;
+    const int nq = (nx / 2 + 1) * ny;
+    double2 *tk = tw + nx + ny;  // (kx, ky)/k2 times the solve's scale
+    float2 *ef = reinterpret_cast<float2 *>(tk + nq);
+    const int pe = nx + ES_EPAD;  // its row pitch: eight rows' words on all banks
+    char *tiles = reinterpret_cast<char *>(F32 ? ef + pe * ny : ef);
     int *itile = reinterpret_cast<int *>(tiles);
     double *dtile = reinterpret_cast<double *>(tiles);
     const bool gather = a.mode != 0, deposit = a.mode != 2;
     const SegF64 &s = a.s64;
+    // Node (i, j) sits at word i ^ f(j) of row j: the 16 lanes an LDS access of
+    // 16-byte words serves at once are two rows (or columns) of eight, which
+    // the flipped bit puts on different halves of the banks, in every pass.
+    const int sw = nx >= 16 ? 8 : 0;
+    auto at = [&](int i, int j) { return j * nx + (i ^ (-((j ^ (j >> 3)) & 1) & sw)); };
 
     // every global load of the launch's first phase is issued here, so that
     // their latencies overlap: this thread's first particle (used after the
-    // solve), its rows of the charge, the spectral tables
+    // solve), its points of the charge, the spectral tables
     // blocks [0, nbp) move the particles; block nbp, launched with the solve,
     // writes the field energy (and the last field) instead
     const bool field = (int)blockIdx.x == a.nbp;
@@ -173,37 +241,34 @@ __global__ __launch_bounds__(ES_T) void k_es_step(EsStep a) {
             pw = s.w ? s.w[p] : s.w0;
         }
     }
-    // rows: 64 / nx per wave and round, lane position i along x; columns:
-    // 64 / ny per wave and round, lane position jp along y; NR rounds
-    const int rw = 64 >> a.lognx, i = lane & mx, ib = brev_bits(i, a.lognx);
-    const int j0 = wave * rw + (lane >> a.lognx), jstep = ES_WAVES * rw;
-    const int cw = 64 >> a.logny, jp = lane & my, jb = brev_bits(jp, a.logny);
-    const int c0 = wave * cw + (lane >> a.logny), cstep = ES_WAVES * cw;
-    double2 zr[NR / 2];
+    // lines along x: lane group tx of T = N/8 lanes works row jr; along y: the
+    // groups of a wave interleave, so that its lanes are neighbouring columns
+    const int ltx = max(a.lognx - 3, 0), lty = max(a.logny - 3, 0);
+    const int jr = tid >> ltx, tx = tid & ((1 << ltx) - 1), dxp = 1 << ltx;
+    const int lcw = 6 - lty;  // log2 of the columns of a wave
+    const int col = (wave << lcw) + (lane & ((1 << lcw) - 1)), ty = lane >> lcw, dyp = 1 << lty;
+    const int npx = min(nx, 8), npy = min(ny, 8);  // points per lane
+    double2 z[8];
     if (a.solve) {
-        // real rows j and j + ny/2 packed as one complex sequence
+        // real rows j and j + ny/2 packed as one complex line
 #pragma unroll
-        for (int r = 0; r < NR / 2; ++r) {
-            const int j = j0 + r * jstep;
-            double u = 0.0, v = 0.0;
-            if (j < ny / 2) {
-                const int64_t g = (int64_t)j * nx + i, g2 = g + (int64_t)(ny / 2) * nx;
+        for (int r = 0; r < 8; ++r) {
+            z[r] = make_double2(0.0, 0.0);
+            if (jr < ny / 2 && r < npx) {
+                const int g = jr * nx + tx + dxp * r, g2 = g + (ny / 2) * nx;
                 if (F32) {
                     const long long *q = reinterpret_cast<const long long *>(a.rin);
-                    u = (double)q[g] * a.unit;
-                    v = (double)q[g2] * a.unit;
+                    z[r] = make_double2((double)q[g], (double)q[g2]);
                 } else {
-                    u = reinterpret_cast<const double *>(a.rin)[g];
-                    v = reinterpret_cast<const double *>(a.rin)[g2];
+                    const double *q = reinterpret_cast<const double *>(a.rin);
+                    z[r] = make_double2(q[g], q[g2]);
                 }
             }
-            zr[r] = make_double2(u, v);
         }
         for (int k = tid; k < nq; k += ES_T) {
-            tkx[k] = a.kxk2[k];
-            tky[k] = a.kyk2[k];
+            tk[k] = make_double2(a.kxk2[k] * a.scale, a.kyk2[k] * a.scale);
         }
-        for (int k = tid; k < nx / 2 + ny / 2; k += ES_T) tw[k] = a.tw[k];
+        for (int k = tid; k < nx + ny; k += ES_T) tw[k] = a.tw[k];
     }
     if (deposit && !field)
         for (int t = tid; t < m; t += ES_T) {
@@ -219,75 +284,100 @@ __global__ __launch_bounds__(ES_T) void k_es_step(EsStep a) {
     __syncthreads();
 
     if (a.solve) {
-        const double2 *twx = tw, *twy = tw + nx / 2;
-        // forward along x of the packed rows; split into the transforms of
-        // rows j, j + ny/2: A = (Z[k] + conj Z[-k]) / 2, B = (Z[k] - conj Z[-k]) / 2i
-        fft_lanes<NR / 2>(zr, i, a.lognx, twx, false);
+        if (F32) {
 #pragma unroll
-        for (int r = 0; r < NR / 2; ++r) {
-            const int j = j0 + r * jstep;
-            if (j >= ny / 2) continue;
-            double2 *row = X + j * PX;
-            row[ib] = zr[r];
-            const double2 zk = row[i], zm = row[(nx - i) & mx];
-            row[i] = make_double2(0.5 * (zk.x + zm.x), 0.5 * (zk.y - zm.y));
-            X[(j + ny / 2) * PX + i] = make_double2(0.5 * (zk.y + zm.y), -0.5 * (zk.x - zm.x));
+            for (int r = 0; r < 8; ++r) z[r] = make_double2(z[r].x * a.unit, z[r].y * a.unit);
+        }
+        auto line = [&](int log, int t, const double2 *w, double sg, auto &&word, auto &&out) {
+            switch (log) {
+                case 6: es_line<6>(z, t, w, sg, word, out); break;
+                case 5: es_line<5>(z, t, w, sg, word, out); break;
+                case 4: es_line<4>(z, t, w, sg, word, out); break;
+                case 3: es_line<3>(z, t, w, sg, word, out); break;
+                default: es_line<2>(z, t, w, sg, word, out); break;
+            }
+        };
+        // word t + c: only bit 3 (and along y bit 0) of c meets the flipped bit
+        auto in_row = [&](int t, int c) { return X + (at(t + (c & 8), jr) + (c & ~8)); };
+        auto in_col = [&](int t, int c) { return X + (at(col, t + (c & 9)) + (c & ~9) * nx); };
+        // forward along x of the packed rows
+        if (jr < ny / 2)
+            line(a.lognx, tx, tw, 1.0, in_row,
+                 [&](int t, int c, double2 v) { *in_row(t, c) = v; });
+        __syncthreads();
+        // forward along y of columns 0 .. nx/2, split on the way in into the
+        // transforms of rows j, j + ny/2: (Z[k] + conj Z[-k]) / 2, (Z[k] - conj
+        // Z[-k]) / 2i
+        if (col <= nx / 2) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (2 * r >= npy) break;
+                const int j = ty + dyp * r;
+                const double2 zk = X[at(col, j)], zm = X[at((nx - col) & mx, j)];
+                z[r] = make_double2(0.5 * (zk.x + zm.x), 0.5 * (zk.y - zm.y));
+                const double2 b = make_double2(0.5 * (zk.y + zm.y), -0.5 * (zk.x - zm.x));
+                if (npy == 8) z[r + 4] = b;
+                else z[(r + 2) & 7] = b;
+            }
+            line(a.logny, ty, tw + nx, 1.0, in_col,
+                 [&](int t, int c, double2 v) { *in_col(t, c) = v; });
         }
         __syncthreads();
-        // forward along y of the half spectrum, columns 0 .. nx/2
-        constexpr int NC = NR - 1;  // (nx/2 + 1) ny / (64 ES_WAVES) <= 3
-        double2 zc[NC];
+        // f + 1i g of (f, g) = -1i (kx, ky)/k2 R, columns past nx/2 the
+        // conjugates of their mirrors.  The self-conjugate columns 0 and nx/2
+        // hold the transforms of real columns, R(-j) = conj R(j): the Hermitian
+        // part of f there is 0, and that of g is g but for its own mirrors 0
+        // and ny/2, where it is 0 (R[0,0] -> 0 with them).
+        if (col < nx) {
+            const bool mir = col > nx / 2;
+            const int ih = mir ? nx - col : col;
+            const bool self = ih == 0 || 2 * ih == nx;
+            const double sm = mir ? -1.0 : 1.0;
 #pragma unroll
-        for (int r = 0; r < NC; ++r) {
-            const int col = c0 + r * cstep;
-            zc[r] = make_double2(0.0, 0.0);
-            if (col <= nx / 2) zc[r] = X[jp * PX + col];
-        }
-        fft_lanes<NC>(zc, jp, a.logny, twy, false);
-#pragma unroll
-        for (int r = 0; r < NC; ++r)
-            if (c0 + r * cstep <= nx / 2) X[jb * PX + c0 + r * cstep] = zc[r];
-        __syncthreads();
-        // spectral values, then inverse along y
-        double2 z[NR];
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-            const int col = c0 + r * cstep;
-            z[r] = make_double2(0.0, 0.0);
-            if (col < nx) z[r] = es_spectral(X, PX, nx, ny, col, jp, tkx, tky, a.scale);
-        }
-        __syncthreads();
-        fft_lanes<NR>(z, jp, a.logny, twy, true);
-#pragma unroll
-        for (int r = 0; r < NR; ++r)
-            if (c0 + r * cstep < nx) X[jb * PX + c0 + r * cstep] = z[r];
-        __syncthreads();
-        // inverse along x: (ex, ey) = (Re, Im); energy sums
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-            const int j = j0 + r * jstep;
-            z[r] = make_double2(0.0, 0.0);
-            if (j < ny) z[r] = X[j * PX + i];
-        }
-        fft_lanes<NR>(z, i, a.lognx, twx, true);
-        double sx = 0.0, sy = 0.0;
-        const bool store = a.write_e && field;
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-            const int j = j0 + r * jstep;
-            if (j >= ny) continue;
-            X[j * PX + ib] = z[r];
-            sx += z[r].x * z[r].x;
-            sy += z[r].y * z[r].y;
-            if (store) {
-                const int64_t g = (int64_t)j * nx + ib;
-                a.ex[g] = z[r].x;
-                a.ey[g] = z[r].y;
-                a.e32[g] = make_float2((float)z[r].x, (float)z[r].y);
+            for (int r = 0; r < 8; ++r) {
+                if (r >= npy) break;
+                const int jk = ty + dyp * r, jh = mir ? (ny - jk) & my : jk;
+                const double2 R = X[at(ih, jh)];
+                double2 k = tk[ih + (nx / 2 + 1) * jh];
+                if (self) {
+                    k.x = 0.0;
+                    if ((jh & (ny / 2 - 1)) == 0) k.y = 0.0;
+                }
+                z[r] = make_double2(__builtin_fma(k.x, R.y, sm * (k.y * R.x)),
+                                    __builtin_fma(k.y, R.y, -sm * (k.x * R.x)));
             }
         }
-        const bool energy = field && a.slot >= 0;
-        if (energy) {  // fixed-order sums: wave trees, then the waves in order
+        __syncthreads();  // every column read before any is written
+        if (col < nx)
+            line(a.logny, ty, tw + nx, -1.0, in_col,
+                 [&](int t, int c, double2 v) { *in_col(t, c) = v; });
+        __syncthreads();
+        // back along x: (ex, ey) = (Re, Im)
+        if (jr < ny) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r)
+                if (r < npx) z[r] = X[at(tx + dxp * r, jr)];
+            float2 *er = ef + jr * pe;
+            line(a.lognx, tx, tw, -1.0, in_row, [&](int t, int c, double2 v) {
+                if (F32 && !field) er[t + c] = make_float2((float)v.x, (float)v.y);
+                else *in_row(t, c) = v;
+            });
+        }
+        __syncthreads();
+        if (field) {
+            double sx = 0.0, sy = 0.0;
+            for (int t = tid; t < m; t += ES_T) {
+                const double2 v = X[at(t & mx, t >> a.lognx)];
+                sx += v.x * v.x;
+                sy += v.y * v.y;
+                if (a.write_e) {
+                    a.ex[t] = v.x;
+                    a.ey[t] = v.y;
+                    a.e32[t] = make_float2((float)v.x, (float)v.y);
+                }
+            }
+            if (a.slot < 0) return;
+            // fixed-order sums: wave trees, then the waves in order
             for (int o = 32; o > 0; o >>= 1) {
                 sx += __shfl_xor(sx, o);
                 sy += __shfl_xor(sy, o);
@@ -296,16 +386,17 @@ __global__ __launch_bounds__(ES_T) void k_es_step(EsStep a) {
                 red[wave] = sx;
                 red[ES_WAVES + wave] = sy;
             }
-        }
-        __syncthreads();
-        if (energy && tid == 0) {
-            double tx = 0.0, ty = 0.0;
-            for (int k = 0; k < ES_WAVES; ++k) {
-                tx += red[k];
-                ty += red[ES_WAVES + k];
+            __syncthreads();
+            if (tid == 0) {
+                sx = sy = 0.0;
+                for (int k = 0; k < ES_WAVES; ++k) {
+                    sx += red[k];
+                    sy += red[ES_WAVES + k];
+                }
+                a.hist[2 * a.slot] = sx * a.dxdy;
+                a.hist[2 * a.slot + 1] = sy * a.dxdy;
             }
-            a.hist[2 * a.slot] = tx * a.dxdy;
-            a.hist[2 * a.slot + 1] = ty * a.dxdy;
+            return;
         }
     }
 
@@ -318,8 +409,7 @@ __global__ __launch_bounds__(ES_T) void k_es_step(EsStep a) {
                 interp32<K, BZ>(
                     fx, fy, ci, cj,
                     [&](int u, int v) {
-                        const double2 e = X[((cj - HL + v) & my) * PX + ((ci - HL + u) & mx)];
-                        return make_float2((float)e.x, (float)e.y);
+                        return ef[((cj - HL + v) & my) * pe + ((ci - HL + u) & mx)];
                     },
                     [&](int, int) { return 0.0f; }, e1, e2, b3);
                 kick32<BZ>(a.hdt, a.bz0, e1, e2, b3, ux, uy);
@@ -349,7 +439,7 @@ __global__ __launch_bounds__(ES_T) void k_es_step(EsStep a) {
                 interp64<K, BZ>(
                     fx, fy, ci, cj,
                     [&](int u, int v) {
-                        return X[((cj - HL + v) & my) * PX + ((ci - HL + u) & mx)];
+                        return X[at((ci - HL + u) & mx, (cj - HL + v) & my)];
                     },
                     [&](int, int) { return 0.0; }, e1, e2, b3);
                 kick64<BZ>(s, e1, e2, b3, pvx, pvy);
@@ -404,12 +494,12 @@ __global__ __launch_bounds__(ES_T) void k_es_step(EsStep a) {
     }
 }
 
-// Twiddles exp(-2 pi i k / N) of the transforms along x (k < nx/2), then y.
+// Twiddles exp(-2 pi i k / N) of the transforms along x (k < nx), then y.
 __global__ void k_es_twiddles(int nx, int ny, int lognx, int logny, double2 *tw) {
     const int k = threadIdx.x;
-    if (k >= nx / 2 + ny / 2) return;
-    const bool along_x = k < nx / 2;
-    const int kk = along_x ? k : k - nx / 2;
+    if (k >= nx + ny) return;
+    const bool along_x = k < nx;
+    const int kk = along_x ? k : k - nx;
     double sn, cs;
     sincospi(ldexp((double)(-2 * kk), -(along_x ? lognx : logny)), &sn, &cs);
     tw[k] = make_double2(cs, sn);
@@ -443,8 +533,9 @@ bool es_step_ok(const Ctx *c) {
 
 static size_t es_lds(const Ctx *c) {
     const size_t nx = c->nx, ny = c->ny;
-    return (ny * (nx + 1) + nx / 2 + ny / 2) * sizeof(double2) +
-           2 * (nx / 2 + 1) * ny * sizeof(double) + nx * ny * (c->state == PIC_STATE_F32 ? 4 : 8);
+    return (nx * ny + nx + ny) * sizeof(double2) + 2 * (nx / 2 + 1) * ny * sizeof(double) +
+           (c->state == PIC_STATE_F32 ? (nx + ES_EPAD) * ny * sizeof(float2) + nx * ny * 4
+                                      : nx * ny * 8);
 }
 
 template <int K, bool F32>
@@ -469,7 +560,7 @@ static int es_launch(const Ctx *c, const EsStep &a, size_t sm) {
 int es_run(Ctx *c, int kernel, double dt, int nsteps) {
     const int64_t m = (int64_t)c->nx * c->ny;
     // three raw charge buffers, then the twiddles
-    const size_t ntw = (size_t)(c->nx / 2 + c->ny / 2);
+    const size_t ntw = (size_t)(c->nx + c->ny);
     if (!c->es_buf) PIC_HIP(hipMalloc(&c->es_buf, (size_t)(3 * m) * 8 + ntw * sizeof(double2)));
     if (c->pending_perm) PIC_TRY(settle_state(c));
     const bool f32 = c->state == PIC_STATE_F32;
@@ -484,7 +575,7 @@ int es_run(Ctx *c, int kernel, double dt, int nsteps) {
     a.logny = log2_of(c->ny);
     a.nbp = nb;
     double2 *tw = reinterpret_cast<double2 *>(c->es_buf + 3 * m);
-    hipLaunchKernelGGL(k_es_twiddles, dim3(1), dim3(64), 0, c->stream, a.nx, a.ny, a.lognx,
+    hipLaunchKernelGGL(k_es_twiddles, dim3(1), dim3(2 * ES_MAX_SIDE), 0, c->stream, a.nx, a.ny, a.lognx,
                        a.logny, tw);
     PIC_HIP(hipGetLastError());
     a.tw = tw;

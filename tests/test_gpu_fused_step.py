@@ -155,3 +155,27 @@ def test_fused_step_tiny_grids(gpu, O, grid):
         assert np.max(np.abs(np.sqrt(e[:, 0]) - eo) / eo) < 1e-10
         assert np.max(_pdist(got[0], q[0], mesh.dimx)) < 1e-9
         assert np.max(np.abs(got[2:4] - q[2:4])) < 1e-9
+
+
+@pytest.mark.parametrize("nx", [4, 8, 16, 32, 64])
+@pytest.mark.parametrize("ny", [4, 8, 16, 32, 64])
+def test_fused_step_every_grid(gpu, nx, ny):
+    """Every grid of the one-launch loop (each side its own transform): the
+    field and charge of the third step on random particles, which fill the
+    whole spectrum, against the separate-kernel loop.  1e-12 normwise: the
+    two solves' transforms of at most 64 points round at a few 1e-16 of the
+    field, and three steps carry that on."""
+    pic = gpu
+    rng = np.random.default_rng(64 * nx + ny)
+    mesh = pic.TwoDGrid(4 * np.pi, nx, 3.0, ny)
+    p = random_particles(rng, 3_001, mesh.dimx, mesh.dimy)
+    got = []
+    for fused in (True, False):
+        sim = pic.Simulation(mesh, p, pic.M6())
+        sim.set_fused_step(fused)
+        e = sim.run(0.05, 3)
+        got.append([e] + [sim.grid(k) for k in (pic._lib.PIC_GRID_RHO, pic._lib.PIC_GRID_EX,
+                                                pic._lib.PIC_GRID_EY)])
+        sim.close()
+    for a, b in zip(*got):
+        assert np.linalg.norm(a - b) <= 1e-12 * np.linalg.norm(b)
