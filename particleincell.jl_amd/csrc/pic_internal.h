@@ -66,6 +66,16 @@ struct Ctx {
     float4 *ov32 = nullptr;
     void *swap = nullptr;               // 40 B/particle reorder scratch
     int64_t swap_bytes = 0;
+    // device staging of the host transfers (pic_api.hip, at most STAGE_KEEP
+    // bytes), and the weights' verdict: a device flag and its pinned host copy
+    void *stage = nullptr;
+    int64_t stage_bytes = 0;
+    double *grid_host = nullptr;  // pinned, nx*ny (grids of at most GRID_PINNED)
+    unsigned *w_flag = nullptr;
+    struct Weights {
+        double w0;
+        int differ;
+    } *w_host = nullptr;
     // second set of state arrays: the sort gathers into these and swaps the
     // pointers (keyed by the address of the Ctx member they pair with)
     static constexpr int NALT = 10;

@@ -1,0 +1,98 @@
+"""Particles and grids between host and device: the weights' verdict wherever a
+weight differs, transfers below and above the size of the kept staging buffer,
+and grids of every layout on both sides of the pinned copy's size."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _context(pic, nx, ny):
+    return pic.api.Context(pic.TwoDGrid(1.0, nx, 1.0, ny))
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 4_097, 1_700_003])
+def test_particles_come_back_and_weights_are_judged(gpu, n):
+    """Bitwise round trips of one context, uniform and weighted in turn: the
+    FP32 state is refused exactly when a weight differs from the first (also
+    the last one, or a NaN)."""
+    pic = gpu
+    ctx = _context(pic, 16, 16)
+    rng = np.random.default_rng(n)
+    p = np.asfortranarray(rng.uniform(0.01, 0.99, (5, n)))
+    for odd in (None, n - 1, None, n // 2, None):
+        p[4] = 0.25
+        differ = odd is not None and n > 1 and odd > 0
+        if odd is not None:
+            p[4, odd] = np.nan if odd == n // 2 else 0.5
+            differ = differ or n == 1 and bool(np.isnan(p[4, 0]))
+        ctx.set_particles(p)
+        np.testing.assert_array_equal(ctx.get_particles(np.empty_like(p)), p)
+        if differ:
+            with pytest.raises(Exception):
+                ctx.set_state(1)
+        else:
+            ctx.set_state(1)
+    ctx.close()
+
+
+@pytest.mark.parametrize("nx,ny", [(4, 4), (33, 20), (512, 256), (400, 350)])
+def test_grids_of_every_layout(gpu, nx, ny):
+    """Set and read back bitwise: packed, with a ghost line to skip, strided;
+    read packed and with the ghost line.  400 x 350 is past the pinned copy."""
+    pic = gpu
+    L = pic._lib
+    ctx = _context(pic, nx, ny)
+    rng = np.random.default_rng(nx)
+    for which in (L.PIC_GRID_RHO, L.PIC_GRID_EX, L.PIC_GRID_EY, L.PIC_GRID_BZ, L.PIC_GRID_PHI):
+        for layout in ("packed", "ghost", "strided"):
+            g = rng.standard_normal((nx, ny))
+            if layout == "packed":
+                ctx.set_grid(which, np.asfortranarray(g))
+            elif layout == "ghost":
+                a = np.full((nx + 1, ny + 1), np.nan, order="F")
+                a[:nx, :ny] = g
+                ctx.set_grid(which, a)
+            else:
+                a = np.full((2, nx, ny), np.nan, order="F")
+                a[0] = g
+                ctx.set_grid(which, a, stride=2)
+            np.testing.assert_array_equal(ctx.get_grid(which), g)
+            full = ctx.get_grid(which, ghost=True)
+            np.testing.assert_array_equal(full[:nx, :ny], g)
+            np.testing.assert_array_equal(full[nx], full[0])
+            np.testing.assert_array_equal(full[:, ny], full[:, 0])
+    ctx.close()
+
+
+@pytest.mark.parametrize("nx,ny", [(32, 16), (512, 512)])
+@pytest.mark.parametrize("order", ["xy", "yx"])
+def test_fields_set_reach_the_fp32_pass(gpu, nx, ny, order):
+    """A kick after ex, ey and bz were set (either first) in FP32 agrees with
+    the FP64 pass.  Bound: offsets, fields and weights rounded to FP32, a cubic
+    of at most 16 weights: under 64 roundings of 6e-8 of the kick (at most 4)."""
+    pic = gpu
+    L = pic._lib
+    rng = np.random.default_rng(nx)
+    n = 5_000
+    p = np.asfortranarray(rng.uniform(0.01, 0.99, (5, n)))
+    p[2:4] *= 1e-3
+    p[4] = 1.0 / n
+    grids = {w: np.asfortranarray(rng.uniform(-1, 1, (nx, ny)))
+             for w in (L.PIC_GRID_EX, L.PIC_GRID_EY, L.PIC_GRID_BZ)}
+    seq = [L.PIC_GRID_EX, L.PIC_GRID_EY, L.PIC_GRID_BZ]
+    if order == "yx":
+        seq.reverse()
+    v = []
+    for state in (0, 1):
+        ctx = _context(pic, nx, ny)
+        ctx.set_particles(p)
+        ctx.set_state(state)
+        for w in seq:
+            ctx.set_grid(w, grids[w])
+        ctx.set_bz(L.PIC_BZ_GRID)
+        L.call("pic_step_pass", ctx.h, 0, 2, 1e-3, None)
+        v.append(ctx.get_particles(np.empty_like(p))[2:4])
+        ctx.close()
+    assert np.abs(v[0] - p[2:4]).max() > 1e-4
+    assert np.abs(v[0] - v[1]).max() <= 64 * 2.0**-24 * 4e-3
