@@ -366,6 +366,20 @@ __device__ __forceinline__ int cell_of(double xp, double fl, int n, double &d) {
     return i;
 }
 
+// a / b for a divisor used several times: with r = 1/b rounded, q = a r and
+// one correction by the exact remainder a - q b give the rounded quotient
+// (Markstein), 3 operations against about 14 of a division.
+struct Div {
+    double b, r;
+    __host__ __device__ Div() {}
+    __host__ __device__ explicit Div(double b_) : b(b_), r(1.0 / b_) {}
+    __host__ __device__ Div(double b_, double r_) : b(b_), r(r_) {}
+    __device__ __forceinline__ double of(double a) const {
+        const double q = a * r;
+        return __builtin_fma(__builtin_fma(-q, b, a), r, q);
+    }
+};
+
 // Quintic B-spline (M6) weights of nodes i-2..i+3 at offset t in [0,1), FP32.
 // The pieces of f_m6 (compute_rho_m6.jl:10-25) are 120 w5 = t^5, 120 w4 =
 // P4(t) = 1+5t+10t^2+10t^3+5t^4-5t^5, 120 w3 = P3(t) =

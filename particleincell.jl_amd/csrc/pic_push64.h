@@ -20,7 +20,11 @@ struct SegF64 {
     const double *ex, *ey, *bz;
     double bz0;
     int nx, ny, ncells;
-    double dx, dy, dimx, dimy, dt, dtd;
+    picd::Div dx, dy;
+    double dimx, dimy, dt, dtd;
+    // uniform weight w0 = wm 2^we that fixed-point charge sums may take (fix)
+    double wm;
+    int we, fix;
     double *acc;
     const int64_t *off;
     int bps, margin, cap;
@@ -34,6 +38,10 @@ struct SegF64 {
 // x >= 0), d = (xp - i) + 1; returns the 0-based wrapped cell.
 __device__ __forceinline__ int ref_cell_s(double x, double dx, int n, bool trunc_, double &d) {
     const double xp = x / dx;
+    return picd::cell_of(xp, trunc_ ? trunc(xp) : floor(xp), n, d);
+}
+__device__ __forceinline__ int ref_cell_s(double x, picd::Div dx, int n, bool trunc_, double &d) {
+    const double xp = dx.of(x);
     return picd::cell_of(xp, trunc_ ? trunc(xp) : floor(xp), n, d);
 }
 
@@ -148,6 +156,44 @@ __device__ __forceinline__ void charge64(double fx, double fy, int ci, int cj, d
         for (int u = 0; u < S; ++u)
 #pragma unroll
             for (int v = 0; v < S; ++v) add(u, v, wx[u] * wy[v] * wgt);
+    }
+}
+
+// Charge in units of a power-of-two quantum, in 64-bit integers: share (u, v)
+// is w_u w_v wu rounded to a whole number by adding C = 1.5 2^52, whose bits
+// come off again (one v_lshl_add_u64), so |share| must stay below 2^51.  Sums
+// of shares are exact.
+// Measured on MI355X, 1024 threads per CU on one 36-node stencil each: a
+// 64-lane ds_add_f64 takes 8.4 clocks with the lanes in adjacent cells and
+// 20-26 once the particles have drifted (two tile copies), a ds_add_u64 6.5
+// and 10.5-14.
+template <int K>
+constexpr int charge64_bits() {
+    return K == PIC_M6 ? 1 : 0;  // a share is at most 2^-bits of the weight
+}
+template <int K, class F>
+__device__ __forceinline__ void charge64_fixed(double fx, double fy, int ci, int cj, double wu,
+                                               F &&add) {
+    constexpr int S = Shape<K>::S;
+    constexpr double C = 6755399441055744.0;
+    double wx[6], wy[6];
+    if (K == PIC_CIC) {
+        wx[0] = 1 - fx;
+        wx[1] = fx;
+        wy[0] = 1 - fy;
+        wy[1] = fy;
+    } else {
+        deposit_w<K>(fx, ci, wx);
+        deposit_w<K>(fy, cj, wy);
+    }
+#pragma unroll
+    for (int v = 0; v < S; ++v) {
+        const double q = wy[v] * wu;
+#pragma unroll
+        for (int u = 0; u < S; ++u)
+            add(u, v,
+                (unsigned long long)(__double_as_longlong(__builtin_fma(wx[u], q, C)) -
+                                     __double_as_longlong(C)));
     }
 }
 

@@ -586,7 +586,7 @@ int es_run(Ctx *c, int kernel, double dt, int nsteps) {
     s.w0 = c->w0;
     s.bz0 = c->bz0;
     s.nx = c->nx; s.ny = c->ny; s.ncells = (int)m;
-    s.dx = c->dx; s.dy = c->dy; s.dimx = c->dimx; s.dimy = c->dimy;
+    s.dx = picd::Div(c->dx); s.dy = picd::Div(c->dy); s.dimx = c->dimx; s.dimy = c->dimy;
     s.dt = dt;
     s.dtd = 0.5 * dt;
     a.cell = c->cell;

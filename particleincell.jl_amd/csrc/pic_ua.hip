@@ -68,18 +68,9 @@ __device__ __forceinline__ int bitrev(int m) {
 
 constexpr int ilog2(int n) { return n <= 1 ? 0 : 1 + ilog2(n / 2); }
 
-// a / b for a divisor used several times: with r = 1/b rounded, q = a r and
-// one correction by the exact remainder a - q b give the rounded quotient
-// (Markstein), 3 operations against about 14 of a division.
-struct Div {
-    double b, r;
-    __host__ __device__ Div() {}
-    __host__ __device__ explicit Div(double b_) : b(b_), r(1.0 / b_) {}
-    __device__ Div(double b_, double r_) : b(b_), r(r_) {}
-    __device__ __forceinline__ double of(double a) const {
-        const double q = a * r;
-        return __builtin_fma(__builtin_fma(-q, b, a), r, q);
-    }
+struct Div : picd::Div {
+    using picd::Div::Div;
+    using picd::Div::of;
     __device__ __forceinline__ cd of(cd a) const { return {of(a.re), of(a.im)}; }
 };
 
