@@ -65,9 +65,9 @@ struct SegF32 {
     int32_t *cell;  // state written by the pass (slot p)
     float4 *ov;     // (ox, oy, vx, vy)
     // state read by the pass: the same arrays, or, right after a lane sort
-    // whose permutation has not been applied, the unsorted arrays read at
-    // perm[p] (the pass then moves every particle into its sorted slot)
-    const int32_t *cell_in;
+    // whose permutation has not been applied, the unsorted offsets and
+    // velocities read at perm[p] (the pass then moves every particle into its
+    // sorted slot) and the cells where that sort left them, in the sorted slots
     const float4 *ov_in;
     const uint32_t *perm;
     float w;
@@ -329,7 +329,7 @@ __global__ __launch_bounds__((seg32_threads<K, DRIFT, DEPOSIT, ACC>()),
     constexpr bool PREFETCH = seg32_wide<K, DRIFT, DEPOSIT, ACC>();
     if (PREFETCH && (uint32_t)p0 + tid < (uint32_t)p1) {
         const uint32_t src = PERM ? a.perm[(uint32_t)p0 + tid] : (uint32_t)p0 + tid;
-        c_next = a.cell_in[src];
+        c_next = a.cell[(uint32_t)p0 + tid];
         o_next = a.ov_in[src];
     }
     for (uint32_t p = (uint32_t)p0 + tid; p < (uint32_t)p1; p += BT) {
@@ -343,11 +343,11 @@ __global__ __launch_bounds__((seg32_threads<K, DRIFT, DEPOSIT, ACC>()),
             // kept for a skipped load (five register moves per particle)
             const uint32_t q = min(p + (uint32_t)BT, (uint32_t)p1 - 1u);
             const uint32_t src = PERM ? a.perm[q] : q;
-            c_next = a.cell_in[src];
+            c_next = a.cell[q];
             o_next = a.ov_in[src];
         } else {
             const uint32_t src = PERM ? a.perm[p] : p;
-            c = a.cell_in[src];
+            c = a.cell[p];
             o = a.ov_in[src];
         }
         int ci = c & mx, cj = c >> a.lognx;
@@ -469,7 +469,7 @@ __global__ __launch_bounds__(DEFER_T) void k_defer_f32(SegF32 a) {
         // a whole particle has not been touched: read it where the pass
         // would have; a deposit-only one is already in its slot
         const uint32_t src = (PERM && whole) ? a.perm[p] : (uint32_t)p;
-        const int c = whole ? a.cell_in[src] : a.cell[p];
+        const int c = a.cell[p];
         int ci = c & mx, cj = c >> a.lognx;
         const float4 o = whole ? a.ov_in[src] : a.ov[p];
         float fx = o.x, fy = o.y;
@@ -811,7 +811,7 @@ int launch_seg32(Ctx *c, int kernel, int mode, double dt, double dtd) {
     PIC_CHECK(c->seg_valid, PIC_ERR_STATE, "segment passes need a lane sort first");
     SegF32 a;
     a.cell = c->cell; a.ov = c->ov32;
-    a.cell_in = c->cell; a.ov_in = c->ov32;
+    a.ov_in = c->ov32;
     a.perm = c->pending_perm;
     if (a.perm) PIC_TRY(alt_f32(c, &a.cell, &a.ov));
     a.w = (float)c->w0;

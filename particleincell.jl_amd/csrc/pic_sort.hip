@@ -347,7 +347,7 @@ __global__ __launch_bounds__(LANE_T) void k_lane_transpose(
     const uint32_t *__restrict__ val, const int64_t *__restrict__ off, int ncells,
     const uint32_t *__restrict__ kmax, const uint32_t *__restrict__ tbl,
     const uint32_t *__restrict__ A, const unsigned long long *__restrict__ M,
-    uint32_t *__restrict__ perm2) {
+    uint32_t *__restrict__ perm2, int32_t *__restrict__ cell) {
     __shared__ uint32_t tile[LANE_KC][65];
     __shared__ int64_t coff[65];
     const int s = blockIdx.x;
@@ -376,7 +376,9 @@ __global__ __launch_bounds__(LANE_T) void k_lane_transpose(
                 const unsigned long long m = M[tb + k];
                 if ((m >> l) & 1ull) {
                     const unsigned long long below = l ? (m & (~0ull >> (64 - l))) : 0ull;
-                    perm2[sbase + A[tb + k] + __popcll(below)] = tile[kk][l];
+                    const int64_t slot = sbase + A[tb + k] + __popcll(below);
+                    perm2[slot] = tile[kk][l];
+                    if (cell) cell[slot] = c0 + l;
                 }
             }
         }
@@ -688,11 +690,18 @@ int sort_by_cell(Ctx *c, int32_t *perm_host, bool lanes, bool apply) {
         const int64_t chunks = (per_cell + LANE_KC - 1) / LANE_KC + 1;
         const int64_t want = std::max<int64_t>(1, (int64_t)c->ncu * 16 / nseg);
         const unsigned gy = (unsigned)std::max<int64_t>(1, std::min<int64_t>(chunks, want));
+        // a permutation left pending in FP32 state: the cells go to their slots
+        // of the alternate array at once, in order, where the pass that applies
+        // it would read one of them per particle from anywhere
+        int32_t *slot_cell = nullptr;
+        float4 *slot_ov = nullptr;
+        if (c->state == PIC_STATE_F32 && !apply && !perm_host)
+            PIC_TRY(alt_f32(c, &slot_cell, &slot_ov));
         hipLaunchKernelGGL(k_lane_transpose, dim3((unsigned)nseg, gy), dim3(LANE_T), 0,
                            c->stream, (const uint32_t *)c->sort_vals[0],
                            (const int64_t *)c->cell_off, ncells, (const uint32_t *)c->seg_k,
                            (const uint32_t *)c->seg_tbl, (const uint32_t *)c->seg_A,
-                           (const unsigned long long *)c->seg_M, c->perm2);
+                           (const unsigned long long *)c->seg_M, c->perm2, slot_cell);
         PIC_HIP(hipGetLastError());
         perm = c->perm2;
         c->seg_valid = true;
