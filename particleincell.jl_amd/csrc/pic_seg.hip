@@ -12,11 +12,17 @@
 //   3. flushes the non-zero charge nodes with FP64 global atomics, once.
 // No block-wide synchronisation inside the particle loop.  A particle whose
 // stencil leaves the window (drifted further than the margin since the sort)
-// is appended to a deferred list instead, whole or for its deposit only; a
-// small kernel launched after the pass completes those from global memory
-// with the same arithmetic and counts them.  Keeping the global-memory path
-// out of the pass kernel keeps its register count, and so its occupancy, at
-// what the LDS path needs.
+// is appended to a deferred list instead, whole or for its deposit only, and
+// completed from global memory with the same arithmetic, and counted.  The
+// 1024-thread passes (seg32_wide, FP64) keep a list per block, in the block's
+// own slice of it, and complete it themselves after the particle loop, where
+// their register count has room for that path; after the others a small
+// kernel completes the list of all blocks, which keeps that path's registers
+// out of them.  Measured on MI355X: the small kernel took 9.6 us a step for
+// FP32 M6 (1e7 particles, 128^2), 11.5 for FP64, 4.6 for 300,007 TSC
+// particles on 100 x 75, next to nothing of it left in the pass (148, 290
+// and 19 us with either); 2e8 M6 particles on 512^2 with a sort every 4
+// steps: pass 3.69 ms and list 0.31 -> 3.21 ms.
 //
 // Arithmetic per particle is the same as in pic_step.hip's kernels (FP64:
 // the reference's operations; FP32: the cell-relative step), so results are
@@ -171,7 +177,7 @@ __device__ __forceinline__ int64_t packed_half(const unsigned long long *tile, i
 // The particles of one segment slice.  A particle whose stencil lies outside
 // the block's LDS window is not touched here: it goes to the deferred list
 // whole (gather outside) or for its deposit only (drifted outside), and
-// k_defer_f32 completes it from global memory after this kernel.
+// is completed from global memory after the particle loop (or by k_defer_f32).
 //
 // Register budget: the passes with 40 KiB windows are held to 64 VGPRs
 // (eight waves per SIMD), so that four blocks share a CU instead of the three
@@ -231,6 +237,59 @@ constexpr int seg32_threads() {
     return seg32_wide<K, DRIFT, DEPOSIT, ACC>() ? 1024 : SEG_T;
 }
 
+// Completes one particle that k_seg_f32 deferred (entry e of its list), from
+// global memory with the same arithmetic.
+template <int K, bool GATHER, bool DRIFT, bool DEPOSIT, int BZ, bool PERM>
+__device__ __forceinline__ void defer_f32(const SegF32 &a, uint32_t e) {
+    constexpr int HL = SegStencil<K>::HL;
+    const int nx = a.nx, mx = a.nx - 1, my = a.ny - 1;
+    const int64_t p = e & ~DEFER_DEPOSIT_ONLY;
+    const bool whole = (e & DEFER_DEPOSIT_ONLY) == 0;
+    // a whole particle has not been touched: read it where the pass
+    // would have; a deposit-only one is already in its slot
+    const uint32_t src = (PERM && whole) ? a.perm[p] : (uint32_t)p;
+    const int c = a.cell[p];
+    int ci = c & mx, cj = c >> a.lognx;
+    const float4 o = whole ? a.ov_in[src] : a.ov[p];
+    float fx = o.x, fy = o.y;
+    if (whole) {
+        float ux = o.z, uy = o.w;
+        if (GATHER) {
+            float e1, e2, b3 = 0.0f;
+            interp32<K, BZ>(
+                fx, fy, ci, cj,
+                [&](int u, int v) {
+                    return a.e32[(int64_t)((ci - HL + u) & mx) +
+                                 (int64_t)nx * ((cj - HL + v) & my)];
+                },
+                [&](int u, int v) {
+                    return a.bz[(int64_t)((ci - HL + u) & mx) +
+                                (int64_t)nx * ((cj - HL + v) & my)];
+                },
+                e1, e2, b3);
+            kick32<BZ>(a.hdt, a.bz0, e1, e2, b3, ux, uy);
+        }
+        if (DRIFT) {
+            float nfx, nfy;
+            const int si = drift1s(fx, ux, a.dtdx, nfx);
+            const int sj = drift1s(fy, uy, a.dtdy, nfy);
+            ci = (ci + si) & mx;
+            cj = (cj + sj) & my;
+            fx = nfx;
+            fy = nfy;
+        }
+        if (DRIFT || PERM) a.cell[p] = ci + nx * cj;
+        if (GATHER || DRIFT || PERM) a.ov[p] = make_float4(fx, fy, ux, uy);
+    }
+    if (DEPOSIT)
+        charge32<K>(fx, fy, ci, cj, a.w, [&](int u, int v, float q) {
+            unsafeAtomicAdd(
+                &a.acc[(int64_t)((ci - HL + u) & mx) + (int64_t)nx * ((cj - HL + v) & my)],
+                (double)q);
+        });
+}
+
+constexpr size_t SEG_OWN_BYTES = 16;
 constexpr size_t SEG_KICK_LDS_BYTES = 160 * 1024;  // the pass without a deposit
 
 template <int K, bool GATHER, bool DRIFT, bool DEPOSIT, int BZ, int ACC, bool PERM>
@@ -239,7 +298,11 @@ __global__ __launch_bounds__((seg32_threads<K, DRIFT, DEPOSIT, ACC>()),
     constexpr int BT = seg32_threads<K, DRIFT, DEPOSIT, ACC>();
     using St = SegStencil<K>;
     constexpr int S = St::S, HL = St::HL;
-    extern __shared__ __align__(16) char smem_s32[];
+    // a pass that completes its deferred particles itself keeps its list in
+    // entries [p0, p1), and its length before the tiles
+    constexpr bool OWN = seg32_wide<K, DRIFT, DEPOSIT, ACC>();
+    extern __shared__ __align__(16) char smem32[];
+    char *smem_s32 = smem32 + (OWN ? SEG_OWN_BYTES : 0);
     const int tid = threadIdx.x;
     const int nx = a.nx, ny = a.ny;
     const int mx = nx - 1, my = ny - 1;  // nx, ny are powers of two
@@ -280,6 +343,9 @@ __global__ __launch_bounds__((seg32_threads<K, DRIFT, DEPOSIT, ACC>()),
     const double unit = !FIX                      ? 0.0
                         : (conserve && R != 0) ? (double)a.w / R
                                                : copysign(ldexp(1.0, qe), (double)a.w);
+    uint32_t *dlist = OWN ? a.dlist + p0 : a.dlist;
+    unsigned *dcount = OWN ? reinterpret_cast<unsigned *>(smem32) : a.dcount;
+    if (OWN && tid == 0) *dcount = 0;
     float2 *teA = reinterpret_cast<float2 *>(smem_s32);
     float2 *teB = teA + cap;  // cap is a multiple of 16: 16-byte aligned
     float *tb = reinterpret_cast<float *>(smem_s32 + 16 * (size_t)cap);
@@ -355,7 +421,7 @@ __global__ __launch_bounds__((seg32_threads<K, DRIFT, DEPOSIT, ACC>()),
         if (GATHER) {
             const int lx = (ci - ox) & mx, ly = (cj - oy) & my;
             const bool in = fits && lx + S - 1 < W.tw && ly + S - 1 < W.th;
-            defer_push(!in, (uint32_t)p, a.dlist, a.dcount);
+            defer_push(!in, (uint32_t)p, dlist, dcount);
             if (!in) continue;
             float e1, e2, b3 = 0.0f;
             const int odd = lx & 1;
@@ -381,7 +447,7 @@ __global__ __launch_bounds__((seg32_threads<K, DRIFT, DEPOSIT, ACC>()),
         if (DEPOSIT) {
             const int lx = (ci - ox) & mx, ly = (cj - oy) & my;
             const bool in = fits && lx + S - 1 < W.tw && ly + S - 1 < W.th;
-            defer_push(!in, (uint32_t)p | DEFER_DEPOSIT_ONLY, a.dlist, a.dcount);
+            defer_push(!in, (uint32_t)p | DEFER_DEPOSIT_ONLY, dlist, dcount);
             if (!in) continue;
             if (ACC == 2) {
                 charge32_fixed<K>(fx, fy, ci, cj, wu, R, conserve, [&](int u, int v, int qi) {
@@ -425,8 +491,15 @@ __global__ __launch_bounds__((seg32_threads<K, DRIFT, DEPOSIT, ACC>()),
             });
         }
     }
-    if (!DEPOSIT || !fits) return;
+    if (!OWN && (!DEPOSIT || !fits)) return;
     __syncthreads();
+    if (OWN) {
+        const unsigned cnt = *dcount;
+        for (unsigned i = tid; i < cnt; i += BT)
+            defer_f32<K, GATHER, DRIFT, DEPOSIT, BZ, PERM>(a, dlist[i]);
+        if (tid == 0 && cnt) atomicAdd(a.slow, (unsigned long long)cnt);
+        if (!DEPOSIT || !fits) return;
+    }
     const int nt = W.tw * W.th;
     for (int t = tid; t < nt; t += BT) {
         const int u = t % W.tw, v = t / W.tw;
@@ -454,67 +527,80 @@ __global__ __launch_bounds__((seg32_threads<K, DRIFT, DEPOSIT, ACC>()),
     }
 }
 
-// Completes the particles k_seg_f32 deferred, from global memory (same
-// arithmetic), adds their number to the slow-path counter, and the last
-// block to finish resets the list for the next pass.
+// The deferred list of a pass that does not complete its own (seg32_wide):
+// adds its length to the slow-path counter, and the last block to finish
+// resets it for the next pass.
 template <int K, bool GATHER, bool DRIFT, bool DEPOSIT, int BZ, bool PERM>
 __global__ __launch_bounds__(DEFER_T) void k_defer_f32(SegF32 a) {
-    constexpr int HL = SegStencil<K>::HL;
     const unsigned cnt = __hip_atomic_load(a.dcount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int nx = a.nx, mx = a.nx - 1, my = a.ny - 1;
-    for (unsigned i = blockIdx.x * DEFER_T + threadIdx.x; i < cnt; i += gridDim.x * DEFER_T) {
-        const uint32_t e = a.dlist[i];
-        const int64_t p = e & ~DEFER_DEPOSIT_ONLY;
-        const bool whole = (e & DEFER_DEPOSIT_ONLY) == 0;
-        // a whole particle has not been touched: read it where the pass
-        // would have; a deposit-only one is already in its slot
-        const uint32_t src = (PERM && whole) ? a.perm[p] : (uint32_t)p;
-        const int c = a.cell[p];
-        int ci = c & mx, cj = c >> a.lognx;
-        const float4 o = whole ? a.ov_in[src] : a.ov[p];
-        float fx = o.x, fy = o.y;
-        if (whole) {
-            float ux = o.z, uy = o.w;
-            if (GATHER) {
-                float e1, e2, b3 = 0.0f;
-                interp32<K, BZ>(
-                    fx, fy, ci, cj,
-                    [&](int u, int v) {
-                        return a.e32[(int64_t)((ci - HL + u) & mx) +
-                                     (int64_t)nx * ((cj - HL + v) & my)];
-                    },
-                    [&](int u, int v) {
-                        return a.bz[(int64_t)((ci - HL + u) & mx) +
-                                    (int64_t)nx * ((cj - HL + v) & my)];
-                    },
-                    e1, e2, b3);
-                kick32<BZ>(a.hdt, a.bz0, e1, e2, b3, ux, uy);
-            }
-            if (DRIFT) {
-                float nfx, nfy;
-                const int si = drift1s(fx, ux, a.dtdx, nfx);
-                const int sj = drift1s(fy, uy, a.dtdy, nfy);
-                ci = (ci + si) & mx;
-                cj = (cj + sj) & my;
-                fx = nfx;
-                fy = nfy;
-            }
-            if (DRIFT || PERM) a.cell[p] = ci + nx * cj;
-            if (GATHER || DRIFT || PERM) a.ov[p] = make_float4(fx, fy, ux, uy);
-        }
-        if (DEPOSIT)
-            charge32<K>(fx, fy, ci, cj, a.w, [&](int u, int v, float q) {
-                unsafeAtomicAdd(
-                    &a.acc[(int64_t)((ci - HL + u) & mx) + (int64_t)nx * ((cj - HL + v) & my)],
-                    (double)q);
-            });
-    }
+    for (unsigned i = blockIdx.x * DEFER_T + threadIdx.x; i < cnt; i += gridDim.x * DEFER_T)
+        defer_f32<K, GATHER, DRIFT, DEPOSIT, BZ, PERM>(a, a.dlist[i]);
     defer_finish(cnt, a.dcount, a.slow);
 }
 
 // ============================================================ FP64 state
 
-// FP64 counterpart of k_seg_f32; out-of-window particles go to k_defer_f64.
+// Completes one particle that k_seg_f64 deferred, from global memory.
+template <int K, bool GATHER, int NDRIFT, bool DEPOSIT, int BZ, bool PERM>
+__device__ __forceinline__ void defer_f64(const SegF64 &a, uint32_t e) {
+    constexpr int HL = SegStencil<K>::HL;
+    const int nx = a.nx, ny = a.ny;
+    const int64_t p = e & ~DEFER_DEPOSIT_ONLY;
+    const bool whole = (e & DEFER_DEPOSIT_ONLY) == 0;
+    // a whole particle is read where the pass would have read it; a
+    // deposit-only one is already in its slot
+    const uint32_t src = (PERM && whole) ? a.perm[p] : (uint32_t)p;
+    double px = whole ? a.x_in[src] : a.x[p], py = whole ? a.y_in[src] : a.y[p];
+    const double wgt = !a.w ? a.w0 : whole ? a.w[src] : PERM ? a.w_out[p] : a.w[p];
+    if (whole) {
+        double pvx = 0.0, pvy = 0.0;
+        if (GATHER || NDRIFT > 0 || PERM) {
+            pvx = a.vx_in[src];
+            pvy = a.vy_in[src];
+        }
+        if (GATHER) {
+            double fx, fy;
+            const int ci = ref_cell_s(px, a.dx, nx, false, fx);
+            const int cj = ref_cell_s(py, a.dy, ny, false, fy);
+            double e1, e2, b3 = 0.0;
+            interp64<K, BZ>(
+                fx, fy, ci, cj,
+                [&](int u, int v) {
+                    const int64_t g = (int64_t)picd::wrap2(ci - HL + u, nx) +
+                                      (int64_t)nx * picd::wrap2(cj - HL + v, ny);
+                    return make_double2(a.ex[g], a.ey[g]);
+                },
+                [&](int u, int v) {
+                    return a.bz[(int64_t)picd::wrap2(ci - HL + u, nx) +
+                                (int64_t)nx * picd::wrap2(cj - HL + v, ny)];
+                },
+                e1, e2, b3);
+            kick64<BZ>(a, e1, e2, b3, pvx, pvy);
+        }
+        if (NDRIFT > 0) drift64<NDRIFT>(a, pvx, pvy, px, py);
+        if (GATHER || PERM) {
+            a.vx[p] = pvx;
+            a.vy[p] = pvy;
+        }
+        if (NDRIFT > 0 || PERM) {
+            a.x[p] = px;
+            a.y[p] = py;
+        }
+        if (PERM && a.w) a.w_out[p] = a.w[src];
+    }
+    if (DEPOSIT) {
+        double fx, fy;
+        const int ci = ref_cell_s(px, a.dx, nx, K == PIC_CIC, fx);
+        const int cj = ref_cell_s(py, a.dy, ny, K == PIC_CIC, fy);
+        charge64<K>(fx, fy, ci, cj, wgt, [&](int u, int v, double q) {
+            unsafeAtomicAdd(&a.acc[(int64_t)picd::wrap2(ci - HL + u, nx) +
+                                   (int64_t)nx * picd::wrap2(cj - HL + v, ny)],
+                            q);
+        });
+    }
+}
+
+// FP64 counterpart of k_seg_f32.
 // LDS bounds it: 36 16-byte reads and 36 adds a particle for M6, and the lanes
 // of drifted particles collide.  With the charge in 64-bit fixed point and the
 // cells' divisions by reciprocals, Landau M6, 1e7 particles on 128^2: 391 ->
@@ -536,7 +622,11 @@ template <int K, bool GATHER, int NDRIFT, bool DEPOSIT, int BZ, bool PERM>
 __global__ __launch_bounds__(SEG64_T) void k_seg_f64(SegF64 a) {
     using St = SegStencil<K>;
     constexpr int S = St::S, HL = St::HL;
-    extern __shared__ __align__(16) char smem_s64[];
+    // the block completes its deferred particles itself: its list in entries
+    // [p0, p1), its length before the tiles
+    extern __shared__ __align__(16) char smem64[];
+    char *smem_s64 = smem64 + SEG_OWN_BYTES;
+    unsigned *dcount = reinterpret_cast<unsigned *>(smem64);
     const int tid = threadIdx.x;
     const int nx = a.nx, ny = a.ny;
     const int s = blockIdx.x / a.bps, bi = blockIdx.x - s * a.bps;
@@ -547,6 +637,8 @@ __global__ __launch_bounds__(SEG64_T) void k_seg_f64(SegF64 a) {
     const Win W = seg_window<S, HL>(s, nx, ny, a.ncells, a.margin, a.cap);
     const bool fits = W.tw * W.th <= a.cap;
     const int cap = a.cap;
+    uint32_t *dlist = a.dlist + p0;
+    if (tid == 0) *dcount = 0;
     double2 *te = reinterpret_cast<double2 *>(smem_s64);
     double *tb = reinterpret_cast<double *>(smem_s64 + 16 * (size_t)cap);
     // two copies of the charge tile, lane l adding into copy l mod 2
@@ -594,7 +686,7 @@ __global__ __launch_bounds__(SEG64_T) void k_seg_f64(SegF64 a) {
             const int cj = ref_cell_s(py, a.dy, ny, false, fy);
             const int lx = picd::wrap2(ci - HL - W.x0, nx), ly = picd::wrap2(cj - HL - W.y0, ny);
             const bool in = fits && lx + S - 1 < W.tw && ly + S - 1 < W.th;
-            defer_push(!in, (uint32_t)p, a.dlist, a.dcount);
+            defer_push(!in, (uint32_t)p, dlist, dcount);
             if (!in) continue;
             pvx = a.vx_in[src];
             pvy = a.vy_in[src];
@@ -626,7 +718,7 @@ __global__ __launch_bounds__(SEG64_T) void k_seg_f64(SegF64 a) {
             // within the bounds: it goes to the FP64 path too)
             const bool in = fits && lx + S - 1 < W.tw && ly + S - 1 < W.th &&
                             fabs(fx - 0.5) <= 0.5 && fabs(fy - 0.5) <= 0.5;
-            defer_push(!in, (uint32_t)p | DEFER_DEPOSIT_ONLY, a.dlist, a.dcount);
+            defer_push(!in, (uint32_t)p | DEFER_DEPOSIT_ONLY, dlist, dcount);
             if (!in) continue;
             if (fix) {
                 charge64_fixed<K>(fx, fy, ci, cj, wu, [&](int u, int v, unsigned long long q) {
@@ -642,8 +734,12 @@ __global__ __launch_bounds__(SEG64_T) void k_seg_f64(SegF64 a) {
             });
         }
     }
-    if (!DEPOSIT || !fits) return;
     __syncthreads();
+    const unsigned cnt = *dcount;
+    for (unsigned i = tid; i < cnt; i += SEG64_T)
+        defer_f64<K, GATHER, NDRIFT, DEPOSIT, BZ, PERM>(a, dlist[i]);
+    if (tid == 0 && cnt) atomicAdd(a.slow, (unsigned long long)cnt);
+    if (!DEPOSIT || !fits) return;
     const int nt = W.tw * W.th;
     const double quantum = ldexp(1.0, a.we - bits);
     for (int t = tid; t < nt; t += SEG64_T) {
@@ -660,77 +756,16 @@ __global__ __launch_bounds__(SEG64_T) void k_seg_f64(SegF64 a) {
     }
 }
 
-// Completes the particles k_seg_f64 deferred, from global memory.
-template <int K, bool GATHER, int NDRIFT, bool DEPOSIT, int BZ, bool PERM>
-__global__ __launch_bounds__(DEFER_T) void k_defer_f64(SegF64 a) {
-    constexpr int HL = SegStencil<K>::HL;
-    const unsigned cnt = __hip_atomic_load(a.dcount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int nx = a.nx, ny = a.ny;
-    for (unsigned i = blockIdx.x * DEFER_T + threadIdx.x; i < cnt; i += gridDim.x * DEFER_T) {
-        const uint32_t e = a.dlist[i];
-        const int64_t p = e & ~DEFER_DEPOSIT_ONLY;
-        const bool whole = (e & DEFER_DEPOSIT_ONLY) == 0;
-        // a whole particle is read where the pass would have read it; a
-        // deposit-only one is already in its slot
-        const uint32_t src = (PERM && whole) ? a.perm[p] : (uint32_t)p;
-        double px = whole ? a.x_in[src] : a.x[p], py = whole ? a.y_in[src] : a.y[p];
-        const double wgt = !a.w ? a.w0 : whole ? a.w[src] : PERM ? a.w_out[p] : a.w[p];
-        if (whole) {
-            double pvx = 0.0, pvy = 0.0;
-            if (GATHER || NDRIFT > 0 || PERM) {
-                pvx = a.vx_in[src];
-                pvy = a.vy_in[src];
-            }
-            if (GATHER) {
-                double fx, fy;
-                const int ci = ref_cell_s(px, a.dx, nx, false, fx);
-                const int cj = ref_cell_s(py, a.dy, ny, false, fy);
-                double e1, e2, b3 = 0.0;
-                interp64<K, BZ>(
-                    fx, fy, ci, cj,
-                    [&](int u, int v) {
-                        const int64_t g = (int64_t)picd::wrap2(ci - HL + u, nx) +
-                                          (int64_t)nx * picd::wrap2(cj - HL + v, ny);
-                        return make_double2(a.ex[g], a.ey[g]);
-                    },
-                    [&](int u, int v) {
-                        return a.bz[(int64_t)picd::wrap2(ci - HL + u, nx) +
-                                    (int64_t)nx * picd::wrap2(cj - HL + v, ny)];
-                    },
-                    e1, e2, b3);
-                kick64<BZ>(a, e1, e2, b3, pvx, pvy);
-            }
-            if (NDRIFT > 0) drift64<NDRIFT>(a, pvx, pvy, px, py);
-            if (GATHER || PERM) {
-                a.vx[p] = pvx;
-                a.vy[p] = pvy;
-            }
-            if (NDRIFT > 0 || PERM) {
-                a.x[p] = px;
-                a.y[p] = py;
-            }
-            if (PERM && a.w) a.w_out[p] = a.w[src];
-        }
-        if (DEPOSIT) {
-            double fx, fy;
-            const int ci = ref_cell_s(px, a.dx, nx, K == PIC_CIC, fx);
-            const int cj = ref_cell_s(py, a.dy, ny, K == PIC_CIC, fy);
-            charge64<K>(fx, fy, ci, cj, wgt, [&](int u, int v, double q) {
-                unsafeAtomicAdd(&a.acc[(int64_t)picd::wrap2(ci - HL + u, nx) +
-                                       (int64_t)nx * picd::wrap2(cj - HL + v, ny)],
-                                q);
-            });
-        }
-    }
-    defer_finish(cnt, a.dcount, a.slow);
-}
-
 // ============================================================== dispatch
 
-// Launches the pass kernel `k` over every segment, then its deferred-list
-// kernel `kd`.
-template <class Kern, class Defer>
-static void seg32_launch(const Ctx *c, SegF32 a, Kern k, Defer kd, size_t sm, int bt) {
+// Launches the pass kernel over every segment, then, unless it completes its
+// deferred particles itself, its deferred-list kernel.
+template <int K, bool G, bool DR, bool D, int BZ, int ACC, bool P>
+static void seg32_launch(const Ctx *c, SegF32 a, size_t sm) {
+    constexpr int bt = seg32_threads<K, DR, D, ACC>();
+    constexpr bool own = seg32_wide<K, DR, D, ACC>();
+    const auto k = k_seg_f32<K, G, DR, D, BZ, ACC, P>;
+    if (own) sm += SEG_OWN_BYTES;
     // windows above 64 KiB need the kernel's dynamic LDS limit raised; a
     // failure here fails the launch, which hipGetLastError reports
     if (sm > 65536)
@@ -739,24 +774,17 @@ static void seg32_launch(const Ctx *c, SegF32 a, Kern k, Defer kd, size_t sm, in
     a.bps = seg_bps(c, reinterpret_cast<const void *>(k), sm, bt);
     dim3 grid((unsigned)(((c->nx * c->ny + 63) / 64) * a.bps));
     hipLaunchKernelGGL(k, grid, dim3(bt), sm, c->stream, a);
-    hipLaunchKernelGGL(kd, dim3(DEFER_BLOCKS), dim3(DEFER_T), 0, c->stream, a);
+    if constexpr (!own)
+        hipLaunchKernelGGL((k_defer_f32<K, G, DR, D, BZ, P>), dim3(DEFER_BLOCKS), dim3(DEFER_T), 0,
+                           c->stream, a);
 }
 
 template <int K, bool G, bool DR, bool D, int ACC, bool P>
 static void seg32_bz(const Ctx *c, const SegF32 &a, int bz, size_t sm) {
-    constexpr int bt = seg32_threads<K, DR, D, ACC>();
     switch (bz) {
-        case PIC_BZ_NONE:
-            seg32_launch(c, a, k_seg_f32<K, G, DR, D, PIC_BZ_NONE, ACC, P>,
-                         k_defer_f32<K, G, DR, D, PIC_BZ_NONE, P>, sm, bt);
-            break;
-        case PIC_BZ_UNIFORM:
-            seg32_launch(c, a, k_seg_f32<K, G, DR, D, PIC_BZ_UNIFORM, ACC, P>,
-                         k_defer_f32<K, G, DR, D, PIC_BZ_UNIFORM, P>, sm, bt);
-            break;
-        default:
-            seg32_launch(c, a, k_seg_f32<K, G, DR, D, PIC_BZ_GRID, ACC, P>,
-                         k_defer_f32<K, G, DR, D, PIC_BZ_GRID, P>, sm, bt);
+        case PIC_BZ_NONE: seg32_launch<K, G, DR, D, PIC_BZ_NONE, ACC, P>(c, a, sm); break;
+        case PIC_BZ_UNIFORM: seg32_launch<K, G, DR, D, PIC_BZ_UNIFORM, ACC, P>(c, a, sm); break;
+        default: seg32_launch<K, G, DR, D, PIC_BZ_GRID, ACC, P>(c, a, sm);
     }
 }
 
@@ -853,7 +881,9 @@ int launch_seg32(Ctx *c, int kernel, int mode, double dt, double dtd) {
     const size_t win = wide        ? (size_t)c->f32_window_kib * 1024
                        : mode == 2 ? SEG_KICK_LDS_BYTES
                                    : SEG_LDS_BYTES;
-    a.cap = (int)(win / (per_node ? per_node : 8)) & ~15;
+    // (a pass that completes its deferred particles keeps their count there too)
+    const size_t room = wide || mode == 2 ? win - SEG_OWN_BYTES : win;
+    a.cap = (int)(room / (per_node ? per_node : 8)) & ~15;
     a.slow = c->slow_chunks;
     PIC_TRY(ensure_defer(c));
     a.dlist = c->defer;
@@ -873,31 +903,28 @@ int launch_seg32(Ctx *c, int kernel, int mode, double dt, double dtd) {
     return rc;
 }
 
-template <class Kern, class Defer>
-static void seg64_launch(const Ctx *c, SegF64 a, Kern k, Defer kd, size_t sm) {
+template <class Kern>
+static void seg64_launch(const Ctx *c, SegF64 a, Kern k, size_t sm) {
+    sm += SEG_OWN_BYTES;
     if (sm > 65536)
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
     a.bps = seg_bps(c, reinterpret_cast<const void *>(k), sm, SEG64_T);
     dim3 grid((unsigned)(((c->nx * c->ny + 63) / 64) * a.bps));
     hipLaunchKernelGGL(k, grid, dim3(SEG64_T), sm, c->stream, a);
-    hipLaunchKernelGGL(kd, dim3(DEFER_BLOCKS), dim3(DEFER_T), 0, c->stream, a);
 }
 
 template <int K, bool G, int ND, bool D, bool P>
 static void seg64_bz(const Ctx *c, const SegF64 &a, int bz, size_t sm) {
     switch (bz) {
         case PIC_BZ_NONE:
-            seg64_launch(c, a, k_seg_f64<K, G, ND, D, PIC_BZ_NONE, P>,
-                         k_defer_f64<K, G, ND, D, PIC_BZ_NONE, P>, sm);
+            seg64_launch(c, a, k_seg_f64<K, G, ND, D, PIC_BZ_NONE, P>, sm);
             break;
         case PIC_BZ_UNIFORM:
-            seg64_launch(c, a, k_seg_f64<K, G, ND, D, PIC_BZ_UNIFORM, P>,
-                         k_defer_f64<K, G, ND, D, PIC_BZ_UNIFORM, P>, sm);
+            seg64_launch(c, a, k_seg_f64<K, G, ND, D, PIC_BZ_UNIFORM, P>, sm);
             break;
         default:
-            seg64_launch(c, a, k_seg_f64<K, G, ND, D, PIC_BZ_GRID, P>,
-                         k_defer_f64<K, G, ND, D, PIC_BZ_GRID, P>, sm);
+            seg64_launch(c, a, k_seg_f64<K, G, ND, D, PIC_BZ_GRID, P>, sm);
     }
 }
 
@@ -941,7 +968,7 @@ int launch_seg64(Ctx *c, int kernel, int mode, double dt, double dtd) {
     const bool gather = mode == 1 || mode == 2;
     const size_t per_node =
         (gather ? (c->bz_mode == PIC_BZ_GRID ? 24 : 16) : 0) + (mode == 2 ? 0 : 16);
-    a.cap = (int)(SEG64_LDS_BYTES / (per_node ? per_node : 8)) & ~15;
+    a.cap = (int)((SEG64_LDS_BYTES - SEG_OWN_BYTES) / (per_node ? per_node : 8)) & ~15;
     a.slow = c->slow_chunks;
     PIC_TRY(ensure_defer(c));
     a.dlist = c->defer;
