@@ -397,6 +397,18 @@ __global__ void k_adj32_seed(int64_t m, const double *ex, const double *ey, doub
     muy[k] = 2.0 * ey[k] * dxdy;
 }
 
+// The FP32 adjoints (x, y, vx, vy) as FP64 pairs: gx = (x, y) and, over lam
+// itself, gv = (vx, vy) + h (x, y).  (Unpacked by the host from a copy of lam,
+// the pairs of 2e6 particles took 2 of 19 ms.)
+__global__ void k_adj32_pairs(int64_t n, double h, float4 *lam, double2 *gx) {
+    int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const float4 L = lam[k];
+    gx[k] = make_double2(L.x, L.y);
+    reinterpret_cast<double2 *>(lam)[k] =
+        make_double2((double)L.z + h * (double)L.x, (double)L.w + h * (double)L.y);
+}
+
 // out[perm[r]] = in[r]: per-slot values into the order the permutation was
 // taken from.
 template <typename T>
@@ -745,20 +757,6 @@ int adjoint32_impl(Ctx *c, double dt, int nsteps, int ckpt, int sort_every, doub
         }
     }
     PIC_HIP(hipGetLastError());
-    std::vector<float4> hl((size_t)n);
-    PIC_HIP(hipMemcpyAsync(hl.data(), lam.p, (size_t)n * 16, hipMemcpyDeviceToHost, c->stream));
-    PIC_HIP(hipStreamSynchronize(c->stream));
-    for (int64_t k = 0; k < n; ++k) {
-        const float4 L = hl[k];
-        if (gx) {
-            gx[2 * k] = L.x;
-            gx[2 * k + 1] = L.y;
-        }
-        if (gv) {
-            gv[2 * k] = (double)L.z + h * (double)L.x;
-            gv[2 * k + 1] = (double)L.w + h * (double)L.y;
-        }
-    }
     // leave the particles as they were at entry: checkpoint 0 carried back
     // through its permutation into the caller's order
     PIC_TRY(restore_from(ckc.p, cko.p, offs.p, 0));
@@ -768,6 +766,15 @@ int adjoint32_impl(Ctx *c, double dt, int nsteps, int ckpt, int sort_every, doub
                        (const uint32_t *)perms.p, (const float4 *)c->ov32, t4.p);
     PIC_TRY(dcopy(c->cell, tc.p, (size_t)n * 4));
     PIC_TRY(dcopy(c->ov32, t4.p, (size_t)n * 16));
+    // the gradients of x_0 and v_0 (before the first half drift) as FP64 pairs,
+    // the latter in lam's own place
+    hipLaunchKernelGGL(k_adj32_pairs, grid_for(n), dim3(AT), 0, c->stream, n, h, lam.p,
+                       reinterpret_cast<double2 *>(t4.p));
+    PIC_HIP(hipGetLastError());
+    if (gx)
+        PIC_HIP(hipMemcpyAsync(gx, t4.p, (size_t)n * 16, hipMemcpyDeviceToHost, c->stream));
+    if (gv)
+        PIC_HIP(hipMemcpyAsync(gv, lam.p, (size_t)n * 16, hipMemcpyDeviceToHost, c->stream));
     PIC_HIP(hipStreamSynchronize(c->stream));
     tm.collect();
     c->seg_valid = false;
