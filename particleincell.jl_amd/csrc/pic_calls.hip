@@ -64,7 +64,7 @@ __global__ void k_interpolate_cic(int64_t n, const double *x, const double *y, i
 using picd::jl_fmod;
 
 // compute_rho_m6!(fields, particles)'s positions into [x0, x0 + dimx), [y0,
-// y0 + dimy) (compute_rho_m6.jl:201-207), for the deposit of pic_deposit.hip.
+// y0 + dimy) (compute_rho_m6.jl:201-207), after the deposit of pic_deposit.hip.
 __global__ void k_mf_wrap(int64_t n, double *x, double *y, double x0, double y0, double dimx,
                           double dimy) {
     int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -276,10 +276,10 @@ int pic_compute_rho_m6_fields(pic_ctx *ctx, int compat) {
     PIC_TRY(need_f64(c));
     const double x0 = compat ? c->xmax : c->xmin, y0 = compat ? c->ymax : c->ymin;
     if (deposit_lds_ok(c)) {
+        PIC_TRY(deposit_rho_mf(c, x0, y0, compat != 0));
         hipLaunchKernelGGL(k_mf_wrap, grid1(c->n), dim3(256), 0, c->stream, c->n, c->x, c->y, x0,
                            y0, c->dimx, c->dimy);
         PIC_HIP(hipGetLastError());
-        PIC_TRY(deposit_rho_mf(c, x0, y0, compat != 0));
         PIC_HIP(hipStreamSynchronize(c->stream));
         return PIC_OK;
     }

@@ -35,17 +35,22 @@ constexpr size_t DEP_LDS = 160 * 1024;
 // How a position gives a cell and an in-cell offset, and where the weights go.
 //   DEP_REF     compute_rho(p, kernel, mesh): pushers_cic.jl:84-105 (trunc for
 //               CIC), pushers_m6.jl:246-338 (floor)
-//   DEP_MF      the MeshFields M6 deposit at x - x0, in [0, dimx]
-//               (compute_rho_m6.jl:70-81)
+//   DEP_MF      the MeshFields M6 deposit at the residue x - x0 mod dimx
+//               (compute_rho_m6.jl:70-81), in [0, dimx]
 //   DEP_COMPAT  the same with the reference's neighbour indices of
 //               compute_rho_m6!(fields, particles) (:216-227), every
 //               off-centre weight one node low
+// The residue is formed here from the position as given, or given itself
+// (UA): a position put back into the domain, residue + x0, has lost the
+// residue's last bits (128 x 64 cells, x0 = xmax: charge 1e-14 off normwise
+// instead of 1e-16).
 enum { DEP_REF, DEP_MF, DEP_COMPAT };
 
 struct DepArgs {
     int64_t n;
     const double *x, *y, *w;  // w null: w0
-    double w0, x0, y0, dx, dy;
+    double w0, x0, y0, dimx, dimy, dx, dy;
+    int residues;             // x, y are residues (DEP_MF)
     int nx, ny;
     double *copies;           // chunk c's grid at c * nx * ny
     int chunks, parts, len;   // len nodes per part
@@ -76,7 +81,8 @@ __global__ __launch_bounds__(DT) void k_deposit_lds(DepArgs a) {
             ci = ref_cell_s(x, a.dx, nx, K == PIC_CIC, fx);
             cj = ref_cell_s(y, a.dy, ny, K == PIC_CIC, fy);
         } else {
-            const double px = (x - a.x0) / a.dx, py = (y - a.y0) / a.dy;
+            const double px = (a.residues ? x : picd::jl_mod_pos(x - a.x0, a.dimx)) / a.dx;
+            const double py = (a.residues ? y : picd::jl_mod_pos(y - a.y0, a.dimy)) / a.dy;
             ci = (int)px;
             cj = (int)py;
             fx = px - (double)ci;
@@ -154,6 +160,14 @@ __global__ __launch_bounds__(64 * W) void k_deposit_reduce(const double *__restr
     }
 }
 
+// Residues back into the domain.
+__global__ void k_residues_back(int64_t n, double *x, double *y, double x0, double y0) {
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    x[k] += x0;
+    y[k] += y0;
+}
+
 constexpr int DEP_PARTS_MAX = 8;
 
 template <int K, int HOW>
@@ -174,7 +188,7 @@ int parts_of(const Ctx *c) {
     return (int)std::min<int64_t>((m + room - 1) / room, DEP_PARTS_MAX + 1);
 }
 
-int deposit(Ctx *c, int kernel, int how, double x0, double y0) {
+int deposit(Ctx *c, int kernel, int how, double x0, double y0, bool residues) {
     const int64_t m = (int64_t)c->nx * c->ny;
     DepArgs a;
     a.n = c->n;
@@ -184,6 +198,9 @@ int deposit(Ctx *c, int kernel, int how, double x0, double y0) {
     a.w0 = c->w0;
     a.x0 = x0;
     a.y0 = y0;
+    a.residues = residues;
+    a.dimx = c->dimx;
+    a.dimy = c->dimy;
     a.dx = c->dx;
     a.dy = c->dy;
     a.nx = c->nx;
@@ -230,10 +247,20 @@ int ensure_copies(Ctx *c, int64_t count) {
 
 bool deposit_lds_ok(const Ctx *c) { return c->n > 0 && parts_of(c) <= DEP_PARTS_MAX; }
 
-int deposit_rho(Ctx *c, int kernel) { return deposit(c, kernel, DEP_REF, 0.0, 0.0); }
+int deposit_rho(Ctx *c, int kernel) { return deposit(c, kernel, DEP_REF, 0.0, 0.0, false); }
 
 int deposit_rho_mf(Ctx *c, double x0, double y0, bool compat) {
-    return deposit(c, PIC_M6, compat ? DEP_COMPAT : DEP_MF, x0, y0);
+    return deposit(c, PIC_M6, compat ? DEP_COMPAT : DEP_MF, x0, y0, false);
+}
+
+int deposit_rho_residues(Ctx *c) {
+    PIC_TRY(deposit(c, PIC_M6, DEP_MF, 0.0, 0.0, true));
+    if (c->n && (c->xmin != 0.0 || c->ymin != 0.0)) {
+        hipLaunchKernelGGL(k_residues_back, dim3((unsigned)((c->n + 255) / 256)), dim3(256), 0,
+                           c->stream, c->n, c->x, c->y, c->xmin, c->ymin);
+        PIC_HIP(hipGetLastError());
+    }
+    return PIC_OK;
 }
 
 }  // namespace pic

@@ -235,10 +235,14 @@ int finalize_rho(Ctx *c, int kernel);
 int shift_rho(Ctx *c, int kernel);
 // compute_rho of the FP64 state's particles, in any order, on grids whose
 // charge fits LDS in a few parts (deposit_lds_ok): rho_acc and rho.
-// deposit_rho_mf: the MeshFields M6 deposit at x - x0, y - y0.
+// deposit_rho_mf: the MeshFields M6 deposit at x - x0 mod dimx, y - y0 mod
+// dimy, the positions left as they are.  deposit_rho_residues: the same with
+// c->x, c->y holding x - xmin mod dimx, y - ymin mod dimy, which are positions
+// again afterwards.
 bool deposit_lds_ok(const Ctx *c);
 int deposit_rho(Ctx *c, int kernel);
 int deposit_rho_mf(Ctx *c, double x0, double y0, bool compat);
+int deposit_rho_residues(Ctx *c);
 int ensure_copies(Ctx *c, int64_t count);
 int field_energy(Ctx *c, double *out2);
 // Queues solve!(fields, poisson): E from rho, and with slot >= 0

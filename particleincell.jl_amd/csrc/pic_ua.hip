@@ -368,9 +368,9 @@ __device__ __forceinline__ void ua_gather(const double xt[2], const UaGrid &g, d
 }
 
 // update_particles_x! for one particle (compute_rho_m6.jl:37-164): x(t) from
-// the spectrum of its tau-samples, into the domain, stored; the M6 deposit
-// (nodes i-2..i+3, wrapped, as in :70-81) spread over the group's lanes where
-// the grid is too large for pic_deposit.hip's.  eplus = exp(+1im l t / eps), the
+// the spectrum of its tau-samples, into the domain, stored (as x - xmin where
+// pic_deposit.hip's deposit follows); else the M6 deposit (nodes i-2..i+3,
+// wrapped, as in :70-81) spread over the group's lanes.  eplus = exp(+1im l t / eps), the
 // conjugate of elt (cos is even and sin odd in the device library, and the two
 // angles differ only in sign).
 template <int NT>
@@ -385,11 +385,12 @@ __device__ __forceinline__ void ua_reconstruct_deposit(const UaLane<NT> &L, cd e
     const double xt1 = picd::jl_mod_pos(pos[0] - g.xmin, g.dimx);
     const double xt2 = picd::jl_mod_pos(pos[1] - g.ymin, g.dimy);
     if (!live) return;
+    const bool follows = !g.rho_acc;  // the deposit, in launches of its own, from the residues
     if (L.m == 0) {
-        *xo = xt1 + g.xmin;
-        *yo = xt2 + g.ymin;
+        *xo = follows ? xt1 : xt1 + g.xmin;
+        *yo = follows ? xt2 : xt2 + g.ymin;
     }
-    if (!g.rho_acc) return;  // the deposit follows in launches of its own
+    if (follows) return;
     const double px = xt1 / g.dx, py = xt2 / g.dy;
     const int i = min(max((int)px, 0), g.nx), j = min(max((int)py, 0), g.ny);
     double wx[6], wy[6];
@@ -941,7 +942,7 @@ int pic_ua_compute_rho(pic_ctx *ctx, const double *t, const double *xt) {
                                             c->stream, a, dxt.p));
         PIC_HIP(hipGetLastError());
     }
-    if (lds) PIC_TRY(deposit_rho_mf(c, c->xmin, c->ymin, false));
+    if (lds) PIC_TRY(deposit_rho_residues(c));
     else PIC_TRY(finalize_rho(c, PIC_M6));
     PIC_HIP(hipStreamSynchronize(c->stream));
     c->seg_valid = false;
@@ -1023,7 +1024,7 @@ int pic_ua_run(pic_ctx *ctx, double dt, int nsteps, double *energy) {
                     c->t_ua_n[half] += 1;
                 }
             }
-            if (lds) PIC_TRY(deposit_rho_mf(c, c->xmin, c->ymin, false));
+            if (lds) PIC_TRY(deposit_rho_residues(c));
             else PIC_TRY(finalize_rho(c, PIC_M6));
             // pic_solve_fields without its wait: E and the energy sums
             PIC_TRY(solve_fields_async(c, energy ? 2 * s + half : -1,
