@@ -205,7 +205,8 @@ int pic_field_energy(pic_ctx *ctx, double out[2]);
  * (:190-191), so the rewritten positions land in [xmax, xmax+dimx), and its
  * neighbour indices mod1(i+k, nx) on the 0-based cell (:216-227), which put
  * every off-centre weight one node low.  compat = 0 uses the unswapped
- * bounds and the neighbours of compute_rho(p, M6(), mesh). */
+ * bounds and the neighbours of compute_rho(p, M6(), mesh).  Every particle
+ * carries the first one's weight (Particles.w is one number). */
 int pic_compute_rho_m6_fields(pic_ctx *ctx, int compat);
 
 /* interpol_eb_m6!(particles, fields): interpolation_m6.jl:125-247, EX/EY ->

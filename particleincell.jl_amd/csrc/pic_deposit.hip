@@ -194,7 +194,9 @@ int deposit(Ctx *c, int kernel, int how, double x0, double y0, bool residues) {
     a.n = c->n;
     a.x = c->x;
     a.y = c->y;
-    a.w = c->uniform_w ? nullptr : c->w;
+    // the MeshFields deposits give every particle w0, as Particles.w is one
+    // number (particles.jl:12-35), whatever the grid and so the kernel
+    a.w = c->uniform_w || how != DEP_REF ? nullptr : c->w;
     a.w0 = c->w0;
     a.x0 = x0;
     a.y0 = y0;

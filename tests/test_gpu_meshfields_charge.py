@@ -93,3 +93,28 @@ def test_ua_charge_at_the_reconstructed_offsets(gpu):
     assert np.array_equal(p.x, moved)
     err = np.linalg.norm((f.rho[:nx, :ny] - want).astype(np.float64))
     assert err <= _bound(n, mesh) * np.linalg.norm(raw.astype(np.float64))
+
+
+@pytest.mark.parametrize("nx,ny", [(32, 16), (400, 400), (512, 512)])  # one part, eight, past them
+def test_one_weight_on_every_grid(gpu, nx, ny):
+    """Particles.w is one number: on a context whose particles' weights differ,
+    compute_rho_m6!(fields, particles) gives all of them the first one's, on
+    grids of either deposit kernel alike: 1e-12 of the charge of particles of
+    that weight, the bar of the FP64 charge sums in another order."""
+    pic = gpu
+    L = pic._lib
+    rng = np.random.default_rng(nx)
+    n = 3_001
+    mesh = pic.TwoDGrid(0.0, DIMX, nx, 0.0, DIMY, ny)
+    p = np.zeros((5, n), order="F")
+    p[0], p[1] = rng.uniform(0, DIMX, n), rng.uniform(0, DIMY, n)
+    p[4] = rng.uniform(0.5, 1.5, n)
+    rho = []
+    for w in (p[4], p[4, 0]):
+        q = p.copy(order="F")
+        q[4] = w
+        sim = pic.Simulation(mesh, q, pic.M6())
+        L.call("pic_compute_rho_m6_fields", sim.ctx.h, 0)
+        rho.append(sim.grid(L.PIC_GRID_RHO))
+        sim.close()
+    assert np.linalg.norm(rho[0] - rho[1]) <= 1e-12 * np.linalg.norm(rho[1])
