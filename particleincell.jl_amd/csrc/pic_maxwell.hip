@@ -1312,7 +1312,7 @@ int pic_run_maxwell(pic_ctx *ctx, int kernel, double dt, int nsteps, double *ene
     };
     int rc = PIC_OK;
     const size_t flds = vm_field_lds(c), plds = vm_pass_lds(c), slds = vm_step_lds(c);
-    const bool one = slds <= VM_STEP_LDS_MAX && flds <= VM_STEP_LDS_MAX && c->vm_path != 2;
+    const bool one = slds <= VM_STEP_LDS_MAX && flds <= VM_STEP_LDS_MAX && c->vm_path == 0;
     const bool fused = !one && flds <= VM_LDS_BYTES_MAX && plds <= VM_LDS_BYTES_MAX &&
                        c->vm_path != 3;
     const VmPartPlan pp = vm_part_plan(c);

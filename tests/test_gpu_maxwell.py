@@ -194,7 +194,8 @@ def test_run_maxwell_first_step_bit_exact(gpu, O):
 @pytest.mark.parametrize("nx,ny,npm,steps,midpoint,path", [
     (128, 16, 100, 100, False, 0), (128, 16, 100, 100, False, 2), (128, 16, 100, 100, False, 3),
     (32, 8, 50, 200, True, 0), (32, 8, 50, 3, True, 0), (32, 8, 50, 200, True, 2),
-    (64, 40, 20, 40, True, 0), (96, 40, 20, 40, True, 0), (128, 64, 10, 40, True, 0)])
+    (64, 40, 20, 40, True, 0), (96, 40, 20, 40, True, 0), (128, 64, 10, 40, True, 0),
+    (96, 40, 20, 40, True, 3), (128, 64, 10, 40, True, 3)])
 def test_run_maxwell_matches_oracle_loop(gpu, O, nx, ny, npm, steps, midpoint, path):
     """pic_run_maxwell against the oracle's loop: the README's 204,800
     particles on 128 x 16 cells for 100 steps (the loop of
@@ -203,7 +204,7 @@ def test_run_maxwell_matches_oracle_loop(gpu, O, nx, ny, npm, steps, midpoint, p
     kernel, 3: one kernel per reference function), a small grid for 200
     and for 3 steps (every current buffer of the one-launch form last), a
     64 x 40 grid (two launches: the one-launch LDS does not fit), 96 x 40 and
-    128 x 64 (one kernel per function).  The current's reordered sums are
+    128 x 64 (three launches, and one kernel per function).  The current's reordered sums are
     the only difference, so energies and particles agree to 1e-10
     relative."""
     pic = gpu
@@ -337,3 +338,27 @@ def test_three_launch_iteration_matches_one_kernel_per_function(gpu, nx, ny, n, 
         sim.close()
     for a, b in zip(*got):
         assert np.max(np.abs(a - b)) <= 1e-12 * max(1.0, np.max(np.abs(b)))
+
+
+@pytest.mark.parametrize("nx,ny", [(32, 8), (128, 16), (96, 40)])
+def test_path_3_is_one_kernel_per_function(gpu, nx, ny):
+    """Path 3 takes the energy with compute_energy's own kernel, also on grids
+    that the fused forms serve by default (their sums run in other orders): bit
+    for bit pic_fdtd_energy of the fields it leaves, ten times."""
+    pic = gpu
+    L = pic._lib
+    rng = np.random.default_rng(nx)
+    mesh = pic.TwoDGrid(0.0, 3.0, nx, 0.0, 2.0, ny)
+    n = 5_000
+    f = pic.FDTD(mesh)
+    for a in (f.ex, f.ey, f.bz):
+        a[...] = 0.1 * rng.normal(size=a.shape)
+    sim = pic.Simulation(mesh, random_particles(rng, n, mesh.dimx, mesh.dimy), pic.CloudInCell())
+    sim.set_maxwell_path(3)
+    sim.set_fdtd(f)
+    e = L.C.c_double()
+    for _ in range(10):
+        got = sim.run_maxwell(0.01, 1)[0]
+        L.call("pic_fdtd_energy", sim.ctx.h, L.C.byref(e))
+        assert got == e.value
+    sim.close()
