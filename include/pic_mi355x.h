@@ -108,7 +108,8 @@ int pic_set_particles(pic_ctx *ctx, const double *p, int64_t n);
 /* Copies the context's particles back into p.array (5 x n).  In FP32 state
  * the positions are rebuilt as (cell + offset) * dx. */
 int pic_get_particles(pic_ctx *ctx, double *p);
-/* The same for a 5 x n particle array already in device memory. */
+/* The same for a 5 x n particle array already in device memory, which has been
+ * read when the call returns. */
 int pic_set_particles_device(pic_ctx *ctx, const double *d_p, int64_t n);
 int pic_get_particles_device(pic_ctx *ctx, double *d_p);
 int pic_num_particles(pic_ctx *ctx, int64_t *n);

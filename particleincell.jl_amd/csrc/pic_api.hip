@@ -310,6 +310,9 @@ static int set_particles_impl(Ctx *c, const double *d_p, int64_t n) {
         PIC_TRY(dalloc(&c->w, c->cap));
         hipLaunchKernelGGL(k_weights, grid1(n), dim3(256), 0, c->stream, d_p, n, c->w);
         PIC_HIP(hipGetLastError());
+        // d_p is the caller's: read to its end before the call returns, with
+        // one weight (above) and with several
+        PIC_HIP(hipStreamSynchronize(c->stream));
     }
     return PIC_OK;
 }

@@ -1,6 +1,8 @@
 """Particles and grids between host and device: the weights' verdict wherever a
 weight differs, transfers below and above the size of the kept staging buffer,
 and grids of every layout on both sides of the pinned copy's size."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -96,3 +98,36 @@ def test_fields_set_reach_the_fp32_pass(gpu, nx, ny, order):
         ctx.close()
     assert np.abs(v[0] - p[2:4]).max() > 1e-4
     assert np.abs(v[0] - v[1]).max() <= 64 * 2.0**-24 * 4e-3
+
+
+def _hip():
+    """The HIP runtime the library has loaded."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64.so" in line)
+    return C.CDLL(path)
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+def test_device_particles_are_read_on_return(gpu, weighted):
+    """pic_set_particles_device has read the caller's array when it returns,
+    with one weight and with several: overwritten at once on another stream,
+    the particles are still the ones given."""
+    pic = gpu
+    n = 4_000_000
+    rng = np.random.default_rng(1)
+    p = np.asfortranarray(rng.uniform(0.05, 0.95, (5, n)))
+    if not weighted:
+        p[4] = 0.25
+    ctx = _context(pic, 16, 16)
+    hip = _hip()
+    d, s = C.c_void_p(), C.c_void_p()
+    assert hip.hipMalloc(C.byref(d), C.c_size_t(p.nbytes)) == 0
+    assert hip.hipStreamCreateWithFlags(C.byref(s), 1) == 0  # non-blocking
+    assert hip.hipMemcpy(d, C.c_void_p(p.ctypes.data), C.c_size_t(p.nbytes), 1) == 0
+    pic._lib.call("pic_set_particles_device", ctx.h, d, n)
+    assert hip.hipMemsetAsync(d, 0, C.c_size_t(p.nbytes), s) == 0
+    assert hip.hipStreamSynchronize(s) == 0
+    got = ctx.get_particles(np.zeros((5, n), order="F"))
+    assert hip.hipFree(d) == 0 and hip.hipStreamDestroy(s) == 0
+    np.testing.assert_array_equal(got, p)
+    ctx.close()
