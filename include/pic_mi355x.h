@@ -434,7 +434,8 @@ int pic_fdtd_energy(pic_ctx *ctx, double *energy);
  * be NULL).  One launch per iteration when 8 (nx(ny+1) + (nx+1)ny + 6 nx ny)
  * bytes fit in 150 KiB of LDS (132 KiB at 128 x 16), else two up to 3072
  * cells, else three up to 81,920 (the current summed in LDS in up to eight
- * parts; a second set of particle arrays with more than one), else one
+ * parts; a second set of particle arrays with more than one, where the
+ * device has room for it), else one
  * kernel per reference function.  kernel must be PIC_CIC; FP64 state. */
 int pic_run_maxwell(pic_ctx *ctx, int kernel, double dt, int nsteps, double *energy);
 

@@ -54,11 +54,7 @@ static void free_particles(Ctx *c) {
     dfree(c->swap);
     dfree(c->defer);
     c->swap_bytes = 0;
-    for (int k = 0; k < Ctx::NALT; ++k) {
-        if (c->alt[k]) (void)hipFree(c->alt[k]);
-        c->alt[k] = nullptr;
-        c->alt_of[k] = nullptr;
-    }
+    drop_alt(c);
     for (int k = 0; k < 2; ++k) { dfree(c->sort_keys[k]); dfree(c->sort_vals[k]); }
     // the histograms and their scan block sums are sized by the particle
     // capacity too: both are reallocated together by the next ensure_sort

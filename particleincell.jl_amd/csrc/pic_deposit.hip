@@ -188,6 +188,13 @@ int parts_of(const Ctx *c) {
     return (int)std::min<int64_t>((m + room - 1) / room, DEP_PARTS_MAX + 1);
 }
 
+// One block per compute unit, at least a particle per thread.
+int chunks_of(const Ctx *c, int parts) {
+    return (int)std::max<int64_t>(1, std::min<int64_t>((c->n + DT - 1) / DT, c->ncu / parts));
+}
+
+int reduce_blocks(int64_t m) { return (int)((m + 63) / 64); }
+
 int deposit(Ctx *c, int kernel, int how, double x0, double y0, bool residues) {
     const int64_t m = (int64_t)c->nx * c->ny;
     DepArgs a;
@@ -209,10 +216,8 @@ int deposit(Ctx *c, int kernel, int how, double x0, double y0, bool residues) {
     a.ny = c->ny;
     a.parts = parts_of(c);
     a.len = (int)((m + a.parts - 1) / a.parts);
-    // one block per compute unit, at least a particle per thread
-    a.chunks = (int)std::max<int64_t>(1, std::min<int64_t>((c->n + DT - 1) / DT, c->ncu / a.parts));
-    const int nblk = (int)((m + 63) / 64);
-    PIC_TRY(ensure_copies(c, (int64_t)a.chunks * m + nblk));
+    a.chunks = chunks_of(c, a.parts);
+    const int nblk = reduce_blocks(m);
     a.copies = c->copies;
     int rc = PIC_OK;
     if (how == DEP_REF) {
@@ -247,7 +252,14 @@ int ensure_copies(Ctx *c, int64_t count) {
     return PIC_OK;
 }
 
-bool deposit_lds_ok(const Ctx *c) { return c->n > 0 && parts_of(c) <= DEP_PARTS_MAX; }
+bool deposit_lds_ok(Ctx *c) {
+    const int parts = parts_of(c);
+    if (c->n == 0 || parts > DEP_PARTS_MAX) return false;
+    const int64_t m = (int64_t)c->nx * c->ny;
+    if (ensure_copies(c, chunks_of(c, parts) * m + reduce_blocks(m)) == PIC_OK) return true;
+    (void)hipGetLastError();  // no room for the copies: the kernels without them
+    return false;
+}
 
 int deposit_rho(Ctx *c, int kernel) { return deposit(c, kernel, DEP_REF, 0.0, 0.0, false); }
 

@@ -234,12 +234,12 @@ int finalize_rho(Ctx *c, int kernel);
 // left in red_part[2 RED_BLOCKS].
 int shift_rho(Ctx *c, int kernel);
 // compute_rho of the FP64 state's particles, in any order, on grids whose
-// charge fits LDS in a few parts (deposit_lds_ok): rho_acc and rho.
+// charge fits LDS in a few parts: rho_acc and rho, after deposit_lds_ok.
 // deposit_rho_mf: the MeshFields M6 deposit at x - x0 mod dimx, y - y0 mod
 // dimy, the positions left as they are.  deposit_rho_residues: the same with
 // c->x, c->y holding x - xmin mod dimx, y - ymin mod dimy, which are positions
 // again afterwards.
-bool deposit_lds_ok(const Ctx *c);
+bool deposit_lds_ok(Ctx *c);
 int deposit_rho(Ctx *c, int kernel);
 int deposit_rho_mf(Ctx *c, double x0, double y0, bool compat);
 int deposit_rho_residues(Ctx *c);
@@ -263,6 +263,9 @@ int settle_state(Ctx *c);
 int alt_f32(Ctx *c, int32_t **cell, float4 **ov);
 void swap_alt_f32(Ctx *c);
 int alt_f64(Ctx *c, double **x, double **y, double **vx, double **vy, double **w);
+// Frees the alternate arrays (none holding anything still wanted: no
+// permutation pending).
+void drop_alt(Ctx *c);
 // Without `weights` the weights stay in the current array (a pass that keeps
 // the particles in their slots).
 void swap_alt_f64(Ctx *c, bool weights = true);

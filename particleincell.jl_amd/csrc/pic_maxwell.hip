@@ -945,12 +945,11 @@ int ensure_fdtd(Ctx *c) {
 
 int ensure_step_buffers(Ctx *c) {
     const size_t nx = c->nx, ny = c->ny;
-    if (!c->fd2_ex) {
-        PIC_HIP(hipMalloc(&c->fd2_ex, nx * (ny + 1) * 8));
-        PIC_HIP(hipMalloc(&c->fd2_ey, (nx + 1) * ny * 8));
-        PIC_HIP(hipMalloc(&c->fd2_bz, nx * ny * 8));
-        for (double *&p : c->jb) PIC_HIP(hipMalloc(&p, nx * ny * 8));
-    }
+    if (!c->fd2_ex) PIC_HIP(hipMalloc(&c->fd2_ex, nx * (ny + 1) * 8));
+    if (!c->fd2_ey) PIC_HIP(hipMalloc(&c->fd2_ey, (nx + 1) * ny * 8));
+    if (!c->fd2_bz) PIC_HIP(hipMalloc(&c->fd2_bz, nx * ny * 8));
+    for (double *&p : c->jb)
+        if (!p) PIC_HIP(hipMalloc(&p, nx * ny * 8));
     return PIC_OK;
 }
 
@@ -1115,8 +1114,22 @@ VmPartPlan vm_part_plan(const Ctx *c) {
 
 int ensure_part_buffers(Ctx *c, const VmPartPlan &p) {
     const size_t m = (size_t)c->nx * c->ny;
+    PIC_TRY(ensure_step_buffers(c));
     if (!c->vm_nodes) PIC_HIP(hipMalloc(&c->vm_nodes, m * sizeof(VmNode)));
-    return ensure_copies(c, (int64_t)p.chunks * 2 * (int64_t)m);
+    PIC_TRY(ensure_copies(c, (int64_t)p.chunks * 2 * (int64_t)m));
+    if (p.parts == 1) return PIC_OK;
+    double *a[4];
+    return alt_f64(c, &a[0], &a[1], &a[2], &a[3], nullptr);
+}
+
+// Whether the three-launch iteration has its buffers.  The second set of
+// particle arrays may be as large as the first, and no other form needs one:
+// where they do not fit, the loop runs without them.
+bool part_buffers(Ctx *c, const VmPartPlan &p) {
+    if (ensure_part_buffers(c, p) == PIC_OK) return true;
+    (void)hipGetLastError();
+    drop_alt(c);
+    return false;
 }
 
 int vm_pass_part(Ctx *c, double dt, const VmPartPlan &p) {
@@ -1316,7 +1329,8 @@ int pic_run_maxwell(pic_ctx *ctx, int kernel, double dt, int nsteps, double *ene
     const bool fused = !one && flds <= VM_LDS_BYTES_MAX && plds <= VM_LDS_BYTES_MAX &&
                        c->vm_path != 3;
     const VmPartPlan pp = vm_part_plan(c);
-    const bool parted = !one && !fused && c->vm_path != 3 && pp.ok && c->n > 0;
+    const bool parted =
+        !one && !fused && c->vm_path != 3 && pp.ok && c->n > 0 && part_buffers(c, pp);
     auto timed_pass = [&](bool lds) {
         int r = c->timing ? mark() : PIC_OK;
         if (r == PIC_OK) r = lds ? vm_pass_lds_launch(c, dt) : vm_pass(c, dt);
@@ -1393,8 +1407,6 @@ int pic_run_maxwell(pic_ctx *ctx, int kernel, double dt, int nsteps, double *ene
     if (parted) {
         // fdtd.ex, fdtd.ey alternate between the context's arrays and the
         // second set; bz goes through the second set within an iteration
-        rc = ensure_step_buffers(c);
-        if (rc == PIC_OK) rc = ensure_part_buffers(c, pp);
         double *ex[2] = {c->fd_ex, c->fd2_ex}, *ey[2] = {c->fd_ey, c->fd2_ey};
         VmNode *nodes = static_cast<VmNode *>(c->vm_nodes);
         if (rc == PIC_OK) rc = update_fields(c, nodes);

@@ -558,6 +558,14 @@ int alt_f64(Ctx *c, double **x, double **y, double **vx, double **vy, double **w
     return PIC_OK;
 }
 
+void drop_alt(Ctx *c) {
+    for (int k = 0; k < Ctx::NALT; ++k) {
+        if (c->alt[k]) (void)hipFree(c->alt[k]);
+        c->alt[k] = nullptr;
+        c->alt_of[k] = nullptr;
+    }
+}
+
 void swap_alt_f64(Ctx *c, bool weights) {
     int s[5] = {0, 0, 0, 0, 0};
     (void)alt_slot(c, c->x, &s[0]);
