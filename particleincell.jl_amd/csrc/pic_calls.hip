@@ -191,7 +191,7 @@ int pic_compute_rho(pic_ctx *ctx, int kernel) {
     PIC_CHECK(valid_shape(kernel), PIC_ERR_ARG, "kernel %d", kernel);
     Ctx *c = ctx_of(ctx);
     PIC_HIP(hipSetDevice(c->device));
-    if (c->state == PIC_STATE_F64 && !c->near_order && deposit_lds_ok(c)) {
+    if (c->state == PIC_STATE_F64 && !c->near_order && deposit_lds_pays(c, kernel)) {
         PIC_TRY(deposit_rho(c, kernel));
         PIC_HIP(hipStreamSynchronize(c->stream));
         return PIC_OK;

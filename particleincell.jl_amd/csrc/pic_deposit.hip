@@ -2,16 +2,15 @@
 // whole grid's charge in LDS.
 //
 // Particles that are not sorted by cell put their charge anywhere, and one
-// FP64 global atomic per stencil node is what that costs.  Measured on MI355X,
-// scattered FP64 global atomics retire at 24e9/s while their targets span
-// 128 KiB, and at 1.3e9/s and 0.3e9/s over 320 KiB and 1 MiB; 204,800 M6
-// particles on 128 x 64 cells took 324 us.  Here block (chunk, r) takes a chunk
-// of the particles and sums the nodes of part r of the grid in LDS (one part
-// up to 20,480 nodes, at most DEP_PARTS_MAX), then stores its copy of that
-// part without atomics; k_deposit_reduce adds the copies in chunk order, and
-// sums the grid for the neutralising shift on the way.  Measured: those 204,800 particles 13
-// us, and 9 for the reduction; 10,000,000 unsorted M6 particles on 128 x 128
-// cells 0.29 ms for the whole call, on 256 x 256 (four parts) 0.71 ms.
+// FP64 global atomic per stencil node is what that costs: measured on MI355X 20
+// to 23e9/s (1,000,000 particles on 128 x 128 to 400 x 400 nodes, CIC and M6),
+// 1.6 ms for 1,000,000 M6 particles.  Here block (chunk, r) takes a chunk of the
+// particles and sums the nodes of part r of the grid in LDS (one part up to
+// 20,480 nodes, at most DEP_PARTS_MAX), then stores its copy of that part
+// without atomics; k_deposit_reduce adds the copies in chunk order, and sums the
+// grid for the neutralising shift on the way.  Measured, the whole call:
+// 1,000,000 unsorted M6 particles on 100 x 100 nodes 59 us, on 256 x 256 (four
+// parts) 99, on 400 x 400 (eight) 167.
 //
 // With R parts every chunk is read and its weights formed R times, so past
 // DEP_PARTS_MAX parts the chunk kernels of pic_step.hip serve; and for particles
@@ -115,47 +114,64 @@ __global__ __launch_bounds__(DT) void k_deposit_lds(DepArgs a) {
     for (int t = tid; t < len; t += DT) out[t] = lds[t];
 }
 
-// acc[t] = the copies' sum, 64 nodes per block, W waves each taking every W-th
-// chunk, the waves' sums added in order; *total = the sum of acc (a wave
-// butterfly, then the blocks in a fixed order by the last one to arrive).
+// acc[t] = the copies' sum, W waves to 64 nodes, each taking every W-th chunk,
+// the waves' sums added in order; *total = the sum of acc (each wave's nodes in
+// order, a wave butterfly, then the waves and the blocks in a fixed order by the
+// last block to arrive).  At most RD_BLOCKS blocks, which walk the grid: every
+// block pays for its arrival, a fence and an atomic on one counter (measured on
+// MI355X, 400 x 400 nodes: 73 us with a block per 64 nodes, whatever the number
+// of copies).
+constexpr int RD_T = 512, RD_BLOCKS = 256;
 template <int W>
-__global__ __launch_bounds__(64 * W) void k_deposit_reduce(const double *__restrict__ copies,
-                                                           int chunks, int m,
-                                                           double *__restrict__ acc, double *part,
-                                                           unsigned *count, double *total) {
-    __shared__ double sh[64 * W];
+__global__ __launch_bounds__(RD_T) void k_deposit_reduce(const double *__restrict__ copies,
+                                                         int chunks, int m,
+                                                         double *__restrict__ acc, double *part,
+                                                         unsigned *count, double *total) {
+    constexpr int G = RD_T / 64 / W;  // groups of 64 nodes a block works at once
+    __shared__ double sh[RD_T];
     __shared__ bool last;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int t = blockIdx.x * 64 + lane;
-    double s = 0.0;
-    if (t < m) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, q = wv % W;
+    double sum = 0.0;
+    for (int g0 = blockIdx.x * G; g0 * 64 < m; g0 += gridDim.x * G) {
+        const int t = (g0 + wv / W) * 64 + lane;
+        double s = 0.0;
+        if (t < m) {
 #pragma unroll 8
-        for (int b = wv; b < chunks; b += W) s += copies[(size_t)b * m + t];
-    }
-    sh[tid] = s;
-    __syncthreads();
-    if (wv == 0) {
-        for (int k = 1; k < W; ++k) s += sh[64 * k + lane];
-        if (t < m) acc[t] = s;
-        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-        if (lane == 0) {
-            part[blockIdx.x] = s;
-            __threadfence();
-            last = atomicAdd(count, 1u) == gridDim.x - 1;
+            for (int b = q; b < chunks; b += W) s += copies[(size_t)b * m + t];
         }
+        if (W > 1) {
+            sh[tid] = s;
+            __syncthreads();
+            if (q == 0)
+                for (int k = 1; k < W; ++k) s += sh[tid + 64 * k];
+            __syncthreads();
+        }
+        if (q == 0 && t < m) {
+            acc[t] = s;
+            sum += s;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    if (lane == 0) sh[wv] = sum;
+    __syncthreads();
+    if (tid == 0) {
+        for (int k = W; k < RD_T / 64; k += W) sum += sh[k];
+        part[blockIdx.x] = sum;
+        __threadfence();
+        last = atomicAdd(count, 1u) == gridDim.x - 1;
     }
     __syncthreads();
     if (!last) return;
     __threadfence();
-    s = 0.0;
-    for (int k = tid; k < (int)gridDim.x; k += 64 * W)
-        s += __hip_atomic_load(&part[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if (lane == 0) sh[wv] = s;
+    sum = 0.0;
+    for (int k = tid; k < (int)gridDim.x; k += RD_T)
+        sum += __hip_atomic_load(&part[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    if (lane == 0) sh[wv] = sum;
     __syncthreads();
     if (tid == 0) {
-        for (int k = 1; k < W; ++k) s += sh[k];
-        *total = s;
+        for (int k = 1; k < RD_T / 64; ++k) sum += sh[k];
+        *total = sum;
         *count = 0u;
     }
 }
@@ -188,12 +204,14 @@ int parts_of(const Ctx *c) {
     return (int)std::min<int64_t>((m + room - 1) / room, DEP_PARTS_MAX + 1);
 }
 
-// One block per compute unit, at least a particle per thread.
+// One block per compute unit, and enough particles per thread that few of
+// them do not pay for many copies of a large grid: measured on MI355X, 30,000
+// particles on 400 x 400 nodes (eight parts), CIC and M6, 49.4 and 52.5 us with
+// one per thread, 40.4 and 50.7 with four.
 int chunks_of(const Ctx *c, int parts) {
-    return (int)std::max<int64_t>(1, std::min<int64_t>((c->n + DT - 1) / DT, c->ncu / parts));
+    const int64_t per = DT * std::max(1, parts / 2);
+    return (int)std::max<int64_t>(1, std::min<int64_t>((c->n + per - 1) / per, c->ncu / parts));
 }
-
-int reduce_blocks(int64_t m) { return (int)((m + 63) / 64); }
 
 int deposit(Ctx *c, int kernel, int how, double x0, double y0, bool residues) {
     const int64_t m = (int64_t)c->nx * c->ny;
@@ -217,7 +235,6 @@ int deposit(Ctx *c, int kernel, int how, double x0, double y0, bool residues) {
     a.parts = parts_of(c);
     a.len = (int)((m + a.parts - 1) / a.parts);
     a.chunks = chunks_of(c, a.parts);
-    const int nblk = reduce_blocks(m);
     a.copies = c->copies;
     int rc = PIC_OK;
     if (how == DEP_REF) {
@@ -230,12 +247,21 @@ int deposit(Ctx *c, int kernel, int how, double x0, double y0, bool residues) {
     PIC_TRY(rc);
     double *part = c->copies + (size_t)a.chunks * m, *total = c->red_part + 2 * RED_BLOCKS;
     auto reduce = [&](auto kern, int w) {
-        hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(64 * w), 0, c->stream,
+        const int64_t per = RD_T / w;  // nodes a block takes at once
+        const int64_t blocks = std::min<int64_t>((m + per - 1) / per, RD_BLOCKS);
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(RD_T), 0, c->stream,
                            (const double *)c->copies, a.chunks, (int)m, c->rho_acc, part,
                            c->red_count, total);
     };
-    if (a.chunks > 32) reduce(k_deposit_reduce<8>, 8);
-    else reduce(k_deposit_reduce<1>, 1);
+    // More waves to a node read more copies at once but need more blocks.
+    // Measured on MI355X, the whole call with CIC, us at 1 / 2 / 8 waves: 64 x 64
+    // nodes and 59 copies 25.9 / 25.0 / 24.5, 143 x 143 and 16 copies 27.4 / 27.1 /
+    // 31.0, 256 x 256 and 64 39.3 / 42.1 / 46.6; 100 x 100 and 256 copies 44.9 /
+    // 38.2 / 34.9, 143 x 143 and 256 49.3 / 43.5 / 47.9, 200 x 200 and 128 42.9 /
+    // 43.2 / 47.0.
+    if (a.chunks <= 64) reduce(k_deposit_reduce<1>, 1);
+    else if (m > 10240) reduce(k_deposit_reduce<2>, 2);
+    else reduce(k_deposit_reduce<8>, 8);
     PIC_HIP(hipGetLastError());
     return shift_rho(c, kernel);
 }
@@ -256,9 +282,20 @@ bool deposit_lds_ok(Ctx *c) {
     const int parts = parts_of(c);
     if (c->n == 0 || parts > DEP_PARTS_MAX) return false;
     const int64_t m = (int64_t)c->nx * c->ny;
-    if (ensure_copies(c, chunks_of(c, parts) * m + reduce_blocks(m)) == PIC_OK) return true;
+    if (ensure_copies(c, chunks_of(c, parts) * m + RD_BLOCKS) == PIC_OK) return true;
     (void)hipGetLastError();  // no room for the copies: the kernels without them
     return false;
+}
+
+// Against the chunk kernels on unsorted particles, measured on MI355X (the whole
+// call): equal or faster from 300 particles on with M6, TSC and M4 and with CIC
+// on up to six parts (30,000 on 300 x 300 nodes 35.0 against 37.7 us); on seven
+// and eight, CIC's four shares a particle pay for the copies from about five
+// particles to eight nodes on (400 x 400: 20,000 39.2 against 39.0, 50,000 44.2
+// against 40.0, 100,000 46.9 against 48.1, 300,000 50.9 against 86.0).
+bool deposit_lds_pays(Ctx *c, int kernel) {
+    if (kernel == PIC_CIC && parts_of(c) > 6 && 8 * c->n < 5 * (int64_t)c->nx * c->ny) return false;
+    return deposit_lds_ok(c);
 }
 
 int deposit_rho(Ctx *c, int kernel) { return deposit(c, kernel, DEP_REF, 0.0, 0.0, false); }

@@ -234,12 +234,14 @@ int finalize_rho(Ctx *c, int kernel);
 // left in red_part[2 RED_BLOCKS].
 int shift_rho(Ctx *c, int kernel);
 // compute_rho of the FP64 state's particles, in any order, on grids whose
-// charge fits LDS in a few parts: rho_acc and rho, after deposit_lds_ok.
+// charge fits LDS in a few parts: rho_acc and rho, after deposit_lds_ok (or
+// deposit_lds_pays, which also asks whether the chunk kernels are slower).
 // deposit_rho_mf: the MeshFields M6 deposit at x - x0 mod dimx, y - y0 mod
 // dimy, the positions left as they are.  deposit_rho_residues: the same with
 // c->x, c->y holding x - xmin mod dimx, y - ymin mod dimy, which are positions
 // again afterwards.
 bool deposit_lds_ok(Ctx *c);
+bool deposit_lds_pays(Ctx *c, int kernel);
 int deposit_rho(Ctx *c, int kernel);
 int deposit_rho_mf(Ctx *c, double x0, double y0, bool compat);
 int deposit_rho_residues(Ctx *c);
