@@ -624,9 +624,7 @@ static int adjoint_impl(Ctx *c, double dt, int nsteps, int ckpt, int sort_every,
             PIC_HIP(hipMemcpyAsync(out, ck.p + (size_t)2 * n * q, (size_t)2 * n * 8,
                                    hipMemcpyDeviceToHost, c->stream));
     PIC_HIP(hipStreamSynchronize(c->stream));
-    c->seg_valid = false;
-    c->near_order = false;
-    c->sort_fresh = false;
+    new_particles(c);
     return PIC_OK;
 }
 

@@ -777,9 +777,7 @@ int adjoint32_impl(Ctx *c, double dt, int nsteps, int ckpt, int sort_every, doub
         PIC_HIP(hipMemcpyAsync(gv, lam.p, (size_t)n * 16, hipMemcpyDeviceToHost, c->stream));
     PIC_HIP(hipStreamSynchronize(c->stream));
     tm.collect();
-    c->seg_valid = false;
-    c->near_order = false;
-    c->sort_fresh = false;
+    new_particles(c);
     return PIC_OK;
 }
 

@@ -140,8 +140,23 @@ int launch_fill(Ctx *c, double *p, double v, int64_t n) {
 // On the way out->differ, in pinned host memory, is set if a weight is not the
 // first one's (by the first wave that finds one: *flag, zero before), and
 // out->w0 to that weight.
-__global__ void k_aos_to_soa(const double *__restrict__ p, int64_t n, double *x, double *y,
-                             double *vx, double *vy, unsigned *flag, Ctx::Weights *out) {
+// Block 4 ch of the 256-particle blocks also judges chunk ch's order, where that
+// is one of the samples (spread over the nch chunks).
+__global__ __launch_bounds__(256) void k_aos_to_soa(const double *__restrict__ p, int64_t n,
+                                                    double *x, double *y, double *vx, double *vy,
+                                                    unsigned *flag, Ctx::Weights *out, int nx,
+                                                    int ny, double dx, double dy, int nch) {
+    static_assert(STEP_CHUNK == 4 * 256, "four blocks to a chunk");
+    if ((blockIdx.x & 3) == 0) {
+        const int ch = blockIdx.x >> 2, smp = min(nch, ORDER_SAMPLES);
+        const int s = (int)(((int64_t)ch * smp + nch - 1) / nch);
+        if (s < smp && (int64_t)s * nch / smp == ch)
+            picd::order_sample(&out->order, s, (int64_t)ch * STEP_CHUNK, n, nx, ny, dx, dy,
+                               [&](int64_t q, double &a, double &b) {
+                                   a = p[5 * q];
+                                   b = p[5 * q + 1];
+                               });
+    }
     int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     const double *q = p + 5 * k;
@@ -277,28 +292,34 @@ static int clear_flag(Ctx *c) {
     return PIC_OK;
 }
 
+int ensure_w_host(Ctx *c) {
+    if (!c->w_host) PIC_HIP(hipHostMalloc(&c->w_host, sizeof(Ctx::Weights), hipHostMallocDefault));
+    return PIC_OK;
+}
+
 static int set_particles_impl(Ctx *c, const double *d_p, int64_t n) {
     PIC_TRY(ensure_particles(c, n));
     c->n = n;
     c->state = PIC_STATE_F64;
-    c->seg_valid = false;
-    c->near_order = false;
-    c->sort_fresh = false;
+    new_particles(c);
     if (n == 0) {
         c->uniform_w = true;
         c->w0 = 0.0;
         return PIC_OK;
     }
-    if (!c->w_host) PIC_HIP(hipHostMalloc(&c->w_host, sizeof(Ctx::Weights), hipHostMallocDefault));
+    PIC_TRY(ensure_w_host(c));
     if (!c->w_flag) {
         PIC_TRY(dalloc(&c->w_flag, 1));
         PIC_TRY(clear_flag(c));
     }
     c->w_host->differ = 0;
     hipLaunchKernelGGL(k_aos_to_soa, grid1(n), dim3(256), 0, c->stream, d_p, n, c->x, c->y,
-                       c->vx, c->vy, c->w_flag, c->w_host);
+                       c->vx, c->vy, c->w_flag, c->w_host, c->nx, c->ny, c->dx, c->dy,
+                       (int)order_chunks(n));
     PIC_HIP(hipGetLastError());
     PIC_HIP(hipStreamSynchronize(c->stream));
+    c->order_known = Ctx::ORDER_JUDGED;
+    c->order_moves = 0;
     c->uniform_w = c->w_host->differ == 0;
     c->w0 = c->w_host->w0;
     if (!c->uniform_w) {
@@ -696,9 +717,7 @@ int pic_set_state_f32(pic_ctx *ctx, const int32_t *cell, const float *ox, const 
     }
     PIC_HIP(hipStreamSynchronize(c->stream));
     c->state = PIC_STATE_F32;
-    c->seg_valid = false;
-    c->near_order = false;
-    c->sort_fresh = false;
+    new_particles(c);
     return PIC_OK;
 }
 

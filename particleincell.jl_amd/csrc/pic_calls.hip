@@ -191,7 +191,9 @@ int pic_compute_rho(pic_ctx *ctx, int kernel) {
     PIC_CHECK(valid_shape(kernel), PIC_ERR_ARG, "kernel %d", kernel);
     Ctx *c = ctx_of(ctx);
     PIC_HIP(hipSetDevice(c->device));
-    if (c->state == PIC_STATE_F64 && !c->near_order && deposit_lds_pays(c, kernel)) {
+    bool near = true;
+    if (c->state == PIC_STATE_F64 && c->n) PIC_TRY(particles_near_order(c, kernel, &near));
+    if (!near && deposit_lds_pays(c, kernel)) {
         PIC_TRY(deposit_rho(c, kernel));
         PIC_HIP(hipStreamSynchronize(c->stream));
         return PIC_OK;
@@ -227,7 +229,7 @@ int pic_push_x(pic_ctx *ctx, double dt) {
                            c->vy, dt, c->dimx, c->dimy);
         PIC_HIP(hipGetLastError());
     }
-    c->sort_fresh = false;
+    particles_moved(c);
     PIC_HIP(hipStreamSynchronize(c->stream));
     return PIC_OK;
 }
@@ -244,7 +246,7 @@ int pic_operator_t(pic_ctx *ctx, double dt) {
     }
     PIC_HIP(hipStreamSynchronize(c->stream));
     c->seg_valid = false;
-    c->sort_fresh = false;
+    particles_moved(c);
     return PIC_OK;
 }
 

@@ -14,11 +14,10 @@
 //
 // With R parts every chunk is read and its weights formed R times, so past
 // DEP_PARTS_MAX parts the chunk kernels of pic_step.hip serve; and for particles
-// that a sort put near their cells' order (Ctx::near_order), whose chunks cover
-// small boxes: measured on lane-sorted M6 particles they take as long as one
-// part does (10,000,000 on 128 x 128: 195 against 174 us; 300,000 CIC on 100 x
-// 100: 28 against 36) and less than several (2,000,000 on 400 x 400: 71 us
-// against 363).
+// near their cells' order (particles_near_order), whose chunks cover small boxes:
+// measured on lane-sorted M6 particles they take as long as one part does
+// (10,000,000 on 128 x 128: 195 against 174 us; 300,000 CIC on 100 x 100: 28
+// against 36) and less than several (2,000,000 on 400 x 400: 71 us against 363).
 #include <algorithm>
 
 #include "pic_internal.h"
@@ -254,19 +253,72 @@ int deposit(Ctx *c, int kernel, int how, double x0, double y0, bool residues) {
                            c->red_count, total);
     };
     // More waves to a node read more copies at once but need more blocks.
-    // Measured on MI355X, the whole call with CIC, us at 1 / 2 / 8 waves: 64 x 64
-    // nodes and 59 copies 25.9 / 25.0 / 24.5, 143 x 143 and 16 copies 27.4 / 27.1 /
+    // Measured on MI355X, the whole call with CIC, us at 1 / 2 / 8 waves: 32 x 32
+    // nodes and 30 copies 24.0 / 23.7 / 22.5, 64 x 64 and 59 25.9 / 25.0 / 24.5,
+    // 100 x 100 and 63 29.5 / 27.8 / 28.8, 143 x 143 and 16 copies 27.4 / 27.1 /
     // 31.0, 256 x 256 and 64 39.3 / 42.1 / 46.6; 100 x 100 and 256 copies 44.9 /
     // 38.2 / 34.9, 143 x 143 and 256 49.3 / 43.5 / 47.9, 200 x 200 and 128 42.9 /
     // 43.2 / 47.0.
-    if (a.chunks <= 64) reduce(k_deposit_reduce<1>, 1);
-    else if (m > 10240) reduce(k_deposit_reduce<2>, 2);
-    else reduce(k_deposit_reduce<8>, 8);
+    if (m <= 10240 && a.chunks > (m <= 4096 ? 8 : 64)) reduce(k_deposit_reduce<8>, 8);
+    else if (a.chunks > 64) reduce(k_deposit_reduce<2>, 2);
+    else reduce(k_deposit_reduce<1>, 1);
     PIC_HIP(hipGetLastError());
     return shift_rho(c, kernel);
 }
 
+// The samples of the particles' order, a block each.
+__global__ __launch_bounds__(256) void k_order(const double *__restrict__ x,
+                                               const double *__restrict__ y, int64_t n, int nx,
+                                               int ny, double dx, double dy, int64_t nch,
+                                               Order *out) {
+    const int s = blockIdx.x;
+    picd::order_sample(out, s, s * nch / gridDim.x * STEP_CHUNK, n, nx, ny, dx, dy,
+                       [&](int64_t k, double &a, double &b) {
+                           a = x[k];
+                           b = y[k];
+                       });
+}
+
 }  // namespace
+
+// Particles as a sort by cell left them, and as callers hand them back later,
+// fill small boxes chunk by chunk, and the chunk kernels are then the faster
+// ones.  So are they told from others by the chunks' extents: taken while
+// particles are handed in, in the kernel that unpacks them, or by a kernel of
+// their own when they are not known; a sort's order, and a verdict, are asked
+// again after ORDER_MOVES moves.  A chunk whose stencils' box does not fit its
+// tile pays for global atomics: one in sixteen of them may (for 2,000,000 M6
+// particles 0.2 of 3.1 ms, as much as the LDS deposit takes).
+// On small grids the LDS deposit serves any order: measured on lane-sorted
+// particles, chunk kernels and LDS, 10,000 CIC on 32 x 32 nodes 26 and 22 us,
+// 300,000 M6 on 64 x 64 35 and 31 (sorted by cell alone 114 and 78); 300,000 CIC
+// on 100 x 100 28 and 36.
+constexpr int64_t DEP_ANY_ORDER = 4096;
+int particles_near_order(Ctx *c, int kernel, bool *near) {
+    *near = false;
+    if ((int64_t)c->nx * c->ny <= DEP_ANY_ORDER) return PIC_OK;
+    const int64_t nch = order_chunks(c->n);
+    const int samples = (int)std::min<int64_t>(nch, ORDER_SAMPLES);
+    if (c->order_known == Ctx::ORDER_UNKNOWN || c->order_moves >= ORDER_MOVES) {
+        PIC_TRY(ensure_w_host(c));
+        hipLaunchKernelGGL(k_order, dim3((unsigned)samples), dim3(256), 0, c->stream,
+                           (const double *)c->x, (const double *)c->y, c->n, c->nx, c->ny, c->dx,
+                           c->dy, nch, &c->w_host->order);
+        PIC_HIP(hipGetLastError());
+        PIC_HIP(hipStreamSynchronize(c->stream));
+        c->order_known = Ctx::ORDER_JUDGED;
+        c->order_moves = 0;
+    }
+    *near = true;
+    if (c->order_known == Ctx::ORDER_SORTED) return PIC_OK;
+    int span = 6;
+    PIC_SHAPE_SWITCH(kernel, span = Shape<KK>::S);
+    int far = 0;
+    for (int s = 0; s < samples; ++s)
+        far += (c->w_host->order.w[s] + span - 1) * (c->w_host->order.h[s] + span - 1) > STEP_CAP64;
+    *near = 16 * far <= samples;
+    return PIC_OK;
+}
 
 int ensure_copies(Ctx *c, int64_t count) {
     if (count <= c->copies_cap) return PIC_OK;

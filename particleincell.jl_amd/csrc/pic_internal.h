@@ -44,6 +44,15 @@ int fail(int code, const char *fmt, ...);
     } while (0)
 
 // ------------------------------------------------------------ the context
+// The extents, in cells, of up to ORDER_SAMPLES chunks of STEP_CHUNK consecutive
+// particles (the blocks of pic_step.hip's FP64 kernels), spread over all.
+constexpr int STEP_CHUNK = 1024, STEP_CAP64 = 2048;  // that kernel's tile: nodes
+constexpr int ORDER_SAMPLES = 64, ORDER_MOVES = 8;
+struct Order {
+    int w[ORDER_SAMPLES], h[ORDER_SAMPLES];
+};
+inline int64_t order_chunks(int64_t n) { return (n + STEP_CHUNK - 1) / STEP_CHUNK; }
+
 struct Ctx {
     int device = 0;
     int ncu = 1;                        // compute units of the device
@@ -75,6 +84,7 @@ struct Ctx {
     struct Weights {
         double w0;
         int differ;
+        Order order;
     } *w_host = nullptr;
     // second set of state arrays: the sort gathers into these and swaps the
     // pointers (keyed by the address of the Ctx member they pair with)
@@ -124,8 +134,11 @@ struct Ctx {
     // after a lane sort, segment s occupies slots [cell_off[64 s],
     // cell_off[min(64 s + 64, ncells)]) until the next sort
     bool seg_valid = false;             // cell_off describes the current slots
-    // a sort of either kind put the current particles near their cells' order
-    bool near_order = false;
+    // how near their cells' order the FP64 state's particles are (see
+    // particles_near_order in pic_deposit.hip): a sort's, or judged from
+    // `order` and good for ORDER_MOVES moves
+    enum { ORDER_UNKNOWN, ORDER_SORTED, ORDER_JUDGED } order_known = ORDER_UNKNOWN;
+    int order_moves = 0;
     // the particles sit in the order the last lane sort left (or its pending
     // permutation gives) and have not moved since: pic_run can skip its own
     // first sort
@@ -242,10 +255,23 @@ int shift_rho(Ctx *c, int kernel);
 // again afterwards.
 bool deposit_lds_ok(Ctx *c);
 bool deposit_lds_pays(Ctx *c, int kernel);
+// Whether chunks of the FP64 state's consecutive particles fit the chunk kernels'
+// tiles; judges the particles anew (and waits) where that is not known.
+int particles_near_order(Ctx *c, int kernel, bool *near);
+// The particles are others (in an order not known), or have moved.
+inline void new_particles(Ctx *c) {
+    c->seg_valid = c->sort_fresh = false;
+    c->order_known = Ctx::ORDER_UNKNOWN;
+}
+inline void particles_moved(Ctx *c, int times = 1) {
+    c->sort_fresh = false;
+    c->order_moves = times < ORDER_MOVES ? c->order_moves + times : ORDER_MOVES;
+}
 int deposit_rho(Ctx *c, int kernel);
 int deposit_rho_mf(Ctx *c, double x0, double y0, bool compat);
 int deposit_rho_residues(Ctx *c);
 int ensure_copies(Ctx *c, int64_t count);
+int ensure_w_host(Ctx *c);
 int field_energy(Ctx *c, double *out2);
 // Queues solve!(fields, poisson): E from rho, and with slot >= 0
 // meshfields.jl:105-106's energy sums: the interior sums times dx dy into
@@ -373,6 +399,53 @@ __device__ __forceinline__ int cell_of(double xp, double fl, int n, double &d) {
         if (i < 0) i += n;
     }
     return i;
+}
+
+// The extent of the chunk starting at particle `base` < n, from every fourth of
+// its particles, into sample s of *out.  xy(k, x, y) reads a position.  Called by
+// all 256 threads of a block.
+template <class F>
+__device__ __forceinline__ void order_sample(pic::Order *out, int s, int64_t base, int64_t n,
+                                             int nx, int ny, double dx, double dy, F &&xy) {
+    __shared__ int box[4];
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        box[0] = box[2] = INT32_MAX;
+        box[1] = box[3] = INT32_MIN;
+    }
+    __syncthreads();
+    double x, y, d;
+    xy(base, x, y);
+    const double xr = x / dx, yr = y / dy;
+    const int i0 = cell_of(xr, floor(xr), nx, d), j0 = cell_of(yr, floor(yr), ny, d);
+    const int64_t k = base + 4 * tid;
+    int di = 0, dj = 0;  // the chunk's first particle
+    if (k < n) {
+        xy(k, x, y);
+        const double xp = x / dx, yp = y / dy;
+        di = cell_of(xp, floor(xp), nx, d) - i0;
+        dj = cell_of(yp, floor(yp), ny, d) - j0;
+        di = di >= nx - nx / 2 ? di - nx : di < -(nx / 2) ? di + nx : di;
+        dj = dj >= ny - ny / 2 ? dj - ny : dj < -(ny / 2) ? dj + ny : dj;
+    }
+    int a = di, b = di, c = dj, e = dj;
+    for (int o = 32; o > 0; o >>= 1) {
+        a = min(a, __shfl_xor(a, o));
+        b = max(b, __shfl_xor(b, o));
+        c = min(c, __shfl_xor(c, o));
+        e = max(e, __shfl_xor(e, o));
+    }
+    if ((tid & 63) == 0) {
+        atomicMin(&box[0], a);
+        atomicMax(&box[1], b);
+        atomicMin(&box[2], c);
+        atomicMax(&box[3], e);
+    }
+    __syncthreads();
+    if (tid == 0) {
+        out->w[s] = box[1] - box[0] + 1;
+        out->h[s] = box[3] - box[2] + 1;
+    }
 }
 
 // a / b for a divisor used several times: with r = 1/b rounded, q = a r and

@@ -262,9 +262,7 @@ int pic_sample_landau(pic_ctx *ctx, int64_t n, double alpha, double kx, int stat
     PIC_TRY(ensure_particles(c, n));
     c->n = n;
     c->state = PIC_STATE_F64;
-    c->seg_valid = false;
-    c->near_order = false;
-    c->sort_fresh = false;
+    new_particles(c);
     c->uniform_w = true;
     c->w0 = n ? (c->dimx * c->dimy) / (double)n : 0.0;
     if (n) {
@@ -294,9 +292,7 @@ int pic_sample_maxwellian(pic_ctx *ctx, int64_t n, double alpha, double kx, doub
     PIC_TRY(ensure_particles(c, n));
     c->n = n;
     c->state = PIC_STATE_F64;
-    c->seg_valid = false;
-    c->near_order = false;
-    c->sort_fresh = false;
+    new_particles(c);
     c->uniform_w = true;
     c->w0 = n ? (c->dimx * c->dimy) / (double)n : 0.0;
     if (n) {

@@ -1479,9 +1479,7 @@ int pic_run_maxwell(pic_ctx *ctx, int kernel, double dt, int nsteps, double *ene
         }
     }
     for (hipEvent_t e : ev) (void)hipEventDestroy(e);
-    c->seg_valid = false;
-    c->near_order = false;
-    c->sort_fresh = false;
+    new_particles(c);
     return rc;
 }
 

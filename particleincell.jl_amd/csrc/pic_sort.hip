@@ -723,7 +723,8 @@ int sort_by_cell(Ctx *c, int32_t *perm_host, bool lanes, bool apply) {
         PIC_HIP(hipStreamSynchronize(c->stream));
     }
     c->sort_fresh = lanes;
-    c->near_order = true;
+    c->order_known = Ctx::ORDER_SORTED;
+    c->order_moves = 0;
     return PIC_OK;
 }
 

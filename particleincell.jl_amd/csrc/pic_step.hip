@@ -39,7 +39,7 @@
 namespace pic {
 
 constexpr int ST = 256;        // threads per block
-constexpr int CAP64 = 2048;    // tile capacity (nodes), FP64 kernels
+constexpr int CAP64 = STEP_CAP64;  // tile capacity (nodes), FP64 kernels
 constexpr int CAP32 = 4096;    // tile capacity (nodes), FP32 kernels
 
 struct ArgsF64 {
@@ -666,7 +666,7 @@ __global__ __launch_bounds__(ST) void k_step_f32(ArgsF32 a) {
 
 // ============================================================== dispatch
 
-constexpr int PPT64 = 4;
+constexpr int PPT64 = STEP_CHUNK / ST;
 constexpr int PPT32 = 4;
 
 static size_t smem64_bytes(int bz) { return (size_t)CAP64 * (bz == PIC_BZ_GRID ? 24 : 16); }
@@ -709,7 +709,7 @@ static int launch64_k(Ctx *c, const ArgsF64 &a, int mode, int bz) {
 
 int launch_step64(Ctx *c, int kernel, int mode, double dt, double dtd) {
     if (c->n == 0) return PIC_OK;
-    if (mode <= 2) c->sort_fresh = false;  // the pass moves the particles
+    if (mode <= 2) particles_moved(c);
     ArgsF64 a;
     a.n = c->n;
     a.x = c->x; a.y = c->y; a.vx = c->vx; a.vy = c->vy;
@@ -762,7 +762,7 @@ static int launch32_k(Ctx *c, const ArgsF32 &a, int mode, int bz) {
 // dt: kick length; dtd: drift length (one full drift per step in FP32).
 int launch_step32(Ctx *c, int kernel, int mode, double dt, double dtd) {
     if (c->n == 0) return PIC_OK;
-    if (mode <= 2) c->sort_fresh = false;  // the pass moves the particles
+    if (mode <= 2) particles_moved(c);
     ArgsF32 a;
     a.n = c->n;
     a.cell = c->cell; a.ov = c->ov32;

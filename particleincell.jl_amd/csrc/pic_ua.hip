@@ -945,9 +945,7 @@ int pic_ua_compute_rho(pic_ctx *ctx, const double *t, const double *xt) {
     if (lds) PIC_TRY(deposit_rho_residues(c));
     else PIC_TRY(finalize_rho(c, PIC_M6));
     PIC_HIP(hipStreamSynchronize(c->stream));
-    c->seg_valid = false;
-    c->near_order = false;
-    c->sort_fresh = false;
+    new_particles(c);
     return PIC_OK;
 }
 
@@ -1040,9 +1038,7 @@ int pic_ua_run(pic_ctx *ctx, double dt, int nsteps, double *energy) {
             energy[k] = h[2 * k] + h[2 * k + 1] + h[2 * nh + k] * c->dx * c->dy;
     }
     PIC_HIP(hipStreamSynchronize(c->stream));
-    c->seg_valid = false;
-    c->near_order = false;
-    c->sort_fresh = false;
+    new_particles(c);
     return PIC_OK;
 }
 
