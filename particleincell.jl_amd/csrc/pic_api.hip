@@ -1,5 +1,6 @@
 // pic_api.hip -- context management, particle/grid transfers and the
 // Fortran-twin drop-ins of libpicmi355x.
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -369,7 +370,7 @@ struct Staging {
             if (c->stage) (void)hipFree(c->stage);
             c->stage = nullptr;
             c->stage_bytes = 0;
-            const int64_t room = bytes + bytes / 4;
+            const int64_t room = std::min(bytes + bytes / 4, STAGE_KEEP);
             PIC_HIP(hipMalloc(&c->stage, (size_t)room));
             c->stage_bytes = room;
         }

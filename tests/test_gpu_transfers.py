@@ -134,3 +134,26 @@ def test_device_particles_are_read_on_return(gpu, weighted):
     assert hip.hipFree(d) == 0 and hip.hipStreamDestroy(s) == 0
     np.testing.assert_array_equal(got, p)
     ctx.close()
+
+
+def test_kept_staging_is_at_most_64_mib(gpu):
+    """60 MiB of particles go up through a staging buffer that the context
+    keeps: it holds no more than 64 MiB beside their four arrays (multiples of
+    the device's 2 MiB pages; a quarter more than the particles were 75)."""
+    pic = gpu
+    n = 60 * 2**20 // 40
+    ctx = _context(pic, 16, 16)
+    p = np.asfortranarray(np.random.default_rng(3).uniform(0.05, 0.95, (5, n)))
+    p[4] = 0.25
+    ctx.set_particles(p[:, :100])  # what a first transfer sets up
+    hip = _hip()
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    before = free()
+    ctx.set_particles(p)
+    assert before - free() <= 4 * 8 * n + 68 * 2**20
+    ctx.close()
