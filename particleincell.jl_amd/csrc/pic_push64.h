@@ -29,8 +29,7 @@ struct SegF64 {
     const int64_t *off;
     int bps, margin, cap;
     unsigned long long *slow;
-    uint32_t *dlist;  // deferred particles and their count
-    unsigned *dcount;
+    uint32_t *dlist;  // deferred particles, a slice per block
 };
 
 // The reference's cell and in-cell offset (pushers_cic.jl:18-29): i =

@@ -25,8 +25,12 @@
 // steps: pass 3.69 ms and list 0.31 -> 3.21 ms.
 //
 // Arithmetic per particle is the same as in pic_step.hip's kernels (FP64:
-// the reference's operations; FP32: the cell-relative step), so results are
-// bit-identical to them up to the order of the charge sums.
+// the reference's operations; FP32: the cell-relative step), so positions and
+// velocities after a pass are bit-identical to theirs.  Charges are not: they
+// are summed in another order, in the FP32 state by the accumulation modes
+// below, and in the FP64 state by blocks of SEG64_FIX or more particles of one
+// weight w with every share rounded to a multiple of w 2^-bits (51 bits up to
+// 4,095 particles a block, one fewer for every doubling; one more for M6).
 //
 // FP32 charge accumulation, three modes (Ctx::f32_acc):
 //  2 fixed-point int32 LDS tiles: every contribution is rounded to a multiple
@@ -649,7 +653,9 @@ __global__ __launch_bounds__(SEG64_T) void k_seg_f64(SegF64 a) {
     // or more of one weight: the quantum is the smallest power of two that
     // keeps a share below 2^51 and the sum of all the block's particles at one
     // node below 2^63 in magnitude.  At 32 particles per cell and more that
-    // rounds no more than adding the shares in FP64 does (normwise error of
+    // rounds no more than adding the shares in FP64 does over the grid as a
+    // whole; a node that only small shares reach loses relative accuracy, down
+    // to shares below half a quantum, which vanish (normwise error of
     // the charge against 80-bit sums, CIC and M6: 2,048 particles in one cell
     // 4.7e-16, 3.9e-16 with FP64 sums -> 4.6e-17, 9e-17; 70,001 in one cell
     // 2.8e-15, 2.7e-15 -> 1e-16, 5e-16; 600,011 on 64^2 1.1e-16, 1.6e-16 both
@@ -972,7 +978,6 @@ int launch_seg64(Ctx *c, int kernel, int mode, double dt, double dtd) {
     a.slow = c->slow_chunks;
     PIC_TRY(ensure_defer(c));
     a.dlist = c->defer;
-    a.dcount = c->defer_count;
     const size_t sm = (size_t)a.cap * (per_node ? per_node : 8);
     int rc;
     PIC_SHAPE_SWITCH(kernel, rc = a.perm ? seg64_mode<KK, true>(c, a, mode, c->bz_mode, sm)

@@ -5,8 +5,10 @@
 // After a lane sort segment s of 64 consecutive cells owns the slots
 // [off[64 s], off[min(64 s + 64, ncells)]) until the next sort; a block takes
 // a slice of one segment, stages a window of the grid around the segment's
-// home cells in LDS and hands particles whose stencil leaves it to a
-// deferred list that a global-memory kernel completes after the pass.
+// home cells in LDS and puts particles whose stencil leaves it on a deferred
+// list, to be completed from global memory: by the block itself after its
+// particle loop (a list per block, in LDS its length), or for all blocks by a
+// kernel after the pass.
 #pragma once
 
 #include "pic_internal.h"
@@ -66,7 +68,7 @@ __device__ __forceinline__ int seg_block_order() {
                         : (int)blockIdx.x;
 }
 
-// End of a deferred-list kernel: block 0 adds the list length to the
+// End of such a kernel: block 0 adds the list length to the
 // slow-path counter; the last block to arrive (every block has read the
 // count by then) clears count and arrivals for the next pass.
 __device__ __forceinline__ void defer_finish(unsigned cnt, unsigned *dcount,

@@ -21,8 +21,10 @@
 // divisions formed anew for every particle took 304 and 458 us (204,800
 // particles, 128 x 64 cells, ntau 16, deposit not counted) against 190 and 215
 // now: 1,209 and 1,701 VALU instructions per wave, 57 % and 72 % of the issue
-// rate, the rest waiting for the gather's nodes.  Three waves per SIMD: at
-// four the correction spills (269 us).
+// rate, the rest waiting for the gather's nodes.  Three waves per SIMD at every
+// ntau: at four the correction spills.  Measured at two, three and four waves,
+// 3,276,800 samples each, correction: ntau 2 359, 358 and 358 us, 8 205, 204 and
+// 260, 16 183, 184 and 229, 64 200, 200 and 298; prediction at 16 145, 146 and 144.
 //
 // The fused loop keeps between the prediction and the correction only the
 // positions at the step's start and the tau-spectra of fx, fy; everything else
@@ -162,13 +164,6 @@ __device__ __forceinline__ cd fft_inv(cd z, const UaLane<NT> &L) {
     if constexpr (NT >= 32) z = fft_pair<NT, 4, true>(z, L);
     if constexpr (NT >= 64) z = fft_pair<NT, 5, true>(z, L);
     return mk(z.re * (1.0 / NT), z.im * (1.0 / NT));
-}
-
-// The value lane bitrev(m) of the group holds: a spectrum between its
-// bit-reversed and the reference's order (either way).
-template <int NT>
-__device__ __forceinline__ cd reorder(cd z, const UaLane<NT> &L) {
-    return shfl(z, L.base + bitrev<NT>(L.m));
 }
 
 // Sum over the NT lanes of a group (every lane receives it).
