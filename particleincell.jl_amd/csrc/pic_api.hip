@@ -142,13 +142,18 @@ int launch_fill(Ctx *c, double *p, double v, int64_t n) {
 // first one's (by the first wave that finds one: *flag, zero before), and
 // out->w0 to that weight.
 // Block 4 ch of the 256-particle blocks also judges chunk ch's order, where that
-// is one of the samples (spread over the nch chunks).
+// is one of the samples (spread over the nch chunks; nch 0: no samples).
 __global__ __launch_bounds__(256) void k_aos_to_soa(const double *__restrict__ p, int64_t n,
                                                     double *x, double *y, double *vx, double *vy,
                                                     unsigned *flag, Ctx::Weights *out, int nx,
                                                     int ny, double dx, double dy, int nch) {
     static_assert(STEP_CHUNK == 4 * 256, "four blocks to a chunk");
-    if ((blockIdx.x & 3) == 0) {
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const double w0 = p[4];
+    double q[5];  // read before the sample is, so that they arrive together
+#pragma unroll
+    for (int i = 0; i < 5; ++i) q[i] = p[5 * min(k, n - 1) + i];
+    if (nch && (blockIdx.x & 3) == 0) {
         const int ch = blockIdx.x >> 2, smp = min(nch, ORDER_SAMPLES);
         const int s = (int)(((int64_t)ch * smp + nch - 1) / nch);
         if (s < smp && (int64_t)s * nch / smp == ch)
@@ -158,14 +163,11 @@ __global__ __launch_bounds__(256) void k_aos_to_soa(const double *__restrict__ p
                                    b = p[5 * q + 1];
                                });
     }
-    int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    const double *q = p + 5 * k;
     x[k] = q[0];
     y[k] = q[1];
     vx[k] = q[2];
     vy[k] = q[3];
-    const double w0 = p[4];
     if (k == 0) out->w0 = w0;
     const unsigned long long b = __ballot(q[4] != w0);
     if (b && (int)(threadIdx.x & 63) == __ffsll((long long)b) - 1 &&
@@ -316,7 +318,7 @@ static int set_particles_impl(Ctx *c, const double *d_p, int64_t n) {
     c->w_host->differ = 0;
     hipLaunchKernelGGL(k_aos_to_soa, grid1(n), dim3(256), 0, c->stream, d_p, n, c->x, c->y,
                        c->vx, c->vy, c->w_flag, c->w_host, c->nx, c->ny, c->dx, c->dy,
-                       (int)order_chunks(n));
+                       (int64_t)c->nx * c->ny > ORDER_ANY ? (int)order_chunks(n) : 0);
     PIC_HIP(hipGetLastError());
     PIC_HIP(hipStreamSynchronize(c->stream));
     c->order_known = Ctx::ORDER_JUDGED;

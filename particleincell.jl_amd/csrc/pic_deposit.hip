@@ -289,14 +289,13 @@ __global__ __launch_bounds__(256) void k_order(const double *__restrict__ x,
 // again after ORDER_MOVES moves.  A chunk whose stencils' box does not fit its
 // tile pays for global atomics: one in sixteen of them may (for 2,000,000 M6
 // particles 0.2 of 3.1 ms, as much as the LDS deposit takes).
-// On small grids the LDS deposit serves any order: measured on lane-sorted
+// On grids of ORDER_ANY nodes and fewer the LDS deposit serves any order: measured on lane-sorted
 // particles, chunk kernels and LDS, 10,000 CIC on 32 x 32 nodes 26 and 22 us,
 // 300,000 M6 on 64 x 64 35 and 31 (sorted by cell alone 114 and 78); 300,000 CIC
 // on 100 x 100 28 and 36.
-constexpr int64_t DEP_ANY_ORDER = 4096;
 int particles_near_order(Ctx *c, int kernel, bool *near) {
     *near = false;
-    if ((int64_t)c->nx * c->ny <= DEP_ANY_ORDER) return PIC_OK;
+    if ((int64_t)c->nx * c->ny <= ORDER_ANY) return PIC_OK;
     const int64_t nch = order_chunks(c->n);
     const int samples = (int)std::min<int64_t>(nch, ORDER_SAMPLES);
     if (c->order_known == Ctx::ORDER_UNKNOWN || c->order_moves >= ORDER_MOVES) {
@@ -315,7 +314,8 @@ int particles_near_order(Ctx *c, int kernel, bool *near) {
     PIC_SHAPE_SWITCH(kernel, span = Shape<KK>::S);
     int far = 0;
     for (int s = 0; s < samples; ++s)
-        far += (c->w_host->order.w[s] + span - 1) * (c->w_host->order.h[s] + span - 1) > STEP_CAP64;
+        far += (int64_t)(c->w_host->order.extent[s].x + span - 1) *
+                   (c->w_host->order.extent[s].y + span - 1) > STEP_CAP64;
     *near = 16 * far <= samples;
     return PIC_OK;
 }

@@ -48,8 +48,9 @@ int fail(int code, const char *fmt, ...);
 // particles (the blocks of pic_step.hip's FP64 kernels), spread over all.
 constexpr int STEP_CHUNK = 1024, STEP_CAP64 = 2048;  // that kernel's tile: nodes
 constexpr int ORDER_SAMPLES = 64, ORDER_MOVES = 8;
+constexpr int64_t ORDER_ANY = 4096;  // grids on which the order does not matter: nodes
 struct Order {
-    int w[ORDER_SAMPLES], h[ORDER_SAMPLES];
+    int2 extent[ORDER_SAMPLES];
 };
 inline int64_t order_chunks(int64_t n) { return (n + STEP_CHUNK - 1) / STEP_CHUNK; }
 
@@ -442,10 +443,7 @@ __device__ __forceinline__ void order_sample(pic::Order *out, int s, int64_t bas
         atomicMax(&box[3], e);
     }
     __syncthreads();
-    if (tid == 0) {
-        out->w[s] = box[1] - box[0] + 1;
-        out->h[s] = box[3] - box[2] + 1;
-    }
+    if (tid == 0) out->extent[s] = make_int2(box[1] - box[0] + 1, box[3] - box[2] + 1);
 }
 
 // a / b for a divisor used several times: with r = 1/b rounded, q = a r and
