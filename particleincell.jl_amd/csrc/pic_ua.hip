@@ -20,7 +20,7 @@
 // prediction and 20 in the correction, and twiddles, cosines and FP64
 // divisions formed anew for every particle took 304 and 458 us (204,800
 // particles, 128 x 64 cells, ntau 16, deposit not counted) against 190 and 215
-// now: 1,209 and 1,701 VALU instructions per wave, 57 % and 72 % of the issue
+// now: 1,213 and 1,705 VALU instructions per wave, 59 % and 73 % of the issue
 // rate, the rest waiting for the gather's nodes.  Three waves per SIMD at every
 // ntau: at four the correction spills.  Measured at two, three and four waves,
 // 3,276,800 samples each, correction: ntau 2 359, 358 and 358 us, 8 205, 204 and
