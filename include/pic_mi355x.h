@@ -259,7 +259,7 @@ int pic_run(pic_ctx *ctx, int kernel, double dt, int nsteps, int sort_every, dou
  * fused = 0 the separate solve, particle-pass and sort kernels.  Measured
  * on MI355X, Landau CIC 64 x 64 with 204,800 particles, 100 steps: one
  * launch 18.6 us (FP32 state) and 20.2 us (FP64) per step of wall time; the
- * separate kernels 37.7 and 38.0 us.  The FP32 state's
+ * separate kernels 32.7 and 33.1 us.  The FP32 state's
  * one-launch charge is int32 fixed point with one quantum for every block,
  * summed as int64 (exact and run-to-run identical).  No reference
  * counterpart. */
