@@ -483,6 +483,8 @@ int pic_ctx_create(pic_ctx **out, int device, int nx, int ny, double xmin, doubl
         if (e == hipSuccess) e = hipMemsetAsync(c->defer_count, 0, 2 * sizeof(unsigned), c->stream);
         if (e == hipSuccess) e = hipMemsetAsync(c->rho, 0, m * 8, c->stream);
         if (e == hipSuccess) e = hipMemsetAsync(c->ex, 0, 2 * m * 8, c->stream);
+        if (e == hipSuccess) e = hipMemsetAsync(c->e32, 0, m * sizeof(float2), c->stream);
+        if (e == hipSuccess) e = hipMemsetAsync(c->phi, 0, m * 8, c->stream);
         if (e == hipSuccess) e = hipMemsetAsync(c->bz, 0, m * 8, c->stream);
         if (e == hipSuccess) e = hipMemsetAsync(c->bz32, 0, m * 4, c->stream);
         if (e == hipSuccess) e = hipMemsetAsync(c->rho_acc, 0, m * 8, c->stream);

@@ -157,3 +157,27 @@ def test_kept_staging_is_at_most_64_mib(gpu):
     ctx.set_particles(p)
     assert before - free() <= 4 * 8 * n + 68 * 2**20
     ctx.close()
+
+
+@pytest.mark.parametrize("state", [0, 1])
+def test_fields_of_a_new_context_are_zero(gpu, state):
+    """A kick before any field was set or solved leaves the velocities alone, in
+    both states, and phi reads as zero: whatever contexts before it left in the
+    memory its grids lie in."""
+    pic = gpu
+    L = pic._lib
+    nx = ny = 128
+    mesh = pic.TwoDGrid(1.0, nx, 1.0, ny)
+    p = np.asfortranarray(np.random.default_rng(9).uniform(0.1, 0.9, (5, 1_000)))
+    p[:4] = p[:4].astype(np.float32)
+    p[4] = 0.25
+    for _ in range(4):
+        ctx = _context(pic, nx, ny)
+        for which in (L.PIC_GRID_RHO, L.PIC_GRID_EX, L.PIC_GRID_EY, L.PIC_GRID_BZ, L.PIC_GRID_PHI):
+            ctx.set_grid(which, np.full((nx, ny), 1e3))
+        ctx.close()
+    sim = pic.Simulation(mesh, p, pic.M6(), state=state)
+    np.testing.assert_array_equal(sim.grid(L.PIC_GRID_PHI), 0.0)
+    sim.step_pass(2, 0.1)
+    np.testing.assert_array_equal(sim.particles()[2:4], p[2:4])
+    sim.close()
