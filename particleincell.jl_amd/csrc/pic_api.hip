@@ -381,23 +381,15 @@ struct Staging {
     }
 };
 
-// Grids pass between host and device as a copy of the caller's array, or through
-// the context's pinned copy (1 MiB at most), which kernels read and write
-// themselves.  Measured on MI355X, pinned against copied, us a call: a pageable
-// copy of up to 16 KiB is slow (45 x 45 nodes set 14.7 against 16.9, read 14.3
-// against 24.1; 48 x 48 14.8 against 10.4, 14.5 against 10.3; 362 x 362 54
-// against 46, 62 against 54).  Where a kernel follows the copy anyway, for the
-// FP32 field, pinned is faster throughout (64 x 64 15.1 against 22.7, 362 x 362
-// 54 against 57), and where the caller's layout is another (a ghost line, a
-// stride), which a copy then passes through a third array, from about 200 x 200
-// on (160 x 160 read with its ghost line 22.8 against 21.6, 200 x 200 28.8 against
-// 29.1, 256 x 256 36 against 43).
-constexpr int64_t GRID_PINNED = 1 << 17, GRID_SLOW_COPY = 2048, GRID_REPACKED = 40000;
-static int pinned_grid(Ctx *c, bool field, bool packed, double **t) {
+// Grids of at most GRID_PINNED points pass between host and device through the
+// context's pinned copy, which kernels read and write themselves: the copy
+// engine's calls cost 10-20 us each, more than such a grid.  Larger ones are
+// copied (*t null).
+constexpr int64_t GRID_PINNED = 1 << 17;
+static int pinned_grid(Ctx *c, double **t) {
     const int64_t m = (int64_t)c->nx * c->ny;
     *t = nullptr;
-    if (m > GRID_PINNED || !(field || m <= GRID_SLOW_COPY || (!packed && m >= GRID_REPACKED)))
-        return PIC_OK;
+    if (m > GRID_PINNED) return PIC_OK;
     if (!c->grid_host)
         PIC_HIP(hipHostMalloc(&c->grid_host, (size_t)m * sizeof(double), hipHostMallocDefault));
     *t = c->grid_host;
@@ -755,10 +747,8 @@ int pic_set_grid(pic_ctx *ctx, int which, const double *host, int ld, int stride
     const int64_t m = (int64_t)c->nx * c->ny;
     double *t = nullptr;
     std::vector<double> own;
-    const bool e = which == PIC_GRID_EX || which == PIC_GRID_EY, b = which == PIC_GRID_BZ;
-    const bool packed = ld == c->nx && stride == 1;
-    PIC_TRY(pinned_grid(c, e || b, packed, &t));
-    if (!t && !packed) {  // packed first
+    PIC_TRY(pinned_grid(c, &t));
+    if (!t && (ld != c->nx || stride != 1)) {  // not the grid's own layout: packed first
         own.resize((size_t)m);
         t = own.data();
     }
@@ -770,6 +760,7 @@ int pic_set_grid(pic_ctx *ctx, int which, const double *host, int ld, int stride
     const bool pinned = t && t == c->grid_host;
     if (!pinned)
         PIC_HIP(hipMemcpyAsync(d, t ? t : host, (size_t)m * 8, hipMemcpyHostToDevice, c->stream));
+    const bool e = which == PIC_GRID_EX || which == PIC_GRID_EY, b = which == PIC_GRID_BZ;
     if (pinned || e || b) {
         hipLaunchKernelGGL(k_set_grid, grid1(m), dim3(256), 0, c->stream,
                            (const double *)(pinned ? t : d), m, d, (const double *)c->ex,
@@ -792,14 +783,13 @@ int pic_get_grid(pic_ctx *ctx, int which, double *host, int ld, int stride, int 
     const int64_t m = (int64_t)c->nx * c->ny;
     double *t = nullptr;
     std::vector<double> own;
-    const bool packed = ld == c->nx && stride == 1 && !ghost;
-    PIC_TRY(pinned_grid(c, false, packed, &t));
+    PIC_TRY(pinned_grid(c, &t));
     if (t) {
         hipLaunchKernelGGL(k_get_grid, grid1(m), dim3(256), 0, c->stream, (const double *)d, m, t);
         PIC_HIP(hipGetLastError());
     } else {
         t = host;
-        if (!packed) {
+        if (ld != c->nx || stride != 1 || ghost) {  // not the grid's own layout
             own.resize((size_t)m);
             t = own.data();
         }
