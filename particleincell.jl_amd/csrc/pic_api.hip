@@ -382,9 +382,14 @@ struct Staging {
 };
 
 // Grids of at most GRID_PINNED points pass between host and device through the
-// context's pinned copy, which kernels read and write themselves: the copy
-// engine's calls cost 10-20 us each, more than such a grid.  Larger ones are
-// copied (*t null).
+// context's pinned copy, which kernels read and write themselves; larger ones are
+// copied (*t null).  Measured on MI355X, us a call: the pinned way takes the same
+// time wherever the caller's array lies, 15-16 up to 64 x 64 nodes, 18 at 100 x
+// 75, 33 at 200 x 200, 70 at 362 x 362.  A pageable copy takes 23-35 up to 16
+// KiB, and past that between 10 (64 x 64), 12 (100 x 75) and 24 (200 x 200), from
+// an array whose pages the runtime finds at hand, and 27, 45 and 154 to a new one
+// after a run.  1 MiB is what a context may hold for this; at 512 x 512 reading
+// takes 125 pinned and 141 copied, writing 105 and 85.
 constexpr int64_t GRID_PINNED = 1 << 17;
 static int pinned_grid(Ctx *c, double **t) {
     const int64_t m = (int64_t)c->nx * c->ny;
